@@ -296,3 +296,18 @@ def test_sort_multi_rejects_more_fp_columns_than_sign_bits(vctx):
     with pytest.raises(velodb_amd.VoError) as e:
         vctx.sort(dummy, [6, 6, 7, 6], [True] * 4, didx, 0, 1 << 29)
     assert e.value.status == 5  # VO_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("n,npad", [(8192, 8192), (8191, 16384), (40000, 65536)])
+def test_sort_equal_records_and_both_directions(vctx, n, npad):
+    """Whole records repeated many times, through the stage between lane
+    neighbours (tiles of 2^13 records, ascending and descending pairs): the
+    output is the sorted multiset, so no copy of a record is lost or doubled."""
+    print(f"sort equal records n={n} npad={npad}", flush=True)
+    rng = np.random.default_rng(n)
+    k = rng.integers(0, 3, n).astype(np.uint64) << np.uint64(33)
+    p = rng.integers(0, 4, n).astype(np.uint32)
+    gk, gp = _run_sort(vctx, k, p, n, npad)
+    order = np.lexsort((p, k))
+    assert np.array_equal(gk[:n], k[order]) and np.array_equal(gp[:n], p[order])
+    assert np.array_equal(gk[n:], np.full(npad - n, M64)) and np.array_equal(gp[n:], np.arange(n, npad, dtype=np.uint32))

@@ -369,41 +369,56 @@ struct TileCT {
     static constexpr int end_layout(int q, int a, int qlo = 0)
     {
         while (q >= qlo) {
-            if (q == 0 && a == 1) break;
+            if (LANE0 && q == 0 && a == 1) break;
             if (!(a <= q && q < a + R_LOG)) a = q - R_LOG + 1 > 0 ? q - R_LOG + 1 : 0;
             q = (a > qlo ? a : qlo) - 1;
         }
         return a;
     }
 
-    // The record in register m of the lane whose index differs in bit 0: a
-    // DPP quad permutation (lanes 1 0 3 2) per 32-bit word, no LDS.
-    static __device__ __forceinline__ uint32_t xor1(uint32_t v)
-    {
-        return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);
-    }
-    static __device__ __forceinline__ R lane_partner(const R &a)
-    {
-        R o;
-#pragma unroll
-        for (int w = 0; w < R::KW; ++w)
-            o.k[w] = (uint64_t)xor1((uint32_t)a.k[w]) | ((uint64_t)xor1((uint32_t)(a.k[w] >> 32)) << 32);
-        if constexpr (sizeof(P) == 8)
-            o.p = (P)((uint64_t)xor1((uint32_t)a.p) | ((uint64_t)xor1((uint32_t)((uint64_t)a.p >> 32)) << 32));
-        else
-            o.p = (P)xor1((uint32_t)a.p);
-        return o;
-    }
-
     // Stage 0 of level P in layout 1: record index bit 0 is thread index
     // bit 0, so the pair of register m is register m of lanes (2t, 2t+1).
-    // Each lane keeps the smaller or the larger record of its pair, as the
-    // compare-exchange would leave it (ties stay in place).
+    // Issue-bound, so it is kept to six VALU instructions a record: the borrow
+    // chain of lt_mask96 reads the partner's words through a DPP quad
+    // permutation (lanes 1 0 3 2), and the words move by DPP moves under the
+    // execution mask of the swapping pairs.  (Written with selects it compiled
+    // to 64-bit compares per record and took 10 us of a 2^23-record pass, as
+    // long as the other twelve stages and the three relayouts together.)
+    // Built for the 12-byte record, the only one whose layouts need it.
+    static constexpr bool LANE0 = R::TIE && R::KW == 1 && sizeof(P) == 4;
+
+    // Exchanges the records of the lane pairs that are out of order: ascending
+    // pairs where the odd lane's record is the smaller one, descending pairs
+    // (both lanes set in descm) where it is not (equal records are identical).
+    static __device__ __forceinline__ void lane_cmpx(R &r, uint64_t descm)
+    {
+        uint32_t w0 = (uint32_t)r.p, w1 = (uint32_t)r.k[0], w2 = (uint32_t)(r.k[0] >> 32), t;
+        uint64_t sw, ex;
+        // s_nop: a DPP read needs two wait states after a VALU write of the register
+        asm("s_nop 1\n\t"
+            "v_sub_co_u32_dpp %3, vcc, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_subb_co_u32_dpp %3, vcc, %1, %1, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_subb_co_u32_dpp %3, vcc, %2, %2, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_and_b64 %4, vcc, %6\n\t" // partner < own, even lanes
+            "s_lshl_b64 vcc, %4, 1\n\t"
+            "s_or_b64 %4, %4, vcc\n\t" // both lanes of the pair
+            "s_xor_b64 %4, %4, %7\n\t"
+            "s_and_saveexec_b64 %5, %4\n\t"
+            "v_mov_b32_dpp %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_mov_b32_dpp %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_mov_b32_dpp %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+            "s_mov_b64 exec, %5"
+            : "+v"(w0), "+v"(w1), "+v"(w2), "=&v"(t), "=&s"(sw), "=&s"(ex)
+            : "s"(0x5555555555555555ull), "s"(descm)
+            : "vcc", "scc");
+        r.p = (P)w0;
+        r.k[0] = (uint64_t)w1 | ((uint64_t)w2 << 32);
+    }
+
     template <int P>
     static __device__ __forceinline__ void lane_stage0(R (&r)[RR], uint32_t tau, bool asc_hi, int p_top)
     {
         const uint32_t base = lay_base<R_LOG>(tau, 1);
-        const bool lower = (tau & 1u) == 0;
 #pragma unroll
         for (int m = 0; m < RR; ++m) {
             bool asc;
@@ -413,14 +428,7 @@ struct TileCT {
                 const uint32_t l = base | ((uint32_t)m << 1);
                 asc = (P >= p_top) | (P >= T_LOG ? asc_hi : (((l >> P) & 1u) == 0));
             }
-            const R o = lane_partner(r[m]);
-            // swap when this lane should keep the smaller and holds the
-            // larger, or the other way round
-            const bool keep_small = asc == lower;
-            const bool sw = keep_small ? rec_gt(r[m], o) : rec_gt(o, r[m]);
-#pragma unroll
-            for (int w = 0; w < R::KW; ++w) r[m].k[w] = sw ? o.k[w] : r[m].k[w];
-            r[m].p = sw ? o.p : r[m].p;
+            lane_cmpx(r[m], __builtin_amdgcn_ballot_w64(!asc));
         }
     }
 
@@ -554,7 +562,7 @@ struct TileCT {
     static __device__ __forceinline__ void level(R (&r)[RR], char *lds, uint32_t tau, bool asc_hi, int p_top,
                                                  uint64_t &h, uint32_t &n)
     {
-        if constexpr (Q == 0 && A == 1 && QLO == 0) {
+        if constexpr (LANE0 && Q == 0 && A == 1 && QLO == 0) {
             lane_stage0<P>(r, tau, asc_hi, p_top);
         } else if constexpr (Q >= QLO) {
             constexpr bool covered = (A <= Q && Q < A + R_LOG);

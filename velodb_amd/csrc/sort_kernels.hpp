@@ -153,6 +153,25 @@ __device__ __forceinline__ void gstore_t(const R &r, const Bufs<R> &b, uint64_t 
     }
 }
 
+// Blocks go to the 8 XCDs in turn; this order gives every XCD one contiguous
+// range of the launch's blocks (the first grid mod 8 ranges are one longer),
+// so a pass finds in its XCD's L2 what the pass before left there.  While an
+// instance fits the MALL every pass gains (12-byte sort, one-stage pass: 8.8
+// -> 5.8 us at 2^20 records, 29.5 -> 28.9 at 2^23; batched sorts 59.2 -> 57.8
+// ms).  Above it strided passes lose (1009 -> 1060 us at 2^28: every run they
+// read is another DRAM page) and keep the plain order; contiguous tiles gain
+// from 3 times the MALL up (merge pass 1219 -> 1123 us at 2^28; whole sorts at
+// 2^26, 2^27 and 2^28: 10.18 -> 10.03, 22.4 -> 21.9 and 48.8 -> 47.3 ms) but
+// lose between (16-byte sort at 2^25: 6.72 -> 6.88 ms; two key words at 2^24:
+// 4.37 -> 4.45 ms), where part of a pass is still found in the MALL.
+template <bool XC = true>
+__device__ __forceinline__ uint32_t xcd_block()
+{
+    if constexpr (!XC) return blockIdx.x;
+    const uint32_t q = gridDim.x >> 3, rem = gridDim.x & 7, x = blockIdx.x & 7;
+    return x * q + (x < rem ? x : rem) + (blockIdx.x >> 3);
+}
+
 // ----------------------------------------------------------- tiny arrays
 
 // n_pad <= 8: one thread runs the network directly.
@@ -273,13 +292,13 @@ __device__ __forceinline__ void body_local_ct(Bufs<R> b, IMap map, int p_top, ui
 
 // 1024-thread blocks: two per CU, 8 waves per SIMD (at most 64 VGPRs; the
 // second bound is the minimum waves per execution unit)
-template <class R, int T_LOG, int R_LOG, int BLOCK, bool TRACE, int CP = 0>
+template <class R, int T_LOG, int R_LOG, int BLOCK, bool TRACE, int CP = 0, bool XC = true>
 __global__ __launch_bounds__(BLOCK, BLOCK >= 1024 ? 8 : 1) void k_sort_local_ct(Bufs<R> b, IMap map, int p_top,
                                                                                 uint64_t n_valid, int fill,
                                                                                 TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
-    body_local_ct<R, T_LOG, R_LOG, BLOCK, TRACE, CP>(b, map, p_top, n_valid, fill, slot, lds, blockIdx.x);
+    body_local_ct<R, T_LOG, R_LOG, BLOCK, TRACE, CP>(b, map, p_top, n_valid, fill, slot, lds, xcd_block<XC>());
 }
 
 // Stages (p, T_LOG-1 .. 0) of one level p > T_LOG on tiles of 2^T_LOG.
@@ -306,11 +325,11 @@ __device__ __forceinline__ void body_merge(Bufs<R> b, IMap map, int p, int p_top
     if constexpr (TRACE) tcommit(slot, (uint64_t)blk * BLOCK + tau, h, nops);
 }
 
-template <class R, int T_LOG, int R_LOG, int BLOCK, bool TRACE, int CP = 0>
+template <class R, int T_LOG, int R_LOG, int BLOCK, bool TRACE, int CP = 0, bool XC = true>
 __global__ __launch_bounds__(BLOCK) void k_sort_merge(Bufs<R> b, IMap map, int p, int p_top, TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
-    body_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP>(b, map, p, p_top, slot, lds, blockIdx.x);
+    body_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP>(b, map, p, p_top, slot, lds, xcd_block<XC>());
 }
 
 // The same merge with resident blocks: each block walks tiles
@@ -401,12 +420,12 @@ __device__ __forceinline__ void body_hybrid(Bufs<R> b, IMap map, int p, int q_lo
     if constexpr (TRACE) tcommit(slot, blk * BLOCK + tau, h, nops);
 }
 
-template <class R, int T_LOG, int R_LOG, int BLOCK, int S, bool TRACE, int CP = 0>
+template <class R, int T_LOG, int R_LOG, int BLOCK, int S, bool TRACE, int CP = 0, bool XC = true>
 __global__ __launch_bounds__(BLOCK) void k_sort_hybrid(Bufs<R> b, IMap map, int p, int q_lo, int p_top,
                                                        TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
-    body_hybrid<R, T_LOG, R_LOG, BLOCK, S, TRACE, CP>(b, map, p, q_lo, p_top, slot, lds, blockIdx.x);
+    body_hybrid<R, T_LOG, R_LOG, BLOCK, S, TRACE, CP>(b, map, p, q_lo, p_top, slot, lds, xcd_block<XC>());
 }
 
 // ------------------------------------------------------------ global pass
@@ -443,11 +462,11 @@ __device__ __forceinline__ void body_global(Bufs<R> b, IMap map, int p, int q_lo
     if constexpr (TRACE) tcommit(slot, g0 + tid, h, nops);
 }
 
-template <class R, int S, bool TRACE, int CP = 0>
+template <class R, int S, bool TRACE, int CP = 0, bool XC = true>
 __global__ __launch_bounds__(256) void k_sort_global(Bufs<R> b, IMap map, int p, int q_lo, int p_top,
                                                      TraceSlot *slot)
 {
-    body_global<R, S, TRACE, CP>(b, map, p, q_lo, p_top, slot, blockIdx.x, threadIdx.x);
+    body_global<R, S, TRACE, CP>(b, map, p, q_lo, p_top, slot, xcd_block<XC>(), threadIdx.x);
 }
 
 } // namespace dev
@@ -537,7 +556,7 @@ struct SortImpl {
     }
     static int hmax(vo_ctx *ctx) { return std::min(H_MAX, ctx->tuning.max_hybrid_stages); }
 
-    template <bool TRACE, int S, int RL, int BL, int CP>
+    template <bool TRACE, int S, int RL, int BL, int CP, bool XC>
     static void hybrid_shape(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int p_top, uint64_t n_virtual)
     {
         using TL = dev::TileCT<R, T_LOG, RL, TRACE>;
@@ -546,12 +565,12 @@ struct SortImpl {
                                             "sort_hybrid_s8"};
         LaunchInfo li{names[S - 4], dim3((uint32_t)(n_virtual >> T_LOG)), dim3(BL), (uint32_t)lds,
                       hash_mix(hash_mix(p, q_lo), hash_mix(S + 100, p_top))};
-        auto k = dev::k_sort_hybrid<R, T_LOG, RL, BL, S, TRACE, CP>;
+        auto k = dev::k_sort_hybrid<R, T_LOG, RL, BL, S, TRACE, CP, XC>;
         VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         launch(ctx, li, k, b, map, p, q_lo, p_top, trace_slot(ctx));
     }
 
-    template <bool TRACE, int S, int CP>
+    template <bool TRACE, int S, int CP, bool XC>
     static void launch_hybrid(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int p_top, uint64_t n_virtual)
     {
         if constexpr (S <= H_MAX && T_LOG - S >= 5) {
@@ -563,23 +582,23 @@ struct SortImpl {
                 // the default policy even at 2^28 (5.53 vs 5.13 TB/s)
                 constexpr int CPS = S == 6 ? 0 : CP;
                 if constexpr (HW_MAX > 0)
-                    hybrid_shape<TRACE, S, R_LOG - 1, 2 * BLOCK, CPS>(ctx, b, map, p, q_lo, p_top, n_virtual);
+                    hybrid_shape<TRACE, S, R_LOG - 1, 2 * BLOCK, CPS, XC>(ctx, b, map, p, q_lo, p_top, n_virtual);
             } else {
-                hybrid_shape<TRACE, S, R_LOG, BLOCK, CP>(ctx, b, map, p, q_lo, p_top, n_virtual);
+                hybrid_shape<TRACE, S, R_LOG, BLOCK, CP, XC>(ctx, b, map, p, q_lo, p_top, n_virtual);
             }
         } else {
             throw Error{VO_ERR_INVALID, "hybrid pass width not built"};
         }
     }
 
-    template <bool TRACE, int S, int CP>
+    template <bool TRACE, int S, int CP, bool XC>
     static void launch_global(vo_ctx *ctx, const LaunchInfo &li, Bufs<R> b, IMap map, int p, int q_lo, int p_top)
     {
         if constexpr (S <= S_MAX)
-            launch(ctx, li, dev::k_sort_global<R, S, TRACE, CP>, b, map, p, q_lo, p_top, trace_slot(ctx));
+            launch(ctx, li, dev::k_sort_global<R, S, TRACE, CP, XC>, b, map, p, q_lo, p_top, trace_slot(ctx));
     }
 
-    template <bool TRACE, int CP>
+    template <bool TRACE, int CP, bool XC>
     static void global_pass(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int s, int p_top, uint64_t n_virtual)
     {
         const uint64_t threads = n_virtual >> s;
@@ -590,16 +609,16 @@ struct SortImpl {
         LaunchInfo li{names[s], dim3((uint32_t)(threads / 256)), dim3(256), 0,
                       hash_mix(hash_mix(p, q_lo), hash_mix(s, p_top))};
         switch (s) {
-        case 1: launch_global<TRACE, 1, CP>(ctx, li, b, map, p, q_lo, p_top); break;
-        case 2: launch_global<TRACE, 2, CP>(ctx, li, b, map, p, q_lo, p_top); break;
-        case 3: launch_global<TRACE, 3, CP>(ctx, li, b, map, p, q_lo, p_top); break;
-        case 4: launch_global<TRACE, 4, CP>(ctx, li, b, map, p, q_lo, p_top); break;
-        case 5: launch_global<TRACE, 5, CP>(ctx, li, b, map, p, q_lo, p_top); break;
+        case 1: launch_global<TRACE, 1, CP, XC>(ctx, li, b, map, p, q_lo, p_top); break;
+        case 2: launch_global<TRACE, 2, CP, XC>(ctx, li, b, map, p, q_lo, p_top); break;
+        case 3: launch_global<TRACE, 3, CP, XC>(ctx, li, b, map, p, q_lo, p_top); break;
+        case 4: launch_global<TRACE, 4, CP, XC>(ctx, li, b, map, p, q_lo, p_top); break;
+        case 5: launch_global<TRACE, 5, CP, XC>(ctx, li, b, map, p, q_lo, p_top); break;
         default: throw Error{VO_ERR_INVALID, "bad fused stage count"};
         }
     }
 
-    template <bool TRACE, int CP>
+    template <bool TRACE, int CP, bool XC>
     static void run_t(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill, IMap map, int p_top,
                       uint64_t n_virtual)
     {
@@ -617,7 +636,8 @@ struct SortImpl {
                 LaunchInfo li{"sort_local", dim3((uint32_t)(n_virtual >> t)), dim3(BLOCK), (uint32_t)lds,
                               hash_mix(hash_mix(t, p_top), fill)};
                 if (ct) {
-                    auto k = dev::k_sort_local_ct<R, T_LOG, R_LOG, BLOCK, TRACE, CP>;
+                    auto k = dev::k_sort_local_ct<R, T_LOG, R_LOG, BLOCK, TRACE, CP, XC>;
+                    if (!XC && tiles_xc(n_log)) k = dev::k_sort_local_ct<R, T_LOG, R_LOG, BLOCK, TRACE, CP, true>;
                     VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                     launch(ctx, li, k, b, map, p_top, n_valid, fill, trace_slot(ctx));
                 } else {
@@ -627,14 +647,14 @@ struct SortImpl {
                 }
                 break;
             }
-            case 2: global_pass<TRACE, CP>(ctx, b, map, ps.p, ps.q_lo, ps.s, p_top, n_virtual); break;
+            case 2: global_pass<TRACE, CP, XC>(ctx, b, map, ps.p, ps.q_lo, ps.s, p_top, n_virtual); break;
             case 4:
                 switch (ps.s) {
-                case 4: launch_hybrid<TRACE, 4, CP>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 5: launch_hybrid<TRACE, 5, CP>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 6: launch_hybrid<TRACE, 6, CP>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 7: launch_hybrid<TRACE, 7, CP>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 8: launch_hybrid<TRACE, 8, CP>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+                case 4: launch_hybrid<TRACE, 4, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+                case 5: launch_hybrid<TRACE, 5, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+                case 6: launch_hybrid<TRACE, 6, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+                case 7: launch_hybrid<TRACE, 7, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+                case 8: launch_hybrid<TRACE, 8, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
                 default: throw Error{VO_ERR_INVALID, "bad hybrid stage count"};
                 }
                 break;
@@ -651,7 +671,8 @@ struct SortImpl {
                     launch(ctx, li, k, b, map, ps.p, p_top, n_tiles, trace_slot(ctx));
                 } else {
                     LaunchInfo li{"sort_merge", dim3(n_tiles), dim3(BLOCK), (uint32_t)lds, hash_mix(ps.p, p_top)};
-                    auto k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP>;
+                    auto k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP, XC>;
+                    if (!XC && tiles_xc(n_log)) k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP, true>;
                     VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                     launch(ctx, li, k, b, map, ps.p, p_top, trace_slot(ctx));
                 }
@@ -666,22 +687,29 @@ struct SortImpl {
     // Measured on the 12-byte sort: +4% at 2^26 and +2.7% at 2^28, but -8% at
     // 2^24, which the MALL holds.  Resident programs keep the default (their
     // bodies are built with it); tuning bit 0x800 flips the choice.
+    static constexpr uint64_t kMallBytes = 256ull << 20;
+    static uint64_t bytes(uint64_t rows) { return rows * (8 * R::KW + sizeof(typename R::P)); }
     static bool streaming(vo_ctx *ctx, uint64_t n_virtual)
     {
-        constexpr uint64_t kMallBytes = 256ull << 20;
-        const bool big = n_virtual * (8 * R::KW + sizeof(typename R::P)) > kMallBytes;
+        const bool big = bytes(n_virtual) > kMallBytes;
         return !ctx->rec && (big != (ctx->tuning.flip_streaming != 0));
     }
+
+    // Block order of the contiguous tile passes (dev::xcd_block) of an instance
+    // above the MALL.
+    static bool tiles_xc(int n_log) { return bytes(1ull << n_log) >= 3 * kMallBytes; }
 
     static void dispatch(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill, IMap map, int p_top,
                          uint64_t n_virtual)
     {
         if (ctx->tracing)
-            run_t<true, 0>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
-        else if (streaming(ctx, n_virtual))
-            run_t<false, dev::kCpStream>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
+            run_t<true, 0, true>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
+        else if (!streaming(ctx, n_virtual))
+            run_t<false, 0, true>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
+        else if (bytes(1ull << n_log) > kMallBytes)
+            run_t<false, dev::kCpStream, false>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
         else
-            run_t<false, 0>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
+            run_t<false, dev::kCpStream, true>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
     }
 
     static void run(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill)
