@@ -311,3 +311,41 @@ def test_sort_equal_records_and_both_directions(vctx, n, npad):
     order = np.lexsort((p, k))
     assert np.array_equal(gk[:n], k[order]) and np.array_equal(gp[:n], p[order])
     assert np.array_equal(gk[n:], np.full(npad - n, M64)) and np.array_equal(gp[n:], np.arange(n, npad, dtype=np.uint32))
+
+
+@pytest.mark.parametrize("log2n", [14, 15, 16, 17, 18, 19, 21])
+@pytest.mark.parametrize("tuning", [0, 0x800])
+def test_sort_pass_schedule_by_size(log2n, tuning):
+    """The default schedule's passes that end one level and start the next
+    take another split of the tile's bits at every size; with both cache
+    policies, on the 12-byte records (odd row counts), the 16-byte ones
+    (shuffle with its permutation) and OP_SORT's ties against the oracle."""
+    import torch
+    import velodb_amd
+    print(f"schedule by size 2^{log2n} tuning={tuning:#x}", flush=True)
+    npad, n = 1 << log2n, (1 << log2n) - 37
+    rng = np.random.default_rng(log2n)
+    with velodb_amd.Context(stream=torch.cuda.current_stream().cuda_stream, tuning=tuning) as ctx:
+        k = rng.integers(0, 1 << 62, n).astype(np.uint64) >> np.uint64(rng.integers(0, 50))
+        p = np.arange(n, dtype=np.uint32)
+        gk, gp = _run_sort(ctx, k, p, n, npad)
+        order = np.lexsort((p, k))
+        assert np.array_equal(gk[:n], k[order]) and np.array_equal(gp[:n], p[order])
+        assert np.array_equal(gp[n:], np.arange(n, npad, dtype=np.uint32))
+        dp, dperm, dq = to_dev(np.arange(npad, dtype=np.uint32)), empty_dev(npad, np.uint32), to_dev(
+            np.arange(npad, dtype=np.uint32))
+        ctx.shuffle(dp, npad, 5, perm_out=dperm, n=n)
+        ctx.shuffle(dq, npad, 5, n=n)  # the 12-byte form: the same permutation
+        assert np.array_equal(from_dev(dp, np.uint32), from_dev(dperm, np.uint32))
+        assert np.array_equal(from_dev(dp, np.uint32), from_dev(dq, np.uint32))
+        if log2n <= 17:
+            types = {14: [5] * 8, 15: [4], 16: [5, 4], 17: [5, 5, 5]}[log2n]
+            asc = [i % 2 == 0 for i in range(len(types))]
+            cols = [_rand_col(rng, t, npad, 3) for t in types]
+            ecols, eidx = oracle.bitonic_sort_multi(cols, types, asc, n, npad)
+            dcols = [to_dev(c) for c in cols]
+            didx = empty_dev(npad, np.int64)
+            ctx.sort(dcols, types, asc, didx, n, npad)
+            assert np.array_equal(from_dev(didx, np.int64), eidx)
+            for dc, ec, t in zip(dcols, ecols, types):
+                assert np.array_equal(from_dev(dc, TYPES[t]).view(np.uint8), ec.view(np.uint8))

@@ -47,7 +47,7 @@
     X(kB_##TAG##_g##S, (dev::k_sort_global<R, S, false>), (dev::body_global<R, S, false>(a..., vb, threadIdx.x)), 0)
 #define VO_SORT_H(X, TAG, R, T, RL, S)                                                                             \
     X(kB_##TAG##_h##S, (dev::k_sort_hybrid<R, T, RL, 256, S, false>),                                              \
-      (dev::body_hybrid<R, T, RL, 256, S, false>(a..., lds, vb)), 0)
+      (dev::body_strided<R, T, RL, 256, T - S, false, false>(a..., lds, vb)), 0)
 
 // (u64 key, u32 payload) at the resident tile 2^12 (launch mode: 2^13 with
 // 512 threads; the network is the same); register passes 1..5, LDS 4..7.

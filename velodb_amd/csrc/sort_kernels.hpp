@@ -375,48 +375,71 @@ __global__ __launch_bounds__(BLOCK) void k_sort_merge_pipe(Bufs<R> b, IMap map, 
     if constexpr (TRACE) tcommit(slot, (uint64_t)blockIdx.x * BLOCK + tau, h, nops);
 }
 
-// ------------------------------------------------------------ hybrid pass
+// ------------------------------------------------------ LDS-staged passes
 
-// S fused stages (p, q_lo+S-1 .. q_lo) with S up to 7, staged through LDS.
-// A block holds 2^T_LOG records: 2^S runs of C = T_LOG - S contiguous
+// A strided tile of 2^T_LOG records: 2^(T_LOG - C) runs of 2^C contiguous
 // records, run r starting at element ubase + r * 2^q_lo.  Tile-local index l
 // maps to element (l mod 2^C) + (l >> C) * 2^q_lo (plus the block's uniform
-// bits), so tile bits [C, T_LOG) are the stage bits and the stages run as a
-// tile schedule on them.  With C >= 6 a wavefront's 64 lanes always read
-// and write 64 consecutive records.
-template <class R, int T_LOG, int R_LOG, int BLOCK, int S, bool TRACE, int CP = 0>
-__device__ __forceinline__ void body_hybrid(Bufs<R> b, IMap map, int p, int q_lo, int p_top, TraceSlot *slot,
-                                            char *lds, uint32_t blk32)
+// bits), so tile bits [0, C) are the array's low bits and tile bits
+// [C, T_LOG) its bits [q_lo, q_lo + T_LOG - C).  Two passes run on it:
+//   * hybrid (TAIL = false): the S = T_LOG - C stages (p, q_lo+S-1 .. q_lo);
+//   * wrap (TAIL = true, q_lo + S == p): the end of level p - 1, its stages
+//     C-1 .. 0, and then the start of level p, its stages p-1 .. q_lo.  A
+//     level's end and the next one's start need the array's lowest and
+//     highest bits, which a tile of contiguous records and a hybrid tile
+//     hold only one half of each; a wrap tile holds both, so one trip to
+//     memory does the work of two.
+// A tile is loaded and stored in whatever layout its first and last stages
+// run in (at least 16 consecutive lanes on consecutive records), which saves
+// the relayouts from and to the layout of 64.
+template <int T_LOG, int R_LOG>
+constexpr int strided_load_layout(int c, bool tail)
+{
+    int a = T_LOG - R_LOG;
+    if (tail)
+        while (a > c - 1 && a - R_LOG >= 4) a -= R_LOG;
+    return a;
+}
+
+template <class R, int T_LOG, int R_LOG, int BLOCK, int C, bool TAIL, bool TRACE, int CP = 0>
+__device__ __forceinline__ void body_strided(Bufs<R> b, IMap map, int p, int q_lo, int p_top, TraceSlot *slot,
+                                             char *lds, uint32_t blk32)
 {
     using TL = TileCT<R, T_LOG, R_LOG, TRACE>;
-    constexpr int C = T_LOG - S;
-    constexpr int A0 = T_LOG - R_LOG;
-    static_assert(C >= 5 && A0 >= 6, "runs of at least 32 records; lanes cover 64 tile-local records");
+    constexpr int S = T_LOG - C;
+    constexpr int AL = strided_load_layout<T_LOG, R_LOG>(C, TAIL);
+    constexpr int AT = TAIL ? TL::end_layout(C - 1, AL) : AL;
+    constexpr int AS = TL::end_layout(T_LOG - 1, AT, C);
+    static_assert(C >= 5 && AL >= 4 && AS >= 4, "runs of at least 32 records, 16 lanes on each");
     const uint32_t tau = threadIdx.x;
-    const uint32_t lane = tau & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tau >> 6);
     const uint64_t blk = blk32;
     const uint64_t b_lo = blk & ((1ull << (q_lo - C)) - 1);
     const uint64_t b_hi = blk >> (q_lo - C);
     const uint64_t ublk = (b_lo << C) | (b_hi << (q_lo + S));
-    // element offset of tile-local index l (a bit permutation, additive over disjoint bit fields)
-    auto eoff = [&](uint64_t l) { return (l & ((1ull << C) - 1)) | ((l >> C) << q_lo); };
-    const uint64_t vw = ublk + eoff((uint64_t)wave << 6);
-    const uint64_t pw = map_uniform(map, vw);
-    // per-lane offset: with runs of 64 or more the wavefront is one run; with
-    // runs of 32 its upper half is the next run, 2^q_lo records further
-    // (below 2^29 elements, so the byte offset fits the 32-bit field)
-    const uint32_t vl = C >= 6 ? lane : ((lane & 31u) | ((lane >> 5) << q_lo));
+    const uint64_t pb = map_uniform(map, ublk);
+    // element offset of tile-local index l (a bit permutation, additive over
+    // disjoint bit fields; below 2^29, so a byte offset fits 32 bits)
+    auto eoff = [&](uint32_t l) { return (l & ((1u << C) - 1)) | ((l >> C) << q_lo); };
     uint64_t h = 0;
     uint32_t nops = 0;
     R r[1 << R_LOG];
+    {
+        const uint32_t vl = eoff(lay_base<R_LOG>(tau, AL));
 #pragma unroll
-    for (int m = 0; m < (1 << R_LOG); ++m) gload_u<R, TRACE, CP>(r[m], b, pw + eoff((uint64_t)m << A0), vl, h, nops);
+        for (int m = 0; m < (1 << R_LOG); ++m)
+            gload_u<R, TRACE, CP>(r[m], b, pb + eoff((uint32_t)m << AL), vl, h, nops);
+    }
+    // tile bit T_LOG - 1 is array bit p - 1, the direction bit of level p - 1
+    // (which is below the top level)
+    if constexpr (TAIL) TL::template level<T_LOG - 1, C - 1, AL>(r, lds, tau, false, 64, h, nops);
     const bool asc = dir_asc(ublk, p, p_top);
-    TL::template level<-1, T_LOG - 1, A0, C>(r, lds, tau, asc, p_top, h, nops);
-    TL::template relayout<TL::end_layout(T_LOG - 1, A0, C), A0>(r, lds, tau, h, nops);
+    TL::template level<-1, T_LOG - 1, AT, C>(r, lds, tau, asc, p_top, h, nops);
+    {
+        const uint32_t vs = eoff(lay_base<R_LOG>(tau, AS));
 #pragma unroll
-    for (int m = 0; m < (1 << R_LOG); ++m) gstore_u<R, TRACE, CP>(r[m], b, pw + eoff((uint64_t)m << A0), vl, h, nops);
+        for (int m = 0; m < (1 << R_LOG); ++m)
+            gstore_u<R, TRACE, CP>(r[m], b, pb + eoff((uint32_t)m << AS), vs, h, nops);
+    }
     if constexpr (TRACE) tcommit(slot, blk * BLOCK + tau, h, nops);
 }
 
@@ -425,7 +448,16 @@ __global__ __launch_bounds__(BLOCK) void k_sort_hybrid(Bufs<R> b, IMap map, int 
                                                        TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
-    body_hybrid<R, T_LOG, R_LOG, BLOCK, S, TRACE, CP>(b, map, p, q_lo, p_top, slot, lds, xcd_block<XC>());
+    body_strided<R, T_LOG, R_LOG, BLOCK, T_LOG - S, false, TRACE, CP>(b, map, p, q_lo, p_top, slot, lds,
+                                                                      xcd_block<XC>());
+}
+
+template <class R, int T_LOG, int R_LOG, int BLOCK, int S, bool TRACE, int CP = 0, bool XC = true>
+__global__ __launch_bounds__(BLOCK) void k_sort_wrap(Bufs<R> b, IMap map, int p, int q_lo, int p_top, TraceSlot *slot)
+{
+    extern __shared__ __align__(16) char lds[];
+    body_strided<R, T_LOG, R_LOG, BLOCK, T_LOG - S, true, TRACE, CP>(b, map, p, q_lo, p_top, slot, lds,
+                                                                     xcd_block<XC>());
 }
 
 // ------------------------------------------------------------ global pass
@@ -483,7 +515,7 @@ using dev::IMap;
 constexpr uint64_t kMaxSortRows = 1ull << 29;
 
 struct Pass {
-    int kind; // 0 tiny, 1 local, 2 global, 3 merge
+    int kind; // 0 tiny, 1 local, 2 global, 3 merge, 4 hybrid, 5 wrap
     int p, q_lo, s;
 };
 
@@ -537,6 +569,57 @@ inline std::vector<Pass> plan_passes(int n_log, int t_log, int s_max, int r_log,
     return v;
 }
 
+// The default schedule: the cheapest sequence of passes over the stages above
+// the tile, in network order, where a pass may also end one level and start the
+// next (wrap).  Found by dynamic programming from the end over (level p, next
+// stage q); the costs are one pass's time at 2^28 records relative to a copy of
+// the array (below the MALL the order is the same).  A level-by-level schedule
+// needs ceil((p - t_log) / h_max) + 1 passes for level p; this one comes close
+// to (p - 5) / h_max on average: 31 passes instead of 38 at 2^28 on 2^13-record
+// tiles, 18 instead of 23 at 2^23.
+inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int s_max, int r_log, int h_max)
+{
+    std::vector<Pass> v;
+    if (n_log <= t_log) return plan_passes(n_log, t_log, s_max, r_log);
+    v.push_back({1, t_log, 0, t_log});
+    struct Best {
+        float cost;
+        Pass pass;
+        int p, q; // state after the pass
+    };
+    std::vector<std::vector<Best>> best(n_log + 2, std::vector<Best>(n_log + 1, Best{0.f, {}, 0, 0}));
+    for (int p = n_log; p > t_log; --p)
+        for (int q = 0; q < p; ++q) {
+            Best &b = best[p][q];
+            b.cost = 1e30f;
+            // the pass ends at (p2, q2); stage -1 of a level is the start of the next
+            auto consider = [&](float cost, Pass ps, int p2, int q2) {
+                if (q2 < 0) {
+                    ++p2;
+                    q2 = p2 - 1;
+                }
+                const float c = cost + (p2 > n_log ? 0.f : best[p2][q2].cost);
+                if (c < b.cost) b = Best{c, ps, p2, q2};
+            };
+            for (int s = 1; s <= s_max && q - s + 1 >= 8; ++s)
+                consider(s <= 3 ? 1.f : 1.08f, {2, p, q - s + 1, s}, p, q - s);
+            for (int s = 4; s <= h_max; ++s)
+                if (q - s + 1 >= t_log - s) consider(s <= 7 ? 1.1f : 1.14f, {4, p, q - s + 1, s}, p, q - s);
+            if (q < t_log) consider(1.12f, {3, p, 0, 0}, p, -1);
+            // stages q .. 0 and the next level's first s (a run of 32 records
+            // may repeat a stage above q, which changes nothing)
+            const int c = std::max(5, q + 1), s = t_log - c;
+            if (s >= 1 && p < n_log) consider(c <= 5 ? 1.17f : 1.13f, {5, p + 1, p + 1 - s, s}, p + 1, p - s);
+        }
+    for (int p = t_log + 1, q = t_log; p <= n_log;) {
+        const Best &b = best[p][q];
+        v.push_back(b.pass);
+        p = b.p;
+        q = b.q;
+    }
+    return v;
+}
+
 // S_LARGE / LARGE_LOG: from n_pad = 2^LARGE_LOG up, register passes take at
 // most S_LARGE stages (wider groups go to the hybrid pass); below, S_MAX.
 // Hybrid passes of at most HW_MAX stages run with twice the threads per block
@@ -555,6 +638,25 @@ struct SortImpl {
         return std::max(1, std::min(cap, ctx->tuning.max_fused_stages));
     }
     static int hmax(vo_ctx *ctx) { return std::min(H_MAX, ctx->tuning.max_hybrid_stages); }
+
+    // The default tuning runs the wrapped schedule; a tuning word that picks
+    // pass widths or block shapes, and recorded programs (whose bodies they
+    // are), run level by level.
+    static std::vector<Pass> plan(vo_ctx *ctx, int n_log)
+    {
+        const SortTuning &t = ctx->tuning, d;
+        const bool wrapped = !ctx->rec && t.max_fused_stages == d.max_fused_stages &&
+                             t.max_hybrid_stages == d.max_hybrid_stages && !t.pipe_merge && !t.wide_block &&
+                             !t.flip_hybrid_block;
+        if (!wrapped) return plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx));
+        static const std::vector<std::vector<Pass>> plans = [] {
+            std::vector<std::vector<Pass>> v;
+            for (int l = 0; (1ull << l) <= kMaxSortRows; ++l)
+                v.push_back(plan_wrapped(l, T_LOG, l >= LARGE_LOG ? S_LARGE : S_MAX, R_LOG, H_MAX));
+            return v;
+        }();
+        return plans[n_log];
+    }
 
     template <bool TRACE, int S, int RL, int BL, int CP, bool XC>
     static void hybrid_shape(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int p_top, uint64_t n_virtual)
@@ -591,6 +693,25 @@ struct SortImpl {
         }
     }
 
+    // Wrap passes of S = 1 .. T_LOG - 5 stages of the upper level.
+    template <bool TRACE, int CP, bool XC, int S = 1>
+    static void launch_wrap(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int s, int p_top, uint64_t n_virtual)
+    {
+        if constexpr (S <= T_LOG - 5) {
+            if (s != S) return launch_wrap<TRACE, CP, XC, S + 1>(ctx, b, map, p, q_lo, s, p_top, n_virtual);
+            static const char *const names[] = {"sort_wrap_s1", "sort_wrap_s2", "sort_wrap_s3", "sort_wrap_s4",
+                                                "sort_wrap_s5", "sort_wrap_s6", "sort_wrap_s7", "sort_wrap_s8"};
+            const size_t lds = dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes();
+            LaunchInfo li{names[S - 1], dim3((uint32_t)(n_virtual >> T_LOG)), dim3(BLOCK), (uint32_t)lds,
+                          hash_mix(hash_mix(p, q_lo), hash_mix(S + 200, p_top))};
+            auto k = dev::k_sort_wrap<R, T_LOG, R_LOG, BLOCK, S, TRACE, CP, XC>;
+            VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            launch(ctx, li, k, b, map, p, q_lo, p_top, trace_slot(ctx));
+        } else {
+            throw Error{VO_ERR_INVALID, "bad wrap stage count"};
+        }
+    }
+
     template <bool TRACE, int S, int CP, bool XC>
     static void launch_global(vo_ctx *ctx, const LaunchInfo &li, Bufs<R> b, IMap map, int p, int q_lo, int p_top)
     {
@@ -622,7 +743,7 @@ struct SortImpl {
     static void run_t(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill, IMap map, int p_top,
                       uint64_t n_virtual)
     {
-        for (const Pass &ps : plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx))) {
+        for (const Pass &ps : plan(ctx, n_log)) {
             switch (ps.kind) {
             case 0: {
                 LaunchInfo li{"sort_tiny", dim3(1), dim3(64), 0, hash_mix(n_log, fill)};
@@ -658,6 +779,7 @@ struct SortImpl {
                 default: throw Error{VO_ERR_INVALID, "bad hybrid stage count"};
                 }
                 break;
+            case 5: launch_wrap<TRACE, CP, XC>(ctx, b, map, ps.p, ps.q_lo, ps.s, p_top, n_virtual); break;
             case 3: {
                 const size_t lds = dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes();
                 const uint32_t n_tiles = (uint32_t)(n_virtual >> T_LOG);
@@ -728,7 +850,7 @@ struct SortImpl {
         dispatch(ctx, b, c, 0, 1, IMap{offsets, c, ns}, c, count << c);
     }
 
-    static int passes(vo_ctx *ctx, int n_log) { return (int)plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx)).size(); }
+    static int passes(vo_ctx *ctx, int n_log) { return (int)plan(ctx, n_log).size(); }
 };
 
 // Record kinds and their tile shapes (LDS = 2^T_LOG * 17/16 * record bytes).
