@@ -357,12 +357,23 @@ __device__ __forceinline__ void tile_level(R (&r)[1 << R_LOG], const Lds<R> &s, 
 // Same schedule as tile_level, with the tile size, every layout and every
 // level fixed at compile time, so that all LDS offsets are immediates and the
 // stage loops fully unroll.  Used for full 2^T_LOG tiles.
+// A block's relayout buffer.  shared: other waves may still read what they (or
+// the block's last tile) moved through it.
+struct TileBuf {
+    char *p;
+    bool shared = true;
+};
+
 template <class R, int T_LOG, int R_LOG, bool TRACE>
 struct TileCT {
     static constexpr int RR = 1 << R_LOG;
     static constexpr uint32_t T = 1u << T_LOG;
     static constexpr uint32_t TPAD = T + (T >> 4);
     using P = typename R::P;
+
+    // Layout in which contiguous tiles meet memory when their stages leave the
+    // choice: 64 lanes on consecutive records, a wavefront on its own ones.
+    static constexpr int A_IO = T_LOG - R_LOG < 6 ? T_LOG - R_LOG : 6;
 
     // layout reached after stages (q_start .. 0) starting from layout a;
     // stage 0 in layout 1 runs across lane pairs and keeps the layout
@@ -432,44 +443,6 @@ struct TileCT {
         }
     }
 
-    template <int A>
-    static __device__ __forceinline__ void put(const R (&r)[RR], char *lds, uint32_t tau, uint64_t &h, uint32_t &n)
-    {
-        uint64_t *sk = reinterpret_cast<uint64_t *>(lds);
-        P *sp = reinterpret_cast<P *>(lds + sizeof(uint64_t) * R::KW * TPAD);
-        const uint32_t lb = lpos(lay_base<R_LOG>(tau, A));
-#pragma unroll
-        for (int m = 0; m < RR; ++m) {
-            const uint32_t l = lb + lpos((uint32_t)m << A);
-#pragma unroll
-            for (int w = 0; w < R::KW; ++w) sk[w * TPAD + l] = r[m].k[w];
-            sp[l] = r[m].p;
-            if constexpr (TRACE) {
-                h = tfold(h, 3, l);
-                ++n;
-            }
-        }
-    }
-
-    template <int A>
-    static __device__ __forceinline__ void get(R (&r)[RR], char *lds, uint32_t tau, uint64_t &h, uint32_t &n)
-    {
-        const uint64_t *sk = reinterpret_cast<const uint64_t *>(lds);
-        const P *sp = reinterpret_cast<const P *>(lds + sizeof(uint64_t) * R::KW * TPAD);
-        const uint32_t lb = lpos(lay_base<R_LOG>(tau, A));
-#pragma unroll
-        for (int m = 0; m < RR; ++m) {
-            const uint32_t l = lb + lpos((uint32_t)m << A);
-#pragma unroll
-            for (int w = 0; w < R::KW; ++w) r[m].k[w] = sk[w * TPAD + l];
-            r[m].p = sp[l];
-            if constexpr (TRACE) {
-                h = tfold(h, 4, l);
-                ++n;
-            }
-        }
-    }
-
     // LDS bytes of one block: a single column buffer (the widest column)
     // that every column passes through in turn.  Keeping it to 8 B per slot
     // lets two 2^13-record tiles share a CU's 160 KB.
@@ -505,31 +478,71 @@ struct TileCT {
         }
     }
 
+    // Layouts up to 6 hold the 64 << R_LOG records of a wavefront in tile order
+    // (the thread bits above the lane's are the tile's top bits), so a relayout
+    // between two of them stays inside one wavefront: it runs in the
+    // wavefront's own part of the buffer without a barrier, and the waves of a
+    // block drift apart, one's LDS phase over another's compare-exchanges.
+    // (With barriers in all 23 relayouts of the local pass its VALU and LDS
+    // times added up.)
+    static constexpr bool in_wave(int a_old, int a_new) { return a_old <= 6 && a_new <= 6; }
+
+    // Keeps the LDS accesses before and after in order for the compiler; a
+    // wavefront's own are in order in hardware.
+    static __device__ __forceinline__ void wave_fence()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+
+    template <int A_OLD, int A_NEW, typename C>
+    static __device__ __forceinline__ void move_col(C (&v)[RR], C *buf, uint32_t tau, uint64_t &h, uint32_t &n)
+    {
+        put_col<A_OLD>(v, buf, tau, h, n);
+        if constexpr (in_wave(A_OLD, A_NEW))
+            wave_fence();
+        else
+            __syncthreads();
+        get_col<A_NEW>(v, buf, tau, h, n);
+    }
+
+    // Before a column enters the buffer: every wave is done with what it read
+    // there.  Between relayouts inside the wavefronts each wave only uses its
+    // own part, [lpos(first record), ...) of 8 bytes a record.
     template <int A_OLD, int A_NEW>
-    static __device__ __forceinline__ void relayout(R (&r)[RR], char *lds, uint32_t tau, uint64_t &h, uint32_t &n)
+    static __device__ __forceinline__ void relayout(R (&r)[RR], TileBuf &lds, uint32_t tau, uint64_t &h, uint32_t &n)
     {
         if constexpr (A_OLD != A_NEW) {
+            constexpr bool IN = in_wave(A_OLD, A_NEW);
+            if (lds.shared || A_OLD > 6)
+                __syncthreads();
+            else
+                wave_fence();
 #pragma unroll
             for (int w = 0; w < R::KW; ++w) {
                 uint64_t v[RR];
 #pragma unroll
                 for (int m = 0; m < RR; ++m) v[m] = r[m].k[w];
-                __syncthreads();
-                put_col<A_OLD>(v, reinterpret_cast<uint64_t *>(lds), tau, h, n);
-                __syncthreads();
-                get_col<A_NEW>(v, reinterpret_cast<const uint64_t *>(lds), tau, h, n);
+                move_col<A_OLD, A_NEW>(v, reinterpret_cast<uint64_t *>(lds.p), tau, h, n);
+                if constexpr (IN)
+                    wave_fence();
+                else
+                    __syncthreads();
 #pragma unroll
                 for (int m = 0; m < RR; ++m) r[m].k[w] = v[m];
             }
             P v[RR];
 #pragma unroll
             for (int m = 0; m < RR; ++m) v[m] = r[m].p;
-            __syncthreads();
-            put_col<A_OLD>(v, reinterpret_cast<P *>(lds), tau, h, n);
-            __syncthreads();
-            get_col<A_NEW>(v, reinterpret_cast<const P *>(lds), tau, h, n);
+            P *buf = reinterpret_cast<P *>(lds.p);
+            // a narrower column starts where the wavefront's 8-byte part does
+            if constexpr (IN && sizeof(P) < 8)
+                buf += lpos(__builtin_amdgcn_readfirstlane(tau >> 6) << (6 + R_LOG)) * (8 / sizeof(P) - 1);
+            move_col<A_OLD, A_NEW>(v, buf, tau, h, n);
 #pragma unroll
             for (int m = 0; m < RR; ++m) r[m].p = v[m];
+            lds.shared = !IN;
         }
     }
 
@@ -559,7 +572,7 @@ struct TileCT {
 
     // Stages (P, Q .. QLO) from layout A, changing layout as needed.
     template <int P, int Q, int A, int QLO = 0>
-    static __device__ __forceinline__ void level(R (&r)[RR], char *lds, uint32_t tau, bool asc_hi, int p_top,
+    static __device__ __forceinline__ void level(R (&r)[RR], TileBuf &lds, uint32_t tau, bool asc_hi, int p_top,
                                                  uint64_t &h, uint32_t &n)
     {
         if constexpr (LANE0 && Q == 0 && A == 1 && QLO == 0) {
@@ -583,7 +596,7 @@ struct TileCT {
     }
 
     template <int P, int A>
-    static __device__ __forceinline__ void levels(R (&r)[RR], char *lds, uint32_t tau, bool asc_hi, int p_top,
+    static __device__ __forceinline__ void levels(R (&r)[RR], TileBuf &lds, uint32_t tau, bool asc_hi, int p_top,
                                                   uint64_t &h, uint32_t &n)
     {
         if constexpr (P <= T_LOG) {

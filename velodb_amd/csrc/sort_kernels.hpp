@@ -266,7 +266,8 @@ __device__ __forceinline__ void body_local_ct(Bufs<R> b, IMap map, int p_top, ui
                                               TraceSlot *slot, char *lds, uint32_t blk)
 {
     using TL = TileCT<R, T_LOG, R_LOG, TRACE>;
-    constexpr int A0 = T_LOG - R_LOG;
+    constexpr int A0 = TL::A_IO;
+    TileBuf buf{lds};
     const uint32_t tau = threadIdx.x;
     const uint64_t vbase = (uint64_t)blk << T_LOG;
     const uint64_t pbase = map_uniform(map, vbase);
@@ -283,8 +284,8 @@ __device__ __forceinline__ void body_local_ct(Bufs<R> b, IMap map, int p_top, ui
         }
     }
     const bool asc_hi = dir_asc(vbase, T_LOG, p_top);
-    TL::template levels<1, A0>(r, lds, tau, asc_hi, p_top, h, nops);
-    TL::template relayout<TL::end_all(1, A0), A0>(r, lds, tau, h, nops);
+    TL::template levels<1, A0>(r, buf, tau, asc_hi, p_top, h, nops);
+    TL::template relayout<TL::end_all(1, A0), A0>(r, buf, tau, h, nops);
 #pragma unroll
     for (int m = 0; m < (1 << R_LOG); ++m) gstore_t<R, TRACE, CP>(r[m], b, pbase, (uint32_t)m << A0, base, h, nops);
     if constexpr (TRACE) tcommit(slot, (uint64_t)blk * BLOCK + tau, h, nops);
@@ -307,7 +308,8 @@ __device__ __forceinline__ void body_merge(Bufs<R> b, IMap map, int p, int p_top
                                            uint32_t blk)
 {
     using TL = TileCT<R, T_LOG, R_LOG, TRACE>;
-    constexpr int A0 = T_LOG - R_LOG;
+    constexpr int A0 = T_LOG - R_LOG, AS = TL::A_IO;
+    TileBuf buf{lds};
     const uint32_t tau = threadIdx.x;
     const uint64_t vbase = (uint64_t)blk << T_LOG;
     const uint64_t pbase = map_uniform(map, vbase);
@@ -318,10 +320,11 @@ __device__ __forceinline__ void body_merge(Bufs<R> b, IMap map, int p, int p_top
 #pragma unroll
     for (int m = 0; m < (1 << R_LOG); ++m) gload_t<R, TRACE, CP>(r[m], b, pbase, (uint32_t)m << A0, base, h, nops);
     const bool asc = dir_asc(vbase, p, p_top);
-    TL::template level<-1, T_LOG - 1, A0>(r, lds, tau, asc, p_top, h, nops);
-    TL::template relayout<TL::end_layout(T_LOG - 1, A0), A0>(r, lds, tau, h, nops);
+    TL::template level<-1, T_LOG - 1, A0>(r, buf, tau, asc, p_top, h, nops);
+    TL::template relayout<TL::end_layout(T_LOG - 1, A0), AS>(r, buf, tau, h, nops);
 #pragma unroll
-    for (int m = 0; m < (1 << R_LOG); ++m) gstore_t<R, TRACE, CP>(r[m], b, pbase, (uint32_t)m << A0, base, h, nops);
+    for (int m = 0; m < (1 << R_LOG); ++m)
+        gstore_t<R, TRACE, CP>(r[m], b, pbase, (uint32_t)m << AS, lay_base<R_LOG>(tau, AS), h, nops);
     if constexpr (TRACE) tcommit(slot, (uint64_t)blk * BLOCK + tau, h, nops);
 }
 
@@ -344,6 +347,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_merge_pipe(Bufs<R> b, IMap map, 
     constexpr int A0 = T_LOG - R_LOG;
     constexpr int RR = 1 << R_LOG;
     extern __shared__ __align__(16) char lds[];
+    TileBuf buf{lds};
     const uint32_t tau = threadIdx.x;
     const uint32_t base = lay_base<R_LOG>(tau, A0);
     uint64_t h = 0;
@@ -365,8 +369,8 @@ __global__ __launch_bounds__(BLOCK) void k_sort_merge_pipe(Bufs<R> b, IMap map, 
         const uint64_t vbase = (uint64_t)t << T_LOG;
         const uint64_t pbase = map_uniform(map, vbase);
         const bool asc = dir_asc(vbase, p, p_top);
-        TL::template level<-1, T_LOG - 1, A0>(cur, lds, tau, asc, p_top, h, nops);
-        TL::template relayout<TL::end_layout(T_LOG - 1, A0), A0>(cur, lds, tau, h, nops);
+        TL::template level<-1, T_LOG - 1, A0>(cur, buf, tau, asc, p_top, h, nops);
+        TL::template relayout<TL::end_layout(T_LOG - 1, A0), A0>(cur, buf, tau, h, nops);
 #pragma unroll
         for (int m = 0; m < RR; ++m) gstore_t<R, TRACE>(cur[m], b, pbase, (uint32_t)m << A0, base, h, nops);
 #pragma unroll
@@ -407,6 +411,7 @@ __device__ __forceinline__ void body_strided(Bufs<R> b, IMap map, int p, int q_l
 {
     using TL = TileCT<R, T_LOG, R_LOG, TRACE>;
     constexpr int S = T_LOG - C;
+    TileBuf buf{lds};
     constexpr int AL = strided_load_layout<T_LOG, R_LOG>(C, TAIL);
     constexpr int AT = TAIL ? TL::end_layout(C - 1, AL) : AL;
     constexpr int AS = TL::end_layout(T_LOG - 1, AT, C);
@@ -431,9 +436,9 @@ __device__ __forceinline__ void body_strided(Bufs<R> b, IMap map, int p, int q_l
     }
     // tile bit T_LOG - 1 is array bit p - 1, the direction bit of level p - 1
     // (which is below the top level)
-    if constexpr (TAIL) TL::template level<T_LOG - 1, C - 1, AL>(r, lds, tau, false, 64, h, nops);
+    if constexpr (TAIL) TL::template level<T_LOG - 1, C - 1, AL>(r, buf, tau, false, 64, h, nops);
     const bool asc = dir_asc(ublk, p, p_top);
-    TL::template level<-1, T_LOG - 1, AT, C>(r, lds, tau, asc, p_top, h, nops);
+    TL::template level<-1, T_LOG - 1, AT, C>(r, buf, tau, asc, p_top, h, nops);
     {
         const uint32_t vs = eoff(lay_base<R_LOG>(tau, AS));
 #pragma unroll
