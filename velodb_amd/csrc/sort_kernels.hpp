@@ -55,57 +55,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *ubase)
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-template <int CP = 0, typename T>
-__device__ __forceinline__ T ld_u(const T *ubase, uint32_t vi)
-{
-    const __amdgpu_buffer_rsrc_t r = buf_rsrc(ubase);
-    if constexpr (sizeof(T) == 8) {
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, vi * 8u, 0, CP));
-    } else {
-        static_assert(sizeof(T) == 4, "4- or 8-byte columns");
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, vi * 4u, 0, CP));
-    }
-}
-
-template <int CP = 0, typename T>
-__device__ __forceinline__ void st_u(T *ubase, uint32_t vi, T v)
-{
-    const __amdgpu_buffer_rsrc_t r = buf_rsrc(ubase);
-    if constexpr (sizeof(T) == 8) {
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, vi * 8u, 0, CP);
-    } else {
-        static_assert(sizeof(T) == 4, "4- or 8-byte columns");
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, vi * 4u, 0, CP);
-    }
-}
-
-// Record at uniform index u plus per-thread offset vi.
-template <class R, bool TRACE, int CP = 0>
-__device__ __forceinline__ void gload_u(R &r, const Bufs<R> &b, uint64_t u, uint32_t vi, uint64_t &h, uint32_t &n)
-{
-#pragma unroll
-    for (int w = 0; w < R::KW; ++w) r.k[w] = ld_u<CP>(b.k[w] + u, vi);
-    r.p = ld_u<CP>(b.p + u, vi);
-    if constexpr (TRACE) {
-        h = tfold(h, 1, u + vi);
-        ++n;
-    }
-}
-
-template <class R, bool TRACE, int CP = 0>
-__device__ __forceinline__ void gstore_u(const R &r, const Bufs<R> &b, uint64_t u, uint32_t vi, uint64_t &h,
-                                         uint32_t &n)
-{
-#pragma unroll
-    for (int w = 0; w < R::KW; ++w) st_u<CP>(b.k[w] + u, vi, r.k[w]);
-    st_u<CP>(b.p + u, vi, r.p);
-    if constexpr (TRACE) {
-        h = tfold(h, 2, u + vi);
-        ++n;
-    }
-}
-
-
 // Tile form: one buffer resource per column for the tile's uniform base u,
 // the per-register offset so (elements, uniform, < 2^16) in the scalar
 // offset field and the per-thread offset vi in the vector offset.
@@ -432,7 +381,7 @@ __device__ __forceinline__ void body_strided(Bufs<R> b, IMap map, int p, int q_l
         const uint32_t vl = eoff(lay_base<R_LOG>(tau, AL));
 #pragma unroll
         for (int m = 0; m < (1 << R_LOG); ++m)
-            gload_u<R, TRACE, CP>(r[m], b, pb + eoff((uint32_t)m << AL), vl, h, nops);
+            gload_t<R, TRACE, CP>(r[m], b, pb, eoff((uint32_t)m << AL), vl, h, nops);
     }
     // tile bit T_LOG - 1 is array bit p - 1, the direction bit of level p - 1
     // (which is below the top level)
@@ -443,7 +392,7 @@ __device__ __forceinline__ void body_strided(Bufs<R> b, IMap map, int p, int q_l
         const uint32_t vs = eoff(lay_base<R_LOG>(tau, AS));
 #pragma unroll
         for (int m = 0; m < (1 << R_LOG); ++m)
-            gstore_u<R, TRACE, CP>(r[m], b, pb + eoff((uint32_t)m << AS), vs, h, nops);
+            gstore_t<R, TRACE, CP>(r[m], b, pb, eoff((uint32_t)m << AS), vs, h, nops);
     }
     if constexpr (TRACE) tcommit(slot, blk * BLOCK + tau, h, nops);
 }
