@@ -227,3 +227,32 @@ def test_filter_sum_3e8_rows_2p29(vctx):
     assert torch.equal(op[:m], p[sel]) and torch.equal(od[:m], c[sel])
     del day, qty, price, disc, op, od, d, q, p, c, sel
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("log2n", [12, 13, 14, 16, 17, 20, 21, 22, 23])
+@pytest.mark.parametrize("widths", [(8, 8), (8, 4, 1), (2,)])
+@pytest.mark.parametrize("tuning", [0, 0x800])
+def test_compact_pass_shapes(log2n, widths, tuning):
+    """Every split of the levels over 2^12- and 2^13-row tiles and over the
+    passes above them, with both cache policies, column widths mixed, odd
+    row counts and a mask at an odd address: whole columns against the
+    oracle's network."""
+    import torch
+    import velodb_amd
+    print(f"compact shapes 2^{log2n} widths={widths} tuning={tuning:#x}", flush=True)
+    npad, n = 1 << log2n, (1 << log2n) - 11
+    rng = np.random.default_rng(log2n)
+    mask = (rng.random(npad) < 0.3).astype(np.uint8) * rng.integers(1, 255, npad).astype(np.uint8)
+    sel = mask.copy()
+    sel[n:] = 0
+    cols = [rng.integers(0, 1 << (8 * w - 1), npad).astype({1: np.uint8, 2: np.uint16, 4: np.uint32, 8: np.uint64}[w])
+            for w in widths]
+    off = log2n % 3  # alignment of the mask
+    dm = torch.from_numpy(np.concatenate([np.zeros(off, np.uint8), mask])).cuda()[off:]
+    dc = [to_dev(c) for c in cols]
+    cnt = torch.zeros(1, dtype=torch.int64, device="cuda:0")
+    with velodb_amd.Context(stream=torch.cuda.current_stream().cuda_stream, tuning=tuning) as ctx:
+        ctx.compact(dm, dc, list(widths), n, npad, out_count=cnt)
+    assert int(cnt.item()) == int((sel != 0).sum())
+    want = oracle.compact(_rows(cols), (sel != 0).astype(np.uint8))
+    assert np.array_equal(_rows([from_dev(d, c.dtype) for d, c in zip(dc, cols)]), want)

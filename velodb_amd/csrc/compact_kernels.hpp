@@ -13,8 +13,13 @@
 //   s  > 2 : m1 = C[b+half] - C[b], om = o mod half, om1 = (o+m1) mod half,
 //            swap = ((om + m1 >= half) ^ (o >= half)) ^ (i >= om1)
 // (the offset form of :88-105; the chain of :121-153 reduces to o = C[b]
-// mod s for the blocks it creates).  Every row is read and written at every
-// level; the swap decision is a select, so addresses depend on n_pad only.
+// mod s for the blocks it creates).  With D = C[b+half] = C[b] + m1 the second
+// form is one bit: om1 is D mod half, the first exclusive-or is bit q of D
+// (C[b]'s bit q plus the carry of om + m1), and adding half-1-i to D carries
+// into bit q exactly when i < om1, so
+//   s  > 2 : swap = !bit q of (D + half - 1 - i).
+// Every row is read and written at every level; the swap decision is a select,
+// so addresses depend on n_pad only.
 //
 // Passes: count (selected rows per tile) -> tile scan -> local levels
 // q < T_LOG inside each tile (LDS) -> fused global levels, S per HBM pass,
@@ -24,7 +29,7 @@
 // from the caller, so the resident kernel can run it over its own blocks.
 #pragma once
 
-#include "vo_internal.hpp"
+#include "sort_core.hpp"
 
 namespace vo {
 namespace compact_k {
@@ -88,32 +93,19 @@ __device__ __forceinline__ void st_col(const Col &c, uint64_t i, uint64_t v)
     }
 }
 
-// swap flag of the pair at offset i in the block starting at prefix count
-// cb, with cbh = prefix count at the block's middle; s2 = half size
-__device__ __forceinline__ bool level_flag(uint64_t cb, uint64_t cbh, uint64_t half, uint64_t i)
+// Lanes whose pair swaps at level q > 0: d = low word of the prefix count at
+// the block's middle plus half - 1 - i (see the top; only the low q + 1 bits
+// matter, and q <= 31).
+__device__ __forceinline__ uint64_t swap_lanes(uint32_t d, int q)
 {
-    const uint64_t s = half * 2;
-    const uint64_t o = cb & (s - 1);
-    const uint64_t m1 = cbh - cb;
-    const uint64_t om = o & (half - 1);
-    const uint64_t om1 = (o + m1) & (half - 1);
-    const bool base = ((om + m1) >= half) ^ (o >= half);
-    return base ^ (i >= om1);
+    return __builtin_amdgcn_ballot_w64((d & (1u << q)) == 0);
 }
 
-// The same flag in 32-bit arithmetic, for n_pad <= 2^32 (q <= 31): only the
-// low 32 bits of the prefix counts matter (o is their low q+1 bits, and the
-// count difference m1 <= half is exact modulo 2^32).
-__device__ __forceinline__ bool level_flag32(uint32_t cb, uint32_t cbh, int q, uint32_t i)
+template <int NW>
+__device__ __forceinline__ void swap_rows(uint64_t m, uint64_t (&x)[NW], uint64_t (&y)[NW])
 {
-    const uint32_t half = 1u << q;
-    const uint32_t smask = half | (half - 1);
-    const uint32_t o = cb & smask;
-    const uint32_t m1 = cbh - cb;
-    const uint32_t om = o & (half - 1);
-    const uint32_t om1 = (o + m1) & (half - 1);
-    const bool base = ((om + m1) >= half) ^ (o >= half);
-    return base ^ (i >= om1);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) dev::swap_m(m, x[w], y[w]);
 }
 
 // Instances of one size class 2^c of a batch: virtual row v of the class is
@@ -422,107 +414,143 @@ __global__ __launch_bounds__(CBLOCK) void k_scan_seg(const uint32_t *__restrict_
 
 // ---------------------------------------------------------- local levels
 
-// Levels q = 0 .. CT_LOG-1 inside each 4096-row tile.  Thread tau holds 16
-// rows of each column in registers under layout a: row base(tau, a) | m << a
-// for m < 16, base(tau, a) = the 8 bits of tau around the 4-bit hole at a.
-// Levels a .. a+3 pair rows inside a thread; layouts a = 0, 4, 8 cover the 12
-// levels, with two LDS transposes between them (and one after the coalesced
-// load, layout 8).  Rows are read from `src` and written to `dst` (which may
-// be the same columns).  cpre (LDS) holds the tile's exclusive prefix counts.
-constexpr uint32_t CTPAD = CT + CT / 16; // transpose buffer: row l at l + l/16
+// Levels q = 0 .. T-1 inside each 2^T-row tile (T = 12, or 13 where that
+// saves a later pass).  A thread holds 16 rows of each column in registers
+// under layout a: rows lay_base(tau, a) | m << a (sort_core.hpp); levels
+// a .. a+3 pair rows inside a thread.  Layout 0 (levels 0-3) is 16 consecutive
+// rows, the ones whose mask bytes the thread reads for the scan, so its prefix
+// counts come from registers; levels from 4 up need counts at multiples of 16
+// only, one word of LDS per thread.  Of the relayouts 6 -> 0 -> 4 (-> 5) -> T-4
+// only the last leaves the wavefront; rows are loaded in layout 6 and stored in
+// layout T-4, both 64 lanes on consecutive rows.  Rows are read from `src` and
+// written to `dst` (which may be the same columns).  (With two counts in LDS
+// per pair and the offset form's arithmetic the pass was issue-bound: two
+// 8-byte columns of 2^23 rows 61.9 -> 51.2 us, 12 bytes of 2^24 144 -> 122 us.)
+template <int T>
+using CTileOf = dev::TileCT<dev::Rec<1, uint64_t, true>, T, 4, false>;
 
-__device__ __forceinline__ uint32_t cpos(uint32_t l) { return l + (l >> 4); }
-
-__device__ __forceinline__ uint32_t clay(uint32_t tau, int a) { return (tau & ((1u << a) - 1)) | ((tau >> a) << (a + 4)); }
-
-template <int NW>
-__device__ __forceinline__ void ctranspose(uint64_t (&r)[16][NW], uint64_t *buf, uint32_t tau, int a_from, int a_to)
+template <int NW, int T, int A_FROM, int A_TO>
+__device__ __forceinline__ void crelayout(uint64_t (&r)[16][NW], dev::TileBuf &buf, uint32_t tau)
 {
-    const uint32_t bf = clay(tau, a_from), bt = clay(tau, a_to);
+    using TL = CTileOf<T>;
+    constexpr bool IN = TL::in_wave(A_FROM, A_TO);
+    uint64_t h = 0;
+    uint32_t n = 0;
+    if (buf.shared || A_FROM > 6)
+        __syncthreads();
+    else
+        TL::wave_fence();
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
+        uint64_t v[16];
 #pragma unroll
-        for (int m = 0; m < 16; ++m) buf[cpos(bf | ((uint32_t)m << a_from))] = r[m][w];
-        __syncthreads();
+        for (int m = 0; m < 16; ++m) v[m] = r[m][w];
+        TL::template move_col<A_FROM, A_TO>(v, reinterpret_cast<uint64_t *>(buf.p), tau, h, n);
+        if (w + 1 < NW) {
+            if constexpr (IN)
+                TL::wave_fence();
+            else
+                __syncthreads();
+        }
 #pragma unroll
-        for (int m = 0; m < 16; ++m) r[m][w] = buf[cpos(bt | ((uint32_t)m << a_to))];
-        __syncthreads();
+        for (int m = 0; m < 16; ++m) r[m][w] = v[m];
+    }
+    buf.shared = !IN;
+}
+
+// Levels 0-3 in layout 0: selm = the select bits of the thread's rows, c0 =
+// low word of the prefix count at its first row.
+template <int NW>
+__device__ __forceinline__ void clevels0(uint64_t (&r)[16][NW], uint32_t selm, uint32_t c0)
+{
+    auto cnt = [&](int e) { return c0 + __popc(selm & ((1u << e) - 1)); };
+#pragma unroll
+    for (int m = 0; m < 16; m += 2) {
+        const uint32_t s0 = selm >> m, s1 = selm >> (m + 1);
+        const uint64_t sw = __builtin_amdgcn_ballot_w64((((~s0 & s1) ^ cnt(m)) & 1u) != 0);
+        swap_rows<NW>(sw, r[m], r[m | 1]);
+    }
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+        const int half = 1 << q;
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            if (m & half) continue;
+            const uint32_t d = cnt((m & ~(2 * half - 1)) + half) + (uint32_t)(half - 1 - (m & (half - 1)));
+            swap_rows<NW>(swap_lanes(d, q), r[m], r[m | half]);
+        }
     }
 }
 
-template <int NW, int A>
-__device__ __forceinline__ void clevels(uint64_t (&r)[16][NW], const uint16_t *cpre, uint32_t tbase, uint32_t tau)
+// Levels Q0 .. Q1 in layout A >= 4; c16 = the tile's prefix counts at rows
+// 16 j, tbase = the low word of the tile's first.
+template <int NW, int A, int Q0, int Q1>
+__device__ __forceinline__ void clevels(uint64_t (&r)[16][NW], const uint32_t *c16, uint32_t tbase, uint32_t tau)
 {
-    const uint32_t base = clay(tau, A);
+    const uint32_t base = dev::lay_base<4>(tau, A);
+    const uint32_t top = (base >> (A + 4)) << A; // 16-row index of the thread's rows, register bits clear
+    const uint32_t rest = tbase + ((1u << A) - 1) - (base & ((1u << A) - 1));
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int q = A + k;
-        const uint32_t half = 1u << q;
+    for (int q = Q0; q <= Q1; ++q) {
+        const int k = q - A;
 #pragma unroll
         for (int m = 0; m < 16; ++m) {
             if (m & (1 << k)) continue;
-            const int m2 = m | (1 << k);
-            const uint32_t e0 = base | ((uint32_t)m << A);
-            const uint32_t b = e0 & ~(2 * half - 1);
-            const uint32_t cb = tbase + cpre[b];
-            bool sw;
-            if (q == 0) {
-                const uint32_t e1 = e0 | 1;
-                const bool s0 = cpre[e0 + 1] != cpre[e0];
-                const bool s1 = cpre[e1 + 1] != cpre[e1];
-                sw = ((!s0) & s1) ^ (bool)(cb & 1);
-            } else {
-                sw = level_flag32(cb, tbase + cpre[b + half], q, e0 & (half - 1));
-            }
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const uint64_t x = r[m][w], y = r[m2][w];
-                r[m][w] = sw ? y : x;
-                r[m2][w] = sw ? x : y;
-            }
+            const uint32_t mid = (uint32_t)((m & ~((2 << k) - 1)) | (1 << k)) << (A - 4);
+            const uint32_t over = (uint32_t)(((1 << k) - 1) - (m & ((1 << k) - 1))) << A;
+            swap_rows<NW>(swap_lanes(c16[top + mid] + rest + over, q), r[m], r[m | (1 << k)]);
         }
     }
 }
 
 // W8: every column is 8 bytes wide (no per-load width dispatch)
-template <int NW, bool W8, bool TRACE, bool NT = false>
+template <int NW, bool W8, bool TRACE, bool NT = false, int T = CT_LOG>
 __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, const uint8_t *__restrict__ mask,
                                                 uint64_t n, const uint64_t *__restrict__ tile_pre, Inst in,
                                                 TraceSlot *slot, char *lds_raw, uint32_t vb)
 {
-    static_assert(CT == 16 * CBLOCK, "16 rows per thread");
-    uint64_t *buf = reinterpret_cast<uint64_t *>(lds_raw);          // one column, CTPAD words
-    uint16_t *cpre = reinterpret_cast<uint16_t *>(buf + CTPAD);      // CT + 1 counts <= 4096
-    __shared__ uint32_t wsum[CBLOCK / 64];
+    using TL = CTileOf<T>;
+    constexpr int NTHR = 1 << (T - 4), AS = T - 4;
+    dev::TileBuf buf{lds_raw};
+    uint32_t *c16 = reinterpret_cast<uint32_t *>(lds_raw + TL::lds_bytes());
+    __shared__ uint32_t wsum[NTHR / 64];
     const uint32_t tid = threadIdx.x;
-    const uint64_t tv = (uint64_t)vb * CT;
+    const uint64_t tv = (uint64_t)vb << T;
     const uint64_t t0 = inst_row(in, tv), l0 = inst_local(in, tv), nn = inst_live(in, tv, n);
-    const uint64_t tbase = tile_pre[vb];
-    constexpr int PER = CT / CBLOCK; // 16 consecutive rows per thread for the scan
+    const uint32_t tbase = (uint32_t)tile_pre[tv >> CT_LOG];
     dev::AtrT<TRACE> tr(slot);
-    tr.at(7, vb);
+    tr.at(7, tv >> CT_LOG);
 
-    // rows, coalesced (layout 8: row tid + 256 m); issued before the scan
+    // rows, coalesced; issued before the scan
+    const uint32_t lb = dev::lay_base<4>(tid, 6);
     uint64_t r[16][NW];
 #pragma unroll
     for (int m = 0; m < 16; ++m)
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            r[m][w] = W8 ? ld_row<NT>((const uint64_t *)src.c[w].p + t0 + tid + 256u * m)
-                         : ld_col<NT>(src.c[w], t0 + tid + 256u * m);
-            tr.at(8 + w, t0 + tid + 256u * m);
+            r[m][w] = W8 ? ld_row<NT>((const uint64_t *)src.c[w].p + t0 + lb + 64u * m)
+                         : ld_col<NT>(src.c[w], t0 + lb + 64u * m);
+            tr.at(8 + w, t0 + lb + 64u * m);
         }
 
-    // exclusive prefix of sel inside the tile: thread tid owns rows [16 tid, 16 tid + 16)
-    uint32_t sel[PER];
-    uint32_t run = 0;
+    // select bits and exclusive prefix: thread tid owns rows [16 tid, 16 tid + 16)
+    uint32_t selm = 0;
+    const uint8_t *mp = mask + t0 + tid * 16;
+    if (((uintptr_t)(mask + t0) & 15) == 0) { // tiles of a 16-byte aligned mask
+        const uint4 v = *reinterpret_cast<const uint4 *>(mp);
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const uint32_t i = tid * PER + k;
-        sel[k] = (mask[t0 + i] != 0) & (l0 + i < nn);
-        run += sel[k];
-        tr.at(1, t0 + i);
+        for (int k = 0; k < 16; ++k) selm |= (((x[k >> 2] >> (8 * (k & 3))) & 0xFFu) != 0 ? 1u : 0u) << k;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) selm |= (mp[k] != 0 ? 1u : 0u) << k;
     }
+    const uint64_t row0 = l0 + tid * 16;
+    const uint32_t live = row0 + 16 <= nn ? 16u : row0 < nn ? (uint32_t)(nn - row0) : 0u;
+    selm &= (1u << live) - 1;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) tr.at(1, t0 + tid * 16 + k);
+    const uint32_t run = __popc(selm);
     uint32_t incl = run;
     const uint32_t lane = tid & 63;
     for (int off = 1; off < 64; off <<= 1) {
@@ -533,42 +561,52 @@ __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, cons
     __syncthreads();
     uint32_t wpre = 0;
     for (uint32_t w = 0; w < (tid >> 6); ++w) wpre += wsum[w];
-    uint32_t c = wpre + incl - run;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        cpre[tid * PER + k] = (uint16_t)c;
-        c += sel[k];
+    const uint32_t c0 = wpre + incl - run;
+    // read inside the wavefront up to layout 6, beyond it after the relayout's barriers
+    c16[tid] = c0;
+    crelayout<NW, T, 6, 0>(r, buf, tid);
+    clevels0<NW>(r, selm, tbase + c0);
+    crelayout<NW, T, 0, 4>(r, buf, tid);
+    clevels<NW, 4, 4, 7>(r, c16, tbase, tid);
+    if constexpr (T == 13) {
+        crelayout<NW, T, 4, 5>(r, buf, tid);
+        clevels<NW, 5, 8, 8>(r, c16, tbase, tid);
+        crelayout<NW, T, 5, AS>(r, buf, tid);
+        clevels<NW, AS, 9, 12>(r, c16, tbase, tid);
+    } else {
+        static_assert(T == 12, "tiles of 2^12 or 2^13 rows");
+        crelayout<NW, T, 4, AS>(r, buf, tid);
+        clevels<NW, AS, 8, 11>(r, c16, tbase, tid);
     }
-    if (tid == CBLOCK - 1) cpre[CT] = (uint16_t)c;
-    // (the first transpose's barriers also publish cpre)
-    ctranspose<NW>(r, buf, tid, 8, 0);
-    clevels<NW, 0>(r, cpre, (uint32_t)tbase, tid);
-    ctranspose<NW>(r, buf, tid, 0, 4);
-    clevels<NW, 4>(r, cpre, (uint32_t)tbase, tid);
-    ctranspose<NW>(r, buf, tid, 4, 8);
-    clevels<NW, 8>(r, cpre, (uint32_t)tbase, tid);
     uint32_t tid_s = tid; // store addresses recomputed here (register pressure)
     asm volatile("" : "+v"(tid_s));
 #pragma unroll
     for (int m = 0; m < 16; ++m)
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
+            const uint64_t i = t0 + tid_s + ((uint32_t)m << AS);
             if (W8)
-                st_row<NT>((uint64_t *)dst.c[w].p + t0 + tid_s + 256u * m, r[m][w]);
+                st_row<NT>((uint64_t *)dst.c[w].p + i, r[m][w]);
             else
-                st_col<NT>(dst.c[w], t0 + tid_s + 256u * m, r[m][w]);
-            tr.at(16 + w, t0 + tid_s + 256u * m);
+                st_col<NT>(dst.c[w], i, r[m][w]);
+            tr.at(16 + w, i);
         }
-    tr.done(dev::gtid());
+    tr.done((uint64_t)vb * NTHR + tid);
 }
 
-template <int NW, bool W8, bool TRACE, bool NT = false>
-__global__ __launch_bounds__(CBLOCK) void k_compact_local(Cols<NW> src, Cols<NW> dst, const uint8_t *__restrict__ mask,
-                                                          uint64_t n, const uint64_t *__restrict__ tile_pre, Inst in,
-                                                          TraceSlot *slot)
+// dynamic LDS of the local pass: the relayout buffer and a count per thread
+template <int T>
+constexpr size_t clocal_lds() { return CTileOf<T>::lds_bytes() + ((size_t)4 << (T - 4)); }
+
+// XC: contiguous block ranges per XCD (dev::xcd_block)
+template <int NW, bool W8, bool TRACE, bool NT = false, int T = CT_LOG, bool XC = true>
+__global__ __launch_bounds__(1 << (T - 4)) void k_compact_local(Cols<NW> src, Cols<NW> dst,
+                                                                const uint8_t *__restrict__ mask, uint64_t n,
+                                                                const uint64_t *__restrict__ tile_pre, Inst in,
+                                                                TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds_raw[];
-    b_compact_local<NW, W8, TRACE, NT>(src, dst, mask, n, tile_pre, in, slot, lds_raw, blockIdx.x);
+    b_compact_local<NW, W8, TRACE, NT, T>(src, dst, mask, n, tile_pre, in, slot, lds_raw, dev::xcd_block<XC>());
 }
 
 // ---------------------------------------------------------- global levels
@@ -597,28 +635,18 @@ __device__ __forceinline__ void b_compact_global(Cols<NW> cols, const uint64_t *
     // uniform part of base (bits >= 8 are shared by the wavefront)
     const uint64_t ubase = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
                            __builtin_amdgcn_readfirstlane((uint32_t)base & ~0xFFu);
+    const uint32_t rest = (uint32_t)((1ull << q_lo) - 1) - ((uint32_t)base & (uint32_t)((1ull << q_lo) - 1));
 #pragma unroll
     for (int k = 0; k < S; ++k) {
-        const int q = q_lo + k;
-        const uint64_t half = 1ull << q;
 #pragma unroll
         for (int m = 0; m < (1 << S); ++m) {
             if (m & (1 << k)) continue;
-            const uint64_t e = base + ((uint64_t)m << q_lo);
             const uint64_t ue = ubase + ((uint64_t)m << q_lo);
-            const uint64_t b = ue & ~(2 * half - 1);
-            const uint64_t cb = tile_pre[b >> CT_LOG];
-            const uint64_t cbh = tile_pre[(b + half) >> CT_LOG];
-            tr.at(7, b >> CT_LOG);
-            tr.at(7, (b + half) >> CT_LOG);
-            const bool sw = level_flag(cb, cbh, half, e & (half - 1));
-            const int m2 = m | (1 << k);
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const uint64_t x = r[m][w], y = r[m2][w];
-                r[m][w] = sw ? y : x;
-                r[m2][w] = sw ? x : y;
-            }
+            const uint64_t mid = (ue & ~((2ull << (q_lo + k)) - 1)) + (1ull << (q_lo + k));
+            const uint32_t d = (uint32_t)tile_pre[mid >> CT_LOG] + rest +
+                               ((uint32_t)(((1 << k) - 1) - (m & ((1 << k) - 1))) << q_lo);
+            tr.at(7, mid >> CT_LOG);
+            swap_rows<NW>(swap_lanes(d, q_lo + k), r[m], r[m | (1 << k)]);
         }
     }
 #pragma unroll
@@ -635,106 +663,116 @@ template <int NW, int S, bool TRACE, bool NT = false>
 __global__ __launch_bounds__(256) void k_compact_global(Cols<NW> cols, const uint64_t *__restrict__ tile_pre, int q_lo,
                                                         Inst in, TraceSlot *slot)
 {
-    b_compact_global<NW, S, TRACE, NT>(cols, tile_pre, q_lo, in, slot, blockIdx.x);
+    b_compact_global<NW, S, TRACE, NT>(cols, tile_pre, q_lo, in, slot, dev::xcd_block<!NT>());
 }
 
 // ------------------------------------------------- LDS-staged global levels
 
-// S = 5..8 levels q_lo .. q_lo+S-1 (q_lo >= CT_LOG) in one pass.  A block
-// takes the 4096 rows hibase + m * 2^q_lo + j0 + c (m < 2^S, c < 2^(12-S)):
-// local row l = m << (12-S) | c, so level q_lo+k pairs local bit 12-S+k.
-// Registers + LDS transposes as in the local pass (layout 4 for local bits
-// 12-S .. 7, layout 8 for bits 8 .. 11); the prefix counts at every block
-// boundary the levels need, tile_pre at hibase + m * 2^q_lo, go to LDS.
-template <int NW, int A, int S>
+// S = 5 .. T-4 levels q_lo .. q_lo+S-1 (q_lo >= T) in one pass.  A block takes
+// the 2^T rows hibase + g * 2^q_lo + j0 + c (g < 2^S, c < 2^C, C = T - S):
+// local row l = g << C | c, so level q_lo+k pairs local bit C+k.  Loaded in
+// layout C, where the first levels run, stored in layout T-4, where the last
+// four do; the prefix counts the levels need, tile_pre at hibase + g * 2^q_lo,
+// go to LDS.
+template <int NW, int T, int A, int S, int B0, int B1>
 __device__ __forceinline__ void hlevels(uint64_t (&r)[16][NW], const uint32_t *P, uint32_t tau, int q_lo, uint32_t j0)
 {
-    constexpr int CB = CT_LOG - S;
-    const uint32_t base = clay(tau, A);
+    constexpr int C = T - S;
+    const uint32_t base = dev::lay_base<4>(tau, A);
+    const uint32_t g0 = base >> C; // the thread's g, register bits clear
+    const uint32_t rest = ((1u << q_lo) - 1) - j0 - (base & ((1u << C) - 1));
 #pragma unroll
-    for (int bit = A; bit < A + 4; ++bit) {
-        if (bit < CB) continue;
-        const int k = bit - CB; // level q_lo + k
+    for (int bit = B0; bit <= B1; ++bit) {
+        const int k = bit - C; // level q_lo + k
+        const uint32_t low = (1u << k) - 1;
+        const uint32_t restk = rest + ((low & ~g0) << q_lo);
 #pragma unroll
         for (int m = 0; m < 16; ++m) {
             if (m & (1 << (bit - A))) continue;
-            const int m2 = m | (1 << (bit - A));
-            const uint32_t l0 = base | ((uint32_t)m << A);
-            const uint32_t ml = l0 >> CB;
-            const uint32_t mb = ml & ~((2u << k) - 1);
-            const uint32_t i = ((ml & ((1u << k) - 1)) << q_lo) + j0 + (l0 & ((1u << CB) - 1));
-            const bool sw = level_flag32(P[mb], P[mb + (1u << k)], q_lo + k, i);
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const uint64_t x = r[m][w], y = r[m2][w];
-                r[m][w] = sw ? y : x;
-                r[m2][w] = sw ? x : y;
-            }
+            const uint32_t gm = (uint32_t)m << (A - C);
+            const uint32_t mid = ((g0 & ~(low * 2 + 1)) | (gm & ~(low * 2 + 1))) + (1u << k);
+            const uint32_t d = P[mid] + restk - ((gm & low) << q_lo);
+            swap_rows<NW>(swap_lanes(d, q_lo + k), r[m], r[m | (1 << (bit - A))]);
         }
     }
 }
 
-template <int NW, int S, bool W8, bool TRACE, bool NT = false>
+template <int NW, int S, bool W8, bool TRACE, bool NT = false, int T = CT_LOG>
 __device__ __forceinline__ void b_compact_hybrid(Cols<NW> cols, const uint64_t *__restrict__ tile_pre, int q_lo,
                                                  Inst in, TraceSlot *slot, char *lds_raw, uint32_t vb)
 {
+    using TL = CTileOf<T>;
     dev::AtrT<TRACE> tr(slot);
-    static_assert(S >= 5 && S <= 8, "hybrid widths 5..8");
-    constexpr int CB = CT_LOG - S;
-    uint64_t *buf = reinterpret_cast<uint64_t *>(lds_raw);     // CTPAD words
-    uint32_t *P = reinterpret_cast<uint32_t *>(buf + CTPAD); // low words of 2^S + 1 prefix counts
+    constexpr int C = T - S, NTHR = 1 << (T - 4), AS = T - 4;
+    static_assert(S >= 5 && C >= 4, "hybrid widths 5..T-4");
+    dev::TileBuf buf{lds_raw};
+    uint32_t *P = reinterpret_cast<uint32_t *>(lds_raw + TL::lds_bytes()); // low words of 2^S prefix counts
     const uint32_t tid = threadIdx.x;
     // row indices fit 32 bits (n_pad <= 2^32)
-    const uint32_t runs = (1u << q_lo) >> CB; // blocks per group of 2^(q_lo+S) rows
+    const uint32_t runs = (1u << q_lo) >> C; // blocks per group of 2^(q_lo+S) rows
     const uint32_t hibase = (vb / runs) << (q_lo + S);
-    const uint32_t j0 = (vb % runs) << CB;
+    const uint32_t j0 = (vb % runs) << C;
     // the group's 2^(q_lo+S) rows lie in one instance: physical row of its first
     const uint64_t ph = inst_row(in, hibase);
-    for (uint32_t k = tid; k <= (1u << S); k += CBLOCK) {
+    auto grow = [&](uint32_t l) { return ((l >> C) << q_lo) + (l & ((1u << C) - 1)); }; // additive over bit fields
+    uint64_t r[16][NW];
+    {
+        const uint32_t gl = j0 + grow(dev::lay_base<4>(tid, C));
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const uint64_t i = ph + gl + grow((uint32_t)m << C);
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                r[m][w] = W8 ? ld_row<NT>((const uint64_t *)cols.c[w].p + i) : ld_col<NT>(cols.c[w], i);
+                tr.at(8 + w, i);
+            }
+        }
+    }
+    __syncthreads(); // (resident blocks: the last step's reads of P)
+    for (uint32_t k = tid; k < (1u << S); k += NTHR) {
         P[k] = (uint32_t)tile_pre[((uint64_t)hibase + ((uint64_t)k << q_lo)) >> CT_LOG];
         tr.at(7, ((uint64_t)hibase + ((uint64_t)k << q_lo)) >> CT_LOG);
     }
-    uint64_t r[16][NW];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {
-        const uint32_t l = tid | ((uint32_t)m << 8);
-        const uint32_t g = ((l >> CB) << q_lo) + j0 + (l & ((1u << CB) - 1)); // row in the group
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            r[m][w] = W8 ? ld_row<NT>((const uint64_t *)cols.c[w].p + ph + g) : ld_col<NT>(cols.c[w], ph + g);
-            tr.at(8 + w, ph + g);
-        }
+    __syncthreads();
+    if constexpr (S == 9) { // five bits below the last four: layouts C and C + 1
+        hlevels<NW, T, C, S, C, C + 3>(r, P, tid, q_lo, j0);
+        crelayout<NW, T, C, C + 1>(r, buf, tid);
+        hlevels<NW, T, C + 1, S, C + 4, C + 4>(r, P, tid, q_lo, j0);
+        crelayout<NW, T, C + 1, AS>(r, buf, tid);
+    } else {
+        hlevels<NW, T, C, S, C, T - 5>(r, P, tid, q_lo, j0);
+        crelayout<NW, T, C, AS>(r, buf, tid);
     }
-    ctranspose<NW>(r, buf, tid, 8, 4); // its barriers also publish P
-    hlevels<NW, 4, S>(r, P, tid, q_lo, j0);
-    ctranspose<NW>(r, buf, tid, 4, 8);
-    hlevels<NW, 8, S>(r, P, tid, q_lo, j0);
+    hlevels<NW, T, AS, S, T - 4, T - 1>(r, P, tid, q_lo, j0);
     // recompute the store addresses here rather than keep the load addresses
     // live across the levels (register pressure)
     uint32_t tid_s = tid;
     asm volatile("" : "+v"(tid_s));
+    const uint32_t gs = j0 + grow(dev::lay_base<4>(tid_s, AS));
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
-        const uint32_t l = tid_s | ((uint32_t)m << 8);
-        const uint32_t g = ((l >> CB) << q_lo) + j0 + (l & ((1u << CB) - 1));
+        const uint64_t i = ph + gs + grow((uint32_t)m << AS);
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
             if (W8)
-                st_row<NT>((uint64_t *)cols.c[w].p + ph + g, r[m][w]);
+                st_row<NT>((uint64_t *)cols.c[w].p + i, r[m][w]);
             else
-                st_col<NT>(cols.c[w], ph + g, r[m][w]);
-            tr.at(16 + w, ph + g);
+                st_col<NT>(cols.c[w], i, r[m][w]);
+            tr.at(16 + w, i);
         }
     }
-    tr.done(dev::gtid());
+    tr.done((uint64_t)vb * NTHR + tid);
 }
 
-template <int NW, int S, bool W8, bool TRACE, bool NT = false>
-__global__ __launch_bounds__(CBLOCK) void k_compact_hybrid(Cols<NW> cols, const uint64_t *__restrict__ tile_pre,
-                                                           int q_lo, Inst in, TraceSlot *slot)
+template <int S, int T>
+constexpr size_t chybrid_lds() { return CTileOf<T>::lds_bytes() + ((size_t)4 << S); }
+
+template <int NW, int S, bool W8, bool TRACE, bool NT = false, int T = CT_LOG, bool XC = true>
+__global__ __launch_bounds__(1 << (T - 4)) void k_compact_hybrid(Cols<NW> cols, const uint64_t *__restrict__ tile_pre,
+                                                                 int q_lo, Inst in, TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds_raw[];
-    b_compact_hybrid<NW, S, W8, TRACE, NT>(cols, tile_pre, q_lo, in, slot, lds_raw, blockIdx.x);
+    b_compact_hybrid<NW, S, W8, TRACE, NT, T>(cols, tile_pre, q_lo, in, slot, lds_raw, dev::xcd_block<XC>());
 }
 
 // ------------------------------------------------------- int128 SUM pass

@@ -246,6 +246,25 @@ __device__ __forceinline__ void pad_select(R &r, uint64_t g, uint64_t n_valid)
     r.p = pad ? (typename R::P)g : r.p;
 }
 
+// Blocks go to the 8 XCDs in turn; this order gives every XCD one contiguous
+// range of the launch's blocks (the first grid mod 8 ranges are one longer),
+// so a pass finds in its XCD's L2 what the pass before left there.  While an
+// instance fits the MALL every pass gains (12-byte sort, one-stage pass: 8.8
+// -> 5.8 us at 2^20 records, 29.5 -> 28.9 at 2^23; batched sorts 59.2 -> 57.8
+// ms).  Above it strided passes lose (1009 -> 1060 us at 2^28: every run they
+// read is another DRAM page) and keep the plain order; contiguous tiles gain
+// from 3 times the MALL up (merge pass 1219 -> 1123 us at 2^28; whole sorts at
+// 2^26, 2^27 and 2^28: 10.18 -> 10.03, 22.4 -> 21.9 and 48.8 -> 47.3 ms) but
+// lose between (16-byte sort at 2^25: 6.72 -> 6.88 ms; two key words at 2^24:
+// 4.37 -> 4.45 ms), where part of a pass is still found in the MALL.
+template <bool XC = true>
+__device__ __forceinline__ uint32_t xcd_block()
+{
+    if constexpr (!XC) return blockIdx.x;
+    const uint32_t q = gridDim.x >> 3, rem = gridDim.x & 7, x = blockIdx.x & 7;
+    return x * q + (x < rem ? x : rem) + (blockIdx.x >> 3);
+}
+
 // ------------------------------------------------------------ tile layout
 
 // LDS position of tile element l: one pad slot per 16 elements keeps the
