@@ -349,3 +349,35 @@ def test_sort_pass_schedule_by_size(log2n, tuning):
             assert np.array_equal(from_dev(didx, np.int64), eidx)
             for dc, ec, t in zip(dcols, ecols, types):
                 assert np.array_equal(from_dev(dc, TYPES[t]).view(np.uint8), ec.view(np.uint8))
+
+
+@pytest.mark.parametrize("log2n", [8, 9, 10, 11, 12])
+@pytest.mark.parametrize("short", [0, 1, 77])
+def test_sort_small_tiles(vctx, log2n, short):
+    """One tile smaller than the full one, at its own compile-time size: the
+    12-byte records, the 16-byte ones (shuffle with its permutation) and
+    OP_SORT with 1, 2, 4 and 8 key words and ties, against the oracle."""
+    npad, n = 1 << log2n, (1 << log2n) - short
+    print(f"small tile n={n} npad={npad}", flush=True)
+    rng = np.random.default_rng(npad + short)
+    k = rng.integers(0, 50, n).astype(np.uint64) << np.uint64(40)
+    p = rng.permutation(n).astype(np.uint32)
+    gk, gp = _run_sort(vctx, k, p, n, npad)
+    ek, ep = oracle.bitonic_sort_kp(k, p, n, npad)
+    assert np.array_equal(gk, ek) and np.array_equal(gp, ep)
+    dp, dperm, dq = to_dev(np.arange(npad, dtype=np.uint32)), empty_dev(npad, np.uint32), to_dev(
+        np.arange(npad, dtype=np.uint32))
+    vctx.shuffle(dp, npad, 11, perm_out=dperm, n=n)
+    vctx.shuffle(dq, npad, 11, n=n)
+    assert np.array_equal(from_dev(dp, np.uint32), from_dev(dperm, np.uint32))
+    assert np.array_equal(from_dev(dp, np.uint32), from_dev(dq, np.uint32))
+    for types in ([4], [5, 4], [5, 5, 5], [5] * 8):
+        asc = [i % 2 == 0 for i in range(len(types))]
+        cols = [_rand_col(rng, t, npad, 2) for t in types]
+        ecols, eidx = oracle.bitonic_sort_multi(cols, types, asc, n, npad)
+        dcols = [to_dev(c) for c in cols]
+        didx = empty_dev(npad, np.int64)
+        vctx.sort(dcols, types, asc, didx, n, npad)
+        assert np.array_equal(from_dev(didx, np.int64), eidx)
+        for dc, ec, t in zip(dcols, ecols, types):
+            assert np.array_equal(from_dev(dc, TYPES[t]).view(np.uint8), ec.view(np.uint8))

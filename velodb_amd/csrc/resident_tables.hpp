@@ -67,7 +67,7 @@
     VO_SORT_H(X, kv, sortimpl::RecKV, 12, 4, 6) VO_SORT_H(X, kv, sortimpl::RecKV, 12, 4, 7)
 
 // multi-column records: as launch mode
-#define VO_SORT_M_BODIES(X)                                                                                        \
+#define VO_SORT_M12_BODIES(X)                                                                                      \
     VO_SORT_TILE(X, m1, sortimpl::RecM1, 12, 4)                                                                    \
     VO_SORT_G(X, m1, sortimpl::RecM1, 1) VO_SORT_G(X, m1, sortimpl::RecM1, 2) VO_SORT_G(X, m1, sortimpl::RecM1, 3) \
     VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 4) VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 5)                        \
@@ -75,13 +75,15 @@
     VO_SORT_TILE(X, m2, sortimpl::RecM2, 12, 4)                                                                    \
     VO_SORT_G(X, m2, sortimpl::RecM2, 1) VO_SORT_G(X, m2, sortimpl::RecM2, 2) VO_SORT_G(X, m2, sortimpl::RecM2, 3) \
     VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 4) VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 5)                        \
-    VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 6) VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 7)                        \
+    VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 6) VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 7)
+#define VO_SORT_M48_BODIES(X)                                                                                      \
     VO_SORT_TILE(X, m4, sortimpl::RecM4, 11, 3)                                                                    \
     VO_SORT_G(X, m4, sortimpl::RecM4, 1) VO_SORT_G(X, m4, sortimpl::RecM4, 2) VO_SORT_G(X, m4, sortimpl::RecM4, 3) \
     VO_SORT_H(X, m4, sortimpl::RecM4, 11, 3, 4) VO_SORT_H(X, m4, sortimpl::RecM4, 11, 3, 5)                        \
     VO_SORT_H(X, m4, sortimpl::RecM4, 11, 3, 6)                                                                    \
     VO_SORT_TILE(X, m8, sortimpl::RecM8, 10, 2)                                                                    \
     VO_SORT_G(X, m8, sortimpl::RecM8, 1) VO_SORT_G(X, m8, sortimpl::RecM8, 2)
+#define VO_SORT_M_BODIES(X) VO_SORT_M12_BODIES(X) VO_SORT_M48_BODIES(X)
 
 #define VO_SORT_PACK_BODIES(X)                                                                                     \
     X(kB_sort_pack, (smulti_k::k_pack_keys), (smulti_k::b_pack_keys(a..., vb, nvb)), 0)                           \
@@ -114,9 +116,6 @@
     X(kB_filter_count, (compact_k::k_filter_count<false>), (compact_k::b_filter_count<false>(a..., vb)), 0)       \
     X(kB_scan_tiles, (compact_k::k_scan_tiles), (compact_k::b_scan_tiles<256>(a..., (uint64_t *)lds)), 2048)      \
     X(kB_scan_seg, (compact_k::k_scan_seg), (compact_k::b_scan_seg(a..., (uint64_t *)lds, vb)), 2048)             \
-    X(kB_sum_prod, (compact_k::k_sum_prod_i128<false>),                                                            \
-      (compact_k::b_sum_prod_i128<false>(a..., (__int128 *)lds, vb, nvb)),                                         \
-      4096)                                                                                                        \
     X(kB_sum_final, (compact_k::k_sum_final), (compact_k::b_sum_final(a..., (__int128 *)lds)), 4096)              \
     X(kB_scatter_positions, (compact_k::k_scatter_positions), (compact_k::b_scatter_positions(a..., vb)), 0)
 

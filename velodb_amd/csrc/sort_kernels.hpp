@@ -560,8 +560,10 @@ inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int s_max, int r_log
 // Hybrid passes of at most HW_MAX stages run with twice the threads per block
 // and half the records per thread (the same tiles, so the same records per
 // block): more waves per SIMD where that pass is faster.
+// WRAP = false builds the level-by-level schedule alone, BATCH = true the
+// passes over many small instances whose arrays together exceed the MALL.
 template <class R, int T_LOG, int R_LOG, int BLOCK, int S_MAX, int H_MAX = 0, int S_LARGE = S_MAX, int LARGE_LOG = 64,
-          int HW_MAX = 0>
+          int HW_MAX = 0, bool WRAP = true, bool BATCH = false>
 struct SortImpl {
     static_assert(T_LOG >= 8, "global passes need q_lo >= 8 (256-thread blocks)");
     static_assert(H_MAX == 0 || (T_LOG - H_MAX >= 5 && BLOCK << R_LOG == 1 << T_LOG), "hybrid tile shape");
@@ -580,7 +582,7 @@ struct SortImpl {
     static std::vector<Pass> plan(vo_ctx *ctx, int n_log)
     {
         const SortTuning &t = ctx->tuning, d;
-        const bool wrapped = !ctx->rec && t.max_fused_stages == d.max_fused_stages &&
+        const bool wrapped = WRAP && !ctx->rec && t.max_fused_stages == d.max_fused_stages &&
                              t.max_hybrid_stages == d.max_hybrid_stages && !t.pipe_merge && !t.wide_block &&
                              !t.flip_hybrid_block;
         if (!wrapped) return plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx));
@@ -628,11 +630,34 @@ struct SortImpl {
         }
     }
 
+    // Arrays of one tile smaller than 2^T_LOG (t = 8 .. T_LOG - 1), of at most
+    // two key words: the
+    // compile-time tile sort at their own size, on at most 16 records a thread
+    // and at least one whole wavefront.  (The run-time form below kept its LDS
+    // addresses in registers and a barrier around every relayout: one array of
+    // 4096 12-byte records, call and wait included: 61 -> 40 us.)
+    template <bool TRACE, int T = 8>
+    static bool launch_small(vo_ctx *ctx, Bufs<R> b, IMap map, int t, int p_top, uint64_t n_valid, int fill,
+                             uint64_t n_virtual)
+    {
+        if constexpr (WRAP && T < T_LOG && R::KW <= 2) {
+            if (t != T) return launch_small<TRACE, T + 1>(ctx, b, map, t, p_top, n_valid, fill, n_virtual);
+            constexpr int RL = T - 6 < R_LOG ? T - 6 : R_LOG;
+            const size_t lds = dev::TileCT<R, T, RL, TRACE>::lds_bytes();
+            LaunchInfo li{"sort_local", dim3((uint32_t)(n_virtual >> T)), dim3(1u << (T - RL)), (uint32_t)lds,
+                          hash_mix(hash_mix(T, p_top), fill)};
+            launch(ctx, li, dev::k_sort_local_ct<R, T, RL, 1 << (T - RL), TRACE, 0, true>, b, map, p_top, n_valid,
+                   fill, trace_slot(ctx));
+            return true;
+        }
+        return false;
+    }
+
     // Wrap passes of S = 1 .. T_LOG - 5 stages of the upper level.
     template <bool TRACE, int CP, bool XC, int S = 1>
     static void launch_wrap(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int s, int p_top, uint64_t n_virtual)
     {
-        if constexpr (S <= T_LOG - 5) {
+        if constexpr (WRAP && S <= T_LOG - 5) {
             if (s != S) return launch_wrap<TRACE, CP, XC, S + 1>(ctx, b, map, p, q_lo, s, p_top, n_virtual);
             static const char *const names[] = {"sort_wrap_s1", "sort_wrap_s2", "sort_wrap_s3", "sort_wrap_s4",
                                                 "sort_wrap_s5", "sort_wrap_s6", "sort_wrap_s7", "sort_wrap_s8"};
@@ -688,6 +713,7 @@ struct SortImpl {
             case 1: {
                 const int t = ps.p;
                 const bool ct = (t == T_LOG && p_top >= T_LOG);
+                if (!ct && !ctx->rec && launch_small<TRACE>(ctx, b, map, t, p_top, n_valid, fill, n_virtual)) break;
                 const size_t lds = ct ? dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes() : dev::lds_bytes<R>(t);
                 LaunchInfo li{"sort_local", dim3((uint32_t)(n_virtual >> t)), dim3(BLOCK), (uint32_t)lds,
                               hash_mix(hash_mix(t, p_top), fill)};
@@ -763,10 +789,10 @@ struct SortImpl {
             run_t<true, 0, true>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
         else if (!streaming(ctx, n_virtual))
             run_t<false, 0, true>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
-        else if (bytes(1ull << n_log) > kMallBytes)
-            run_t<false, dev::kCpStream, false>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
+        else if (BATCH && bytes(1ull << n_log) <= kMallBytes)
+            run_t<false, dev::kCpStream, BATCH>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
         else
-            run_t<false, dev::kCpStream, true>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
+            run_t<false, dev::kCpStream, false>(ctx, b, n_log, n_valid, fill, map, p_top, n_virtual);
     }
 
     static void run(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill)

@@ -1,5 +1,5 @@
 // sort_kp.hip -- the (u64 key, u32 payload) oblivious sort (the headline
-// path) and the (u64 key, u64 value) sort used by the join.
+// path), its batched form and the autotuner.
 #include "resident_tables.hpp"
 #include "sort_kernels.hpp"
 
@@ -9,7 +9,7 @@ using namespace sortimpl;
 
 namespace {
 
-const std::pair<const void *, BodyInfo> kBodies[] = {VO_SORT_KP_BODIES(VO_BODY_ENTRY) VO_SORT_KV_BODIES(VO_BODY_ENTRY)};
+const std::pair<const void *, BodyInfo> kBodies[] = {VO_SORT_KP_BODIES(VO_BODY_ENTRY)};
 const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodies[0]), true);
 
 // Register-only global passes take up to 5 stages below 2^27 records and up
@@ -18,18 +18,13 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // passes win (2^25: 5.06 vs 5.13 ms per sort, 2^23: 1.107 vs 1.128 ms).
 // Hybrid passes of 4-6 stages with 1024-thread blocks: at 2^28, 5494 -> 5611,
 // 5147 -> 5216 and 5319 -> 5483 GB/s (7 and 8 stages are faster at 512).
-using SortKP = SortImpl<RecKP, 13, 4, 512, 5, 8, 3, 27, 6>;
-// the 16-byte sort likewise: at 2^28 its 4-5 stage register passes ran at
-// 4.80-4.99 TB/s against 5.11-5.36 for its LDS-staged passes
-// (512-thread hybrid passes measured no faster for it: 78.04-78.05 vs 78.06-78.14 ms per
-// 2^28-row shuffle with permutation output)
-using SortKV = SortImpl<RecKV, 12, 4, 256, 5, 7, 3, 27>;
+using SortKP = SortImpl<RecKP, 13, 4, 512, 5, 8, 3, 27, 6, true, true>;
 // The resident queue kernel runs 256-thread blocks: the 12-byte sort runs
 // there on 2^12-record tiles (the same network, so the same output).
-using SortKP_R = SortImpl<RecKP, 12, 4, 256, 5, 7, 3, 27>;
+using SortKP_R = SortImpl<RecKP, 12, 4, 256, 5, 7, 3, 27, 0, false>;
 // The same tiles with 1024-thread blocks of 8 records per thread (tuning
 // bit 0x200): the same passes at up to twice the waves per SIMD.
-using SortKP_W = SortImpl<RecKP, 13, 3, 1024, 5, 8, 3, 27>;
+using SortKP_W = SortImpl<RecKP, 13, 3, 1024, 5, 8, 3, 27, 0, false>;
 
 void run_kp(vo_ctx *ctx, Bufs<RecKP> b, int n_log, uint64_t n_valid, int fill)
 {
@@ -59,14 +54,6 @@ void sort_kp_full(vo_ctx *ctx, uint64_t *keys, uint32_t *payload, uint64_t n_pad
     b.k[0] = keys;
     b.p = payload;
     run_kp(ctx, b, ilog2(n_pad), n_pad, 0);
-}
-
-void sort_kv(vo_ctx *ctx, uint64_t *keys, uint64_t *vals, uint64_t n_pad)
-{
-    Bufs<RecKV> b;
-    b.k[0] = keys;
-    b.p = vals;
-    SortKV::run(ctx, b, ilog2(n_pad), n_pad, 0);
 }
 
 int sort_plan_passes(vo_ctx *ctx, uint64_t n_pad) { return SortKP::passes(ctx, ilog2(n_pad)); }

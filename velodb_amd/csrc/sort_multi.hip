@@ -14,15 +14,13 @@ namespace {
 
 using namespace smulti_k;
 
-const std::pair<const void *, BodyInfo> kBodies[] = {VO_SORT_M_BODIES(VO_BODY_ENTRY) VO_SORT_PACK_BODIES(VO_BODY_ENTRY)};
+const std::pair<const void *, BodyInfo> kBodies[] = {VO_SORT_M12_BODIES(VO_BODY_ENTRY) VO_SORT_PACK_BODIES(VO_BODY_ENTRY)};
 const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodies[0]), true);
 
 // 1- and 2-word keys: register passes of at most 3 stages, wider groups as
 // LDS-staged hybrid passes (ORDER BY of two keys at 2^24: 5.66 -> 5.39 ms)
 using SortM1 = SortImpl<RecM1, 12, 4, 256, 3, 7>;
 using SortM2 = SortImpl<RecM2, 12, 4, 256, 3, 7>;
-using SortM4 = SortImpl<RecM4, 11, 3, 256, 3, 6>;
-using SortM8 = SortImpl<RecM8, 10, 2, 256, 2>;
 
 // ------------------------------------------------- multi-column (OP_SORT)
 
@@ -135,20 +133,8 @@ void op_sort_multi(vo_ctx *ctx, const vo_sort_args &a)
         SortM2::run(ctx, b, n_log, n_pad, 0);
         break;
     }
-    case 4: {
-        Bufs<RecM4> b;
-        for (int w = 0; w < 4; ++w) b.k[w] = wp[w];
-        b.p = idx;
-        SortM4::run(ctx, b, n_log, n_pad, 0);
-        break;
-    }
-    default: {
-        Bufs<RecM8> b;
-        for (int w = 0; w < 8; ++w) b.k[w] = wp[w];
-        b.p = idx;
-        SortM8::run(ctx, b, n_log, n_pad, 0);
-        break;
-    }
+    case 4: sort_words4(ctx, wp, idx, n_log); break;
+    default: sort_words8(ctx, wp, idx, n_log); break;
     }
     LaunchInfo lu{"sort_unpack", dim3(blocks), dim3(256), 0, hash_mix(ps.ncols, ps.nwords)};
     launch(ctx, lu, k_unpack_keys, ps, wp[0], wp[1], wp[2], wp[3], wp[4], wp[5], wp[6], wp[7],
