@@ -186,8 +186,7 @@ def bench_filter(args):
     torch.cuda.synchronize()
     dt = (time.perf_counter() - t0) / args.steps
     o = out.cpu().numpy().view(np.uint64)
-    stats = _family_stats(ctx, ["filter_count", "compact_scan", "compact_local", "compact_hybrid", "compact_global",
-                                "filter_sum"])
+    stats = _family_stats(ctx, ["filter_count", "compact_scan", "compact_local", "compact_hybrid", "compact_global"])
     # the same WHERE clause as five generic device terms (OP_PREDICATE_MASK):
     # reads day, disc, qty once each (20 B/row) and writes the mask (1 B/row)
     mask = torch.empty(n_pad, dtype=torch.uint8, device=dev)
@@ -208,7 +207,7 @@ def bench_filter(args):
     # and writes the mask; the local network reads the mask and both columns
     # and writes the columns; a global or LDS-staged pass reads and writes both
     bpr = {"filter_count": 4 + 8 + 8 + 1, "compact_local": 1 + 2 * 16, "compact_hybrid": 2 * 16,
-           "compact_global": 2 * 16, "filter_sum": 16}
+           "compact_global": 2 * 16}
     _line("oblivious filter + compaction + int128 SUM (Mrows/s)", n / dt / 1e6, "Mrows/s", args.steps,
           args.warmup, dt * 1e3, "int64/int128",
           {"workload": f"Q6-style filter over {n} rows padded to 2^{ilog2(n_pad)}, ORCompact of (price, disc), "

@@ -35,10 +35,10 @@ struct Workspace {
     __int128 *partial;
 };
 
-constexpr uint32_t kSumBlocks = 2048;
+constexpr uint32_t kScanTmp = 2048; // scan_tiles' temporaries
 
 // The workspace laid out from `base` (nullptr: only the size); returns its
-// bytes.
+// bytes.  want_mask: the filter's, with a mask and one partial sum per tile.
 size_t workspace_at(char *base, uint64_t n_pad, bool want_mask, Workspace *ws)
 {
     const uint64_t nt = n_pad / CT;
@@ -49,7 +49,8 @@ size_t workspace_at(char *base, uint64_t n_pad, bool want_mask, Workspace *ws)
         return o;
     };
     const size_t o_cnt = take(nt * 4), o_pre = take((nt + 1) * 8), o_count = take(8),
-                 o_part = take(kSumBlocks * sizeof(__int128)), o_mask = take(want_mask ? n_pad : 0);
+                 o_part = take(std::max<size_t>(kScanTmp, want_mask ? nt * sizeof(__int128) : 0)),
+                 o_mask = take(want_mask ? n_pad : 0);
     if (ws)
         *ws = Workspace{(uint32_t *)(base + o_cnt), (uint64_t *)(base + o_pre), (uint64_t *)(base + o_count),
                         want_mask ? (uint8_t *)(base + o_mask) : nullptr, (__int128 *)(base + o_part)};
@@ -92,6 +93,15 @@ void scan_tiles(vo_ctx *ctx, const uint32_t *cnt, uint32_t nt, uint64_t *pre, ui
 // most t - 4 levels (LDS-staged tiles keep runs of 16 rows), as even as possible.
 int level_groups(int n_log, int t) { return (n_log - t + t - 5) / (t - 4); }
 
+// Tiles of 2^13 rows where they save a pass over the rows (2^13, 2^21, 2^22
+// and from 2^29): filter + SUM at 2^29 15.9 -> 13.2 ms with two passes above
+// the tile instead of three.  Elsewhere twice the blocks, of 2^12 rows.
+// Resident bodies are built for 2^12.
+int tile_log(vo_ctx *ctx, int n_log)
+{
+    return !ctx->rec && n_log >= 13 && level_groups(n_log, 13) < level_groups(n_log, 12) ? 13 : 12;
+}
+
 // Launches one kernel over tiles of 2^t rows.
 template <class K, class... A>
 void launch_tiles(vo_ctx *ctx, const char *family, uint64_t rows, int t, size_t lds, uint64_t hash, K k, A... args)
@@ -103,22 +113,19 @@ void launch_tiles(vo_ctx *ctx, const char *family, uint64_t rows, int t, size_t 
 // The network's passes with one tracing mode (TR) and cache policy (NT).
 template <int NW, bool TR, bool NT>
 void run_network_t(vo_ctx *ctx, Cols<NW> src, Cols<NW> cols, const uint8_t *mask, uint64_t n,
-                   const uint64_t *tile_pre, Inst in, uint64_t rows, int n_log, bool w8, bool tiles_xc)
+                   const uint64_t *tile_pre, Inst in, uint64_t rows, int n_log, bool w8, bool tiles_xc,
+                   __int128 *partial)
 {
-    // 2^13-row tiles where they save a pass over the rows (2^13, 2^21, 2^22
-    // and from 2^29): filter + SUM at 2^29 15.9 -> 13.2 ms with two passes
-    // above the tile instead of three.  Elsewhere twice the blocks of 2^12
-    // rows.  Resident bodies are built for 2^12.
-    const int t = !ctx->rec && n_log >= 13 && level_groups(n_log, 13) < level_groups(n_log, 12) ? 13 : 12;
+    const int t = tile_log(ctx, n_log);
     TraceSlot *slot = trace_slot(ctx);
     {
         auto go = [&](auto k12, auto k13) {
             if (t == 12)
                 launch_tiles(ctx, "compact_local", rows, 12, clocal_lds<12>(), hash_mix(NW, n_log), k12, src, cols,
-                             mask, n, tile_pre, in, slot);
+                             mask, n, tile_pre, in, partial, slot);
             else
                 launch_tiles(ctx, "compact_local", rows, 13, clocal_lds<13>(), hash_mix(NW, n_log), k13, src, cols,
-                             mask, n, tile_pre, in, slot);
+                             mask, n, tile_pre, in, partial, slot);
         };
         auto pick = [&](auto w) {
             constexpr bool W8 = decltype(w)::value;
@@ -191,24 +198,25 @@ void run_network_t(vo_ctx *ctx, Cols<NW> src, Cols<NW> cols, const uint8_t *mask
 // the choice.
 template <int NW>
 void run_network(vo_ctx *ctx, Cols<NW> src, Cols<NW> cols, const uint8_t *mask, uint64_t n, uint64_t n_pad,
-                 const uint64_t *tile_pre, Inst in = Inst{nullptr, nullptr, 0}, uint64_t rows = 0)
+                 const uint64_t *tile_pre, Inst in = Inst{nullptr, nullptr, 0}, uint64_t rows = 0,
+                 __int128 *partial = nullptr)
 {
     const int n_log = in.off ? in.c : ilog2(n_pad);
     if (!in.off) rows = n_pad;
     bool w8 = true;
     uint64_t row_bytes = 0;
     for (int w = 0; w < NW; ++w) {
-        w8 = w8 && src.c[w].w == 8 && cols.c[w].w == 8;
-        row_bytes += cols.c[w].w;
+        w8 = w8 && src.c[w].w[0] == 8 && cols.c[w].w[0] == 8;
+        for (uint32_t b : cols.c[w].w) row_bytes += b;
     }
     constexpr uint64_t kMallBytes = 256ull << 20;
     const bool txc = rows * row_bytes >= 3 * kMallBytes; // block order of streaming tiles (dev::xcd_block)
     if (ctx->tracing)
-        run_network_t<NW, true, false>(ctx, src, cols, mask, n, tile_pre, in, rows, n_log, w8, txc);
+        run_network_t<NW, true, false>(ctx, src, cols, mask, n, tile_pre, in, rows, n_log, w8, txc, partial);
     else if (!ctx->rec && ((rows * row_bytes > kMallBytes) != (ctx->tuning.flip_streaming != 0)))
-        run_network_t<NW, false, true>(ctx, src, cols, mask, n, tile_pre, in, rows, n_log, w8, txc);
+        run_network_t<NW, false, true>(ctx, src, cols, mask, n, tile_pre, in, rows, n_log, w8, txc, partial);
     else
-        run_network_t<NW, false, false>(ctx, src, cols, mask, n, tile_pre, in, rows, n_log, w8, txc);
+        run_network_t<NW, false, false>(ctx, src, cols, mask, n, tile_pre, in, rows, n_log, w8, txc, partial);
 }
 
 // Count + scan for a mask already in device memory.
@@ -220,6 +228,47 @@ void count_and_scan(vo_ctx *ctx, const uint8_t *mask, uint64_t n, uint64_t n_pad
            Inst{nullptr, nullptr, 0}, trace_slot(ctx));
     // the sum partials' region is free until a sum pass: the scan's temporaries
     scan_tiles(ctx, ws.tile_cnt, nt, ws.tile_pre, out_count ? out_count : ws.count, ws.partial);
+}
+
+Word word8(void *p) { return Word{{p}, {8}}; }
+
+// Columns packed into the network's 64-bit words, widest first: an 8-byte
+// column is a word, narrower ones fill words together.  The routing depends on
+// the mask only, so how columns share words changes no output.  (8-, 4- and
+// 1-byte columns of 10M rows / 2^24: one run of two words instead of one of two
+// and one of one, WHERE and compaction together 616 -> 432 us.)
+std::vector<Word> pack_words(void *const *cols, const uint32_t *bytes, uint32_t n)
+{
+    std::vector<Word> v;
+    std::vector<uint32_t> used;
+    for (uint32_t width : {8u, 4u, 2u, 1u})
+        for (uint32_t c = 0; c < n; ++c) {
+            if (bytes[c] != width) continue;
+            size_t i = 0;
+            while (i < v.size() && (used[i] + width > 8 || v[i].w[kParts - 1] != 0)) ++i;
+            if (i == v.size()) {
+                v.push_back(Word{});
+                used.push_back(0);
+            }
+            int k = 0;
+            while (v[i].w[k] != 0) ++k;
+            v[i].p[k] = cols[c];
+            v[i].w[k] = width;
+            used[i] += width;
+        }
+    return v;
+}
+
+// One run of the network per two words.
+template <class F>
+void run_words(const std::vector<Word> &v, F &&run)
+{
+    for (size_t i = 0; i < v.size(); i += 2) {
+        if (i + 1 < v.size())
+            run(Cols<2>{{v[i], v[i + 1]}});
+        else
+            run(Cols<1>{{v[i]}});
+    }
 }
 
 void check_pad(uint64_t n, uint64_t n_pad)
@@ -245,7 +294,7 @@ void compact_rows2(vo_ctx *ctx, uint64_t *c0, uint64_t *c1, const uint8_t *mask,
            Inst{nullptr, nullptr, 0}, trace_slot(ctx));
     launch(ctx, LaunchInfo{"compact_scan", dim3(1), dim3(1024), 0, nt}, k_scan_tiles, (const uint32_t *)tile_cnt, nt,
            tile_pre, count_dev, trace_slot(ctx));
-    Cols<2> cs{{{c0, 8}, {c1, 8}}};
+    Cols<2> cs{{word8(c0), word8(c1)}};
     run_network<2>(ctx, cs, cs, mask, n_pad, n_pad, tile_pre);
 }
 
@@ -260,7 +309,7 @@ void compact_rows1(vo_ctx *ctx, uint64_t *c0, const uint8_t *mask, uint64_t n_pa
            Inst{nullptr, nullptr, 0}, trace_slot(ctx));
     launch(ctx, LaunchInfo{"compact_scan", dim3(1), dim3(1024), 0, nt}, k_scan_tiles, (const uint32_t *)tile_cnt, nt,
            tile_pre, count_dev, trace_slot(ctx));
-    Cols<1> cs{{{c0, 8}}};
+    Cols<1> cs{{word8(c0)}};
     run_network<1>(ctx, cs, cs, mask, n_pad, n_pad, tile_pre);
 }
 
@@ -282,20 +331,9 @@ void compact_with(vo_ctx *ctx, const vo_compact_args &a, const Workspace &ws)
         VO_CHECK(a.cols[c] && (w == 1 || w == 2 || w == 4 || w == 8), VO_ERR_INVALID, "bad column");
     }
     count_and_scan(ctx, a.mask, a.n, a.n_pad, ws, a.out_count);
-    // columns in pairs of two words per network run; the network depends on
-    // the mask only, so each run applies the same routing
-    uint32_t c = 0;
-    while (c < a.n_cols) {
-        const uint32_t take = std::min<uint32_t>(2, a.n_cols - c);
-        if (take == 2) {
-            Cols<2> cs{{{a.cols[c], a.col_bytes[c]}, {a.cols[c + 1], a.col_bytes[c + 1]}}};
-            run_network<2>(ctx, cs, cs, a.mask, a.n, a.n_pad, ws.tile_pre);
-        } else {
-            Cols<1> cs{{{a.cols[c], a.col_bytes[c]}}};
-            run_network<1>(ctx, cs, cs, a.mask, a.n, a.n_pad, ws.tile_pre);
-        }
-        c += take;
-    }
+    run_words(pack_words(a.cols, a.col_bytes, a.n_cols), [&](auto cs) {
+        run_network(ctx, cs, cs, a.mask, a.n, a.n_pad, ws.tile_pre);
+    });
 }
 
 } // namespace
@@ -361,6 +399,7 @@ void op_compact_batch(vo_ctx *ctx, const vo_compact_batch_args &a)
     char *base = (char *)scratch(ctx, bytes);
     uint64_t *dtab = (uint64_t *)base;
     upload_async(ctx, dtab, host.data(), host.size() * 8);
+    const std::vector<Word> words = pack_words(a.cols, a.col_bytes, a.n_cols);
     run_tracks(ctx, classes.size(), [&](size_t t) {
         const int c = classes[t];
         const uint64_t k = off[c].size();
@@ -375,18 +414,7 @@ void op_compact_batch(vo_ctx *ctx, const vo_compact_batch_args &a)
         launch(ctx, LaunchInfo{"compact_scan_seg", dim3((uint32_t)k), dim3(CBLOCK), 0, hash_mix(k, c)}, k_scan_seg,
                (const uint32_t *)tile_cnt, nts, tile_pre, a.out_counts, ix, trace_slot(ctx));
         const uint64_t rows = k << c;
-        uint32_t j = 0;
-        while (j < a.n_cols) {
-            const uint32_t take = std::min<uint32_t>(2, a.n_cols - j);
-            if (take == 2) {
-                Cols<2> cs{{{a.cols[j], a.col_bytes[j]}, {a.cols[j + 1], a.col_bytes[j + 1]}}};
-                run_network<2>(ctx, cs, cs, a.mask, 0, 0, tile_pre, in, rows);
-            } else {
-                Cols<1> cs{{{a.cols[j], a.col_bytes[j]}}};
-                run_network<1>(ctx, cs, cs, a.mask, 0, 0, tile_pre, in, rows);
-            }
-            j += take;
-        }
+        run_words(words, [&](auto cs) { run_network(ctx, cs, cs, a.mask, 0, 0, tile_pre, in, rows); });
     });
     // the host table must outlive its upload (recorded: it travels with the program)
     if (!ctx->rec) VO_HIP(hipStreamSynchronize(ctx->stream));
@@ -463,8 +491,8 @@ void filter_sum_with(vo_ctx *ctx, const vo_filter_args &a, const Workspace &ws)
     const bool in_place_copy = a.out_price != nullptr;
     const uint32_t nt = (uint32_t)(a.n_pad / CT);
     Pred pr{a.day_lo, a.day_hi, a.disc_lo, a.disc_hi, a.qty_lt};
-    // the count pass reads 20 B per row, the sum pass 16: streaming loads
-    // beyond the MALL, as in the network passes
+    // the count pass reads 20 B per row: streaming loads beyond the MALL, as in
+    // the network passes, whose local one also leaves a sum per tile
     const bool stream = !ctx->rec && !ctx->tracing &&
                         ((a.n_pad * 16 > (256ull << 20)) != (ctx->tuning.flip_streaming != 0));
     launch(ctx, LaunchInfo{"filter_count", dim3(nt), dim3(CBLOCK), 0, a.n_pad},
@@ -475,14 +503,10 @@ void filter_sum_with(vo_ctx *ctx, const vo_filter_args &a, const Workspace &ws)
     // output columns (or the inputs in place when no outputs are given)
     int64_t *op = in_place_copy ? a.out_price : const_cast<int64_t *>(a.price);
     int64_t *od = in_place_copy ? a.out_disc : const_cast<int64_t *>(a.disc);
-    Cols<2> in{{{const_cast<int64_t *>(a.price), 8}, {const_cast<int64_t *>(a.disc), 8}}};
-    Cols<2> cs{{{op, 8}, {od, 8}}};
-    run_network<2>(ctx, in, cs, ws.mask, a.n, a.n_pad, ws.tile_pre);
-    // at least 8 rows per thread, at most kSumBlocks partial sums
-    const uint32_t sb = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kSumBlocks, a.n_pad / 2048));
-    launch(ctx, LaunchInfo{"filter_sum", dim3(sb), dim3(256), 0, a.n_pad},
-           stream ? k_sum_prod_i128<true> : k_sum_prod_i128<false>, (const int64_t *)op,
-           (const int64_t *)od, a.n_pad, (const uint64_t *)ws.count, ws.partial, trace_slot(ctx));
+    Cols<2> in{{word8(const_cast<int64_t *>(a.price)), word8(const_cast<int64_t *>(a.disc))}};
+    Cols<2> cs{{word8(op), word8(od)}};
+    run_network<2>(ctx, in, cs, ws.mask, a.n, a.n_pad, ws.tile_pre, Inst{nullptr, nullptr, 0}, 0, ws.partial);
+    const uint32_t sb = (uint32_t)(a.n_pad >> tile_log(ctx, ilog2(a.n_pad)));
     launch(ctx, LaunchInfo{"filter_sum_final", dim3(1), dim3(256), 0, 0}, k_sum_final, (const __int128 *)ws.partial,
            sb, (const uint64_t *)ws.count, a.out, trace_slot(ctx));
 }

@@ -31,6 +31,8 @@
 
 #include "sort_core.hpp"
 
+#include <type_traits>
+
 namespace vo {
 namespace compact_k {
 namespace {
@@ -39,15 +41,19 @@ constexpr int CT_LOG = 12; // tile: 4096 rows
 constexpr int CT = 1 << CT_LOG;
 constexpr int CBLOCK = 256;
 
-// A column of the compaction: pointer and element width (1, 2, 4, 8 bytes).
-struct Col {
-    void *p;
-    uint32_t w;
+// A word the network moves: up to kParts columns (pointer and element width 1,
+// 2, 4 or 8 bytes; width 0 ends the list) side by side in 64 bits, so that
+// narrow columns share a run of the network instead of taking a register pair
+// and LDS traffic each.
+constexpr int kParts = 4;
+struct Word {
+    void *p[kParts];
+    uint32_t w[kParts];
 };
 
 template <int NW>
 struct Cols {
-    Col c[NW];
+    Word c[NW];
 };
 
 // Row loads and stores of the network passes.  NT: non-temporal, for rows
@@ -71,25 +77,68 @@ __device__ __forceinline__ void st_row(T *p, T v)
         *p = v;
 }
 
-template <bool NT = false>
-__device__ __forceinline__ uint64_t ld_col(const Col &c, uint64_t i)
+// Rows idx(m), m < RR, of every word.  W8: every word is one 8-byte column;
+// otherwise the widths are uniform over the launch, and each part's loads (or
+// stores) are issued together.
+template <bool W8, bool NT, int RR, int NW, class I>
+__device__ __forceinline__ void ld_rows(uint64_t (&r)[RR][NW], const Cols<NW> &c, I idx)
 {
-    switch (c.w) {
-    case 8: return ld_row<NT>((const uint64_t *)c.p + i);
-    case 4: return ld_row<NT>((const uint32_t *)c.p + i);
-    case 2: return ld_row<NT>((const uint16_t *)c.p + i);
-    default: return ld_row<NT>((const uint8_t *)c.p + i);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        uint32_t sh = 0;
+#pragma unroll
+        for (int k = 0; k < (W8 ? 1 : kParts); ++k) {
+            const uint32_t wd = W8 ? 8 : c.c[w].w[k];
+            if (wd == 0) break;
+            uint32_t z = 0; // a row index of its own per part (register pressure)
+            if (!W8) asm volatile("" : "+v"(z));
+            auto part = [&](auto *p) {
+#pragma unroll
+                for (int m = 0; m < RR; ++m) {
+                    const uint64_t v = ld_row<NT>(p + (idx(m) + z));
+                    r[m][w] = k == 0 ? v : r[m][w] | (v << sh);
+                }
+            };
+            if (wd == 8)
+                part((const uint64_t *)c.c[w].p[k]);
+            else if (wd == 4)
+                part((const uint32_t *)c.c[w].p[k]);
+            else if (wd == 2)
+                part((const uint16_t *)c.c[w].p[k]);
+            else
+                part((const uint8_t *)c.c[w].p[k]);
+            sh += 8 * wd;
+        }
     }
 }
 
-template <bool NT = false>
-__device__ __forceinline__ void st_col(const Col &c, uint64_t i, uint64_t v)
+template <bool W8, bool NT, int RR, int NW, class I>
+__device__ __forceinline__ void st_rows(const uint64_t (&r)[RR][NW], const Cols<NW> &c, I idx)
 {
-    switch (c.w) {
-    case 8: st_row<NT>((uint64_t *)c.p + i, v); break;
-    case 4: st_row<NT>((uint32_t *)c.p + i, (uint32_t)v); break;
-    case 2: st_row<NT>((uint16_t *)c.p + i, (uint16_t)v); break;
-    default: st_row<NT>((uint8_t *)c.p + i, (uint8_t)v); break;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        uint32_t sh = 0;
+#pragma unroll
+        for (int k = 0; k < (W8 ? 1 : kParts); ++k) {
+            const uint32_t wd = W8 ? 8 : c.c[w].w[k];
+            if (wd == 0) break;
+            uint32_t z = 0;
+            if (!W8) asm volatile("" : "+v"(z));
+            auto part = [&](auto *p) {
+                using E = std::remove_reference_t<decltype(*p)>;
+#pragma unroll
+                for (int m = 0; m < RR; ++m) st_row<NT>(p + (idx(m) + z), (E)(k == 0 ? r[m][w] : r[m][w] >> sh));
+            };
+            if (wd == 8)
+                part((uint64_t *)c.c[w].p[k]);
+            else if (wd == 4)
+                part((uint32_t *)c.c[w].p[k]);
+            else if (wd == 2)
+                part((uint16_t *)c.c[w].p[k]);
+            else
+                part((uint8_t *)c.c[w].p[k]);
+            sh += 8 * wd;
+        }
     }
 }
 
@@ -429,6 +478,10 @@ __global__ __launch_bounds__(CBLOCK) void k_scan_seg(const uint32_t *__restrict_
 template <int T>
 using CTileOf = dev::TileCT<dev::Rec<1, uint64_t, true>, T, 4, false>;
 
+// relayout buffer: one 8-byte column
+template <int T>
+constexpr size_t cbuf_bytes() { return (size_t)CTileOf<T>::TPAD * 8; }
+
 template <int NW, int T, int A_FROM, int A_TO>
 __device__ __forceinline__ void crelayout(uint64_t (&r)[16][NW], dev::TileBuf &buf, uint32_t tau)
 {
@@ -503,16 +556,53 @@ __device__ __forceinline__ void clevels(uint64_t (&r)[16][NW], const uint32_t *c
     }
 }
 
-// W8: every column is 8 bytes wide (no per-load width dispatch)
+// Exact sum of a[i] * b[i] over the thread's selected rows (layout 0), added
+// over the block into partial[vb].  Summing selected rows here, where the tile
+// has them in registers with their mask bits, is the sum over the compacted
+// prefix without the pass that re-read both columns (1.46 of 13.2 ms at 2^29).
+template <int NTHR>
+__device__ __forceinline__ void csum(const uint64_t (&r)[16][2], uint32_t selm, __int128 *__restrict__ partial,
+                                     uint32_t vb, uint32_t tid)
+{
+    __shared__ __int128 red[NTHR / 64];
+    unsigned __int128 acc = 0;
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        const __int128 prod = (__int128)(int64_t)r[m][0] * (__int128)(int64_t)r[m][1];
+        const uint64_t on = 0 - (uint64_t)((selm >> m) & 1u);
+        acc += ((unsigned __int128)((uint64_t)((unsigned __int128)prod >> 64) & on) << 64) | ((uint64_t)prod & on);
+        // one product at a time: all sixteen in flight pass the 128 VGPRs that
+        // let two 2^13-row blocks share a CU
+        uint64_t lo = (uint64_t)acc, hi = (uint64_t)(acc >> 64);
+        asm volatile("" : "+v"(lo), "+v"(hi));
+        acc = ((unsigned __int128)hi << 64) | lo;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const uint64_t lo = __shfl_xor((uint64_t)acc, off), hi = __shfl_xor((uint64_t)(acc >> 64), off);
+        acc += ((unsigned __int128)hi << 64) | lo;
+    }
+    if ((tid & 63) == 0) red[tid >> 6] = (__int128)acc;
+    __syncthreads();
+    if (tid == 0) {
+        unsigned __int128 t = 0;
+        for (int w = 0; w < NTHR / 64; ++w) t += (unsigned __int128)red[w];
+        partial[vb] = (__int128)t;
+    }
+}
+
+// W8: every column is 8 bytes wide (no per-load width dispatch).  partial (two
+// 8-byte columns only): the tile's sum of products of its selected rows.
 template <int NW, bool W8, bool TRACE, bool NT = false, int T = CT_LOG>
 __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, const uint8_t *__restrict__ mask,
                                                 uint64_t n, const uint64_t *__restrict__ tile_pre, Inst in,
-                                                TraceSlot *slot, char *lds_raw, uint32_t vb)
+                                                __int128 *__restrict__ partial, TraceSlot *slot, char *lds_raw,
+                                                uint32_t vb)
 {
     using TL = CTileOf<T>;
     constexpr int NTHR = 1 << (T - 4), AS = T - 4;
     dev::TileBuf buf{lds_raw};
-    uint32_t *c16 = reinterpret_cast<uint32_t *>(lds_raw + TL::lds_bytes());
+    uint32_t *c16 = reinterpret_cast<uint32_t *>(lds_raw + cbuf_bytes<T>());
     __shared__ uint32_t wsum[NTHR / 64];
     const uint32_t tid = threadIdx.x;
     const uint64_t tv = (uint64_t)vb << T;
@@ -524,14 +614,12 @@ __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, cons
     // rows, coalesced; issued before the scan
     const uint32_t lb = dev::lay_base<4>(tid, 6);
     uint64_t r[16][NW];
+    auto at_in = [&](int m) { return t0 + lb + 64u * m; };
+    ld_rows<W8, NT>(r, src, at_in);
 #pragma unroll
     for (int m = 0; m < 16; ++m)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            r[m][w] = W8 ? ld_row<NT>((const uint64_t *)src.c[w].p + t0 + lb + 64u * m)
-                         : ld_col<NT>(src.c[w], t0 + lb + 64u * m);
-            tr.at(8 + w, t0 + lb + 64u * m);
-        }
+        for (int w = 0; w < NW; ++w) tr.at(8 + w, at_in(m));
 
     // select bits and exclusive prefix: thread tid owns rows [16 tid, 16 tid + 16)
     uint32_t selm = 0;
@@ -565,6 +653,12 @@ __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, cons
     // read inside the wavefront up to layout 6, beyond it after the relayout's barriers
     c16[tid] = c0;
     crelayout<NW, T, 6, 0>(r, buf, tid);
+    if constexpr (NW == 2 && W8) {
+        if (partial) {
+            csum<NTHR>(r, selm, partial, vb, tid);
+            tr.at(16, vb);
+        }
+    }
     clevels0<NW>(r, selm, tbase + c0);
     crelayout<NW, T, 0, 4>(r, buf, tid);
     clevels<NW, 4, 4, 7>(r, c16, tbase, tid);
@@ -580,33 +674,29 @@ __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, cons
     }
     uint32_t tid_s = tid; // store addresses recomputed here (register pressure)
     asm volatile("" : "+v"(tid_s));
+    auto at_out = [&](int m) { return t0 + tid_s + ((uint32_t)m << AS); };
+    st_rows<W8, NT>(r, dst, at_out);
 #pragma unroll
     for (int m = 0; m < 16; ++m)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            const uint64_t i = t0 + tid_s + ((uint32_t)m << AS);
-            if (W8)
-                st_row<NT>((uint64_t *)dst.c[w].p + i, r[m][w]);
-            else
-                st_col<NT>(dst.c[w], i, r[m][w]);
-            tr.at(16 + w, i);
-        }
+        for (int w = 0; w < NW; ++w) tr.at(16 + w, at_out(m));
     tr.done((uint64_t)vb * NTHR + tid);
 }
 
 // dynamic LDS of the local pass: the relayout buffer and a count per thread
 template <int T>
-constexpr size_t clocal_lds() { return CTileOf<T>::lds_bytes() + ((size_t)4 << (T - 4)); }
+constexpr size_t clocal_lds() { return cbuf_bytes<T>() + ((size_t)4 << (T - 4)); }
 
 // XC: contiguous block ranges per XCD (dev::xcd_block)
 template <int NW, bool W8, bool TRACE, bool NT = false, int T = CT_LOG, bool XC = true>
-__global__ __launch_bounds__(1 << (T - 4)) void k_compact_local(Cols<NW> src, Cols<NW> dst,
+__global__ __launch_bounds__(1 << (T - 4), W8 ? 4 : 1) void k_compact_local(Cols<NW> src, Cols<NW> dst,
                                                                 const uint8_t *__restrict__ mask, uint64_t n,
                                                                 const uint64_t *__restrict__ tile_pre, Inst in,
-                                                                TraceSlot *slot)
+                                                                __int128 *__restrict__ partial, TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds_raw[];
-    b_compact_local<NW, W8, TRACE, NT, T>(src, dst, mask, n, tile_pre, in, slot, lds_raw, dev::xcd_block<XC>());
+    b_compact_local<NW, W8, TRACE, NT, T>(src, dst, mask, n, tile_pre, in, partial, slot, lds_raw,
+                                          dev::xcd_block<XC>());
 }
 
 // ---------------------------------------------------------- global levels
@@ -625,13 +715,12 @@ __device__ __forceinline__ void b_compact_global(Cols<NW> cols, const uint64_t *
     // the 2^S rows lie in one instance (q_lo + S <= its size class)
     const uint64_t pb = inst_row(in, base);
     uint64_t r[1 << S][NW];
+    auto at = [&](int m) { return pb + ((uint64_t)m << q_lo); };
+    ld_rows<false, NT>(r, cols, at);
 #pragma unroll
     for (int m = 0; m < (1 << S); ++m)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            r[m][w] = ld_col<NT>(cols.c[w], pb + ((uint64_t)m << q_lo));
-            tr.at(8 + w, pb + ((uint64_t)m << q_lo));
-        }
+        for (int w = 0; w < NW; ++w) tr.at(8 + w, at(m));
     // uniform part of base (bits >= 8 are shared by the wavefront)
     const uint64_t ubase = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(base >> 32)) << 32) |
                            __builtin_amdgcn_readfirstlane((uint32_t)base & ~0xFFu);
@@ -649,13 +738,11 @@ __device__ __forceinline__ void b_compact_global(Cols<NW> cols, const uint64_t *
             swap_rows<NW>(swap_lanes(d, q_lo + k), r[m], r[m | (1 << k)]);
         }
     }
+    st_rows<false, NT>(r, cols, at);
 #pragma unroll
     for (int m = 0; m < (1 << S); ++m)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            st_col<NT>(cols.c[w], pb + ((uint64_t)m << q_lo), r[m][w]);
-            tr.at(16 + w, pb + ((uint64_t)m << q_lo));
-        }
+        for (int w = 0; w < NW; ++w) tr.at(16 + w, at(m));
     tr.done(dev::gtid());
 }
 
@@ -706,7 +793,7 @@ __device__ __forceinline__ void b_compact_hybrid(Cols<NW> cols, const uint64_t *
     constexpr int C = T - S, NTHR = 1 << (T - 4), AS = T - 4;
     static_assert(S >= 5 && C >= 4, "hybrid widths 5..T-4");
     dev::TileBuf buf{lds_raw};
-    uint32_t *P = reinterpret_cast<uint32_t *>(lds_raw + TL::lds_bytes()); // low words of 2^S prefix counts
+    uint32_t *P = reinterpret_cast<uint32_t *>(lds_raw + cbuf_bytes<T>()); // low words of 2^S prefix counts
     const uint32_t tid = threadIdx.x;
     // row indices fit 32 bits (n_pad <= 2^32)
     const uint32_t runs = (1u << q_lo) >> C; // blocks per group of 2^(q_lo+S) rows
@@ -718,15 +805,12 @@ __device__ __forceinline__ void b_compact_hybrid(Cols<NW> cols, const uint64_t *
     uint64_t r[16][NW];
     {
         const uint32_t gl = j0 + grow(dev::lay_base<4>(tid, C));
+        auto at = [&](int m) { return ph + gl + grow((uint32_t)m << C); };
+        ld_rows<W8, NT>(r, cols, at);
 #pragma unroll
-        for (int m = 0; m < 16; ++m) {
-            const uint64_t i = ph + gl + grow((uint32_t)m << C);
+        for (int m = 0; m < 16; ++m)
 #pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                r[m][w] = W8 ? ld_row<NT>((const uint64_t *)cols.c[w].p + i) : ld_col<NT>(cols.c[w], i);
-                tr.at(8 + w, i);
-            }
-        }
+            for (int w = 0; w < NW; ++w) tr.at(8 + w, at(m));
     }
     __syncthreads(); // (resident blocks: the last step's reads of P)
     for (uint32_t k = tid; k < (1u << S); k += NTHR) {
@@ -749,72 +833,27 @@ __device__ __forceinline__ void b_compact_hybrid(Cols<NW> cols, const uint64_t *
     uint32_t tid_s = tid;
     asm volatile("" : "+v"(tid_s));
     const uint32_t gs = j0 + grow(dev::lay_base<4>(tid_s, AS));
+    auto at_out = [&](int m) { return ph + gs + grow((uint32_t)m << AS); };
+    st_rows<W8, NT>(r, cols, at_out);
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
-        const uint64_t i = ph + gs + grow((uint32_t)m << AS);
+    for (int m = 0; m < 16; ++m)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            if (W8)
-                st_row<NT>((uint64_t *)cols.c[w].p + i, r[m][w]);
-            else
-                st_col<NT>(cols.c[w], i, r[m][w]);
-            tr.at(16 + w, i);
-        }
-    }
+        for (int w = 0; w < NW; ++w) tr.at(16 + w, at_out(m));
     tr.done((uint64_t)vb * NTHR + tid);
 }
 
 template <int S, int T>
-constexpr size_t chybrid_lds() { return CTileOf<T>::lds_bytes() + ((size_t)4 << S); }
+constexpr size_t chybrid_lds() { return cbuf_bytes<T>() + ((size_t)4 << S); }
 
 template <int NW, int S, bool W8, bool TRACE, bool NT = false, int T = CT_LOG, bool XC = true>
-__global__ __launch_bounds__(1 << (T - 4)) void k_compact_hybrid(Cols<NW> cols, const uint64_t *__restrict__ tile_pre,
+__global__ __launch_bounds__(1 << (T - 4), W8 ? 4 : 1) void k_compact_hybrid(Cols<NW> cols, const uint64_t *__restrict__ tile_pre,
                                                                  int q_lo, Inst in, TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds_raw[];
     b_compact_hybrid<NW, S, W8, TRACE, NT, T>(cols, tile_pre, q_lo, in, slot, lds_raw, dev::xcd_block<XC>());
 }
 
-// ------------------------------------------------------- int128 SUM pass
-
-// Exact SUM(a[i] * b[i]) over rows i < count (count read on the device);
-// every row is read, rows >= count contribute a multiplied-out zero.
-// red: 256 int128 of LDS.
-template <bool NT = false>
-__device__ __forceinline__ void b_sum_prod_i128(const int64_t *__restrict__ a, const int64_t *__restrict__ b,
-                                                uint64_t n_pad, const uint64_t *__restrict__ count,
-                                                __int128 *__restrict__ partial, TraceSlot *slot, __int128 *red,
-                                                uint32_t vb, uint32_t nvb)
-{
-    dev::Atr tr(slot);
-    const uint64_t m = *count;
-    __int128 acc = 0;
-    for (uint64_t i = (uint64_t)vb * 256 + threadIdx.x; i < n_pad; i += (uint64_t)nvb * 256) {
-        const __int128 prod = (__int128)ld_row<NT>(a + i) * (__int128)ld_row<NT>(b + i);
-        acc += prod * (__int128)(i < m);
-        tr.at(8, i);
-    }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < (uint32_t)off) red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        partial[vb] = red[0];
-        tr.at(16, vb);
-    }
-    tr.done(dev::gtid());
-}
-
-template <bool NT = false>
-__global__ __launch_bounds__(256) void k_sum_prod_i128(const int64_t *__restrict__ a, const int64_t *__restrict__ b,
-                                                       uint64_t n_pad, const uint64_t *__restrict__ count,
-                                                       __int128 *__restrict__ partial, TraceSlot *slot)
-{
-    __shared__ __int128 red[256];
-    b_sum_prod_i128<NT>(a, b, n_pad, count, partial, slot, red, blockIdx.x, gridDim.x);
-}
+// --------------------------------------------------------- int128 SUM
 
 // One 256-thread block: strided partial sums, then a tree in LDS (exact:
 // int128 addition is associative).
@@ -823,10 +862,18 @@ __device__ __forceinline__ void b_sum_final(const __int128 *__restrict__ partial
                                             TraceSlot *slot, __int128 *red)
 {
     dev::Atr tr(slot);
+    // groups of 8 loads in flight (one per tile: 2^16 partials at 2^29 rows)
+    constexpr uint32_t G = 8;
     __int128 s = 0;
-    for (uint32_t i = threadIdx.x; i < np; i += 256) {
-        s += partial[i];
-        tr.at(8, i);
+    for (uint32_t i0 = threadIdx.x; i0 < np; i0 += 256 * G) {
+        __int128 v[G];
+#pragma unroll
+        for (uint32_t j = 0; j < G; ++j) v[j] = i0 + 256 * j < np ? partial[i0 + 256 * j] : 0;
+#pragma unroll
+        for (uint32_t j = 0; j < G; ++j) {
+            s += v[j];
+            if (i0 + 256 * j < np) tr.at(8, i0 + 256 * j);
+        }
     }
     red[threadIdx.x] = s;
     __syncthreads();
