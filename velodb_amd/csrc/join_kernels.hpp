@@ -770,10 +770,23 @@ __device__ __forceinline__ void b_dense_out(const int64_t *__restrict__ part_sum
     const uint32_t t = threadIdx.x;
     int64_t s = 0, c = 0;
     const uint64_t total = (uint64_t)nparts * G;
-    for (uint64_t i = t; i < total; i += NT) {
-        s += part_sum[i];
-        c += part_cnt[i];
-        tr.at(1, i);
+    // groups of 8 loads in flight: one block walks all partials, so its time is
+    // memory round trips (2048 x 32 partials one by one: 33 us)
+    constexpr uint32_t B = 8;
+    for (uint64_t i0 = t; i0 < total; i0 += (uint64_t)NT * B) {
+        int64_t vs[B], vc[B];
+#pragma unroll
+        for (uint32_t j = 0; j < B; ++j) {
+            const uint64_t i = i0 + (uint64_t)j * NT;
+            vs[j] = i < total ? part_sum[i] : 0;
+            vc[j] = i < total ? part_cnt[i] : 0;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < B; ++j) {
+            s += vs[j];
+            c += vc[j];
+            if (i0 + (uint64_t)j * NT < total) tr.at(1, i0 + (uint64_t)j * NT);
+        }
     }
     ss[t] = s;
     sc[t] = c;
@@ -808,7 +821,13 @@ __device__ __forceinline__ void b_dense_out(const int64_t *__restrict__ part_sum
     }
     // a fact value that the 12-byte union cannot hold: report UINT64_MAX
     int over = 0;
-    for (uint32_t b = t; b < n_bad; b += NT) over |= (int)(bad[b] != 0);
+    for (uint32_t b0 = t; b0 < n_bad; b0 += NT * B) {
+        uint32_t v[B];
+#pragma unroll
+        for (uint32_t j = 0; j < B; ++j) v[j] = b0 + j * NT < n_bad ? bad[b0 + j * NT] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < B; ++j) over |= (int)(v[j] != 0);
+    }
     over = __syncthreads_or(over);
     if (t == 0 && out_n) *out_n = over ? ~0ull : present;
     tr.done(dev::gtid());
