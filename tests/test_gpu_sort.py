@@ -381,3 +381,37 @@ def test_sort_small_tiles(vctx, log2n, short):
         assert np.array_equal(from_dev(didx, np.int64), eidx)
         for dc, ec, t in zip(dcols, ecols, types):
             assert np.array_equal(from_dev(dc, TYPES[t]).view(np.uint8), ec.view(np.uint8))
+
+
+@pytest.mark.parametrize("log2n,short", [(22, 5), (23, 0), (23, 1001), (24, 3)])
+def test_sort_wide_tiles(vctx, log2n, short):
+    """Sizes whose passes above the local one run on the wide tiles: the
+    12-byte records, the 16-byte ones (a shuffle's two forms agree and give a
+    permutation) and OP_SORT of one and two key words, against torch's sort."""
+    import torch
+    npad, n = 1 << log2n, (1 << log2n) - short
+    print(f"wide tiles n={n} npad={npad}", flush=True)
+    g = torch.Generator(device="cuda:0").manual_seed(log2n)
+    k0 = torch.randint(0, 1 << 40, (npad,), device="cuda:0", generator=g)
+    k, p = k0.clone(), torch.arange(npad, device="cuda:0", dtype=torch.int32)
+    vctx.sort_kp(k, p, n, npad)
+    ek, order = torch.sort(k0[:n], stable=True)
+    assert torch.equal(k[:n], ek) and torch.equal(p[:n].long(), order)
+    assert torch.equal(p[n:].long(), torch.arange(n, npad, device="cuda:0")) and bool(torch.all(k[n:] == -1))
+    a, b = (torch.arange(npad, device="cuda:0", dtype=torch.int32) for _ in range(2))
+    perm = torch.empty_like(a)
+    vctx.shuffle(a, npad, 3, perm_out=perm, n=n)
+    vctx.shuffle(b, npad, 3, n=n)
+    assert torch.equal(a, perm) and torch.equal(a, b)
+    assert torch.equal(torch.sort(a).values.long(), torch.arange(npad, device="cuda:0"))
+    idx = torch.empty(npad, dtype=torch.int64, device="cuda:0")
+    k = k0.clone()
+    vctx.sort([k], [5], [True], idx, n, npad)  # unique keys but for a few ties
+    assert torch.equal(k[:n], ek) and torch.equal(k0[idx[:n]], ek)
+    first = torch.randint(-3, 3, (npad,), device="cuda:0", generator=g, dtype=torch.int32)
+    c, k = first.clone(), k0.clone()
+    vctx.sort([c, k], [4, 5], [False, True], idx, n, npad)
+    o = torch.sort(k0[:n], stable=True).indices
+    o = o[torch.sort(first[:n][o], descending=True, stable=True).indices]
+    assert torch.equal(c[:n], first[:n][o]) and torch.equal(k[:n], k0[:n][o])
+    assert torch.equal(torch.sort(idx[:n]).values, torch.arange(n, device="cuda:0"))

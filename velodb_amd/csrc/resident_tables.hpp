@@ -67,11 +67,12 @@
     VO_SORT_H(X, kv, sortimpl::RecKV, 12, 4, 6) VO_SORT_H(X, kv, sortimpl::RecKV, 12, 4, 7)
 
 // multi-column records: as launch mode
-#define VO_SORT_M12_BODIES(X)                                                                                      \
+#define VO_SORT_M1_BODIES(X)                                                                                       \
     VO_SORT_TILE(X, m1, sortimpl::RecM1, 12, 4)                                                                    \
     VO_SORT_G(X, m1, sortimpl::RecM1, 1) VO_SORT_G(X, m1, sortimpl::RecM1, 2) VO_SORT_G(X, m1, sortimpl::RecM1, 3) \
     VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 4) VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 5)                        \
-    VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 6) VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 7)                        \
+    VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 6) VO_SORT_H(X, m1, sortimpl::RecM1, 12, 4, 7)
+#define VO_SORT_M2_BODIES(X)                                                                                       \
     VO_SORT_TILE(X, m2, sortimpl::RecM2, 12, 4)                                                                    \
     VO_SORT_G(X, m2, sortimpl::RecM2, 1) VO_SORT_G(X, m2, sortimpl::RecM2, 2) VO_SORT_G(X, m2, sortimpl::RecM2, 3) \
     VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 4) VO_SORT_H(X, m2, sortimpl::RecM2, 12, 4, 5)                        \
@@ -83,7 +84,7 @@
     VO_SORT_H(X, m4, sortimpl::RecM4, 11, 3, 6)                                                                    \
     VO_SORT_TILE(X, m8, sortimpl::RecM8, 10, 2)                                                                    \
     VO_SORT_G(X, m8, sortimpl::RecM8, 1) VO_SORT_G(X, m8, sortimpl::RecM8, 2)
-#define VO_SORT_M_BODIES(X) VO_SORT_M12_BODIES(X) VO_SORT_M48_BODIES(X)
+#define VO_SORT_M_BODIES(X) VO_SORT_M1_BODIES(X) VO_SORT_M2_BODIES(X) VO_SORT_M48_BODIES(X)
 
 #define VO_SORT_PACK_BODIES(X)                                                                                     \
     X(kB_sort_pack, (smulti_k::k_pack_keys), (smulti_k::b_pack_keys(a..., vb, nvb)), 0)                           \

@@ -410,78 +410,103 @@ struct TileCT {
     // choice: 64 lanes on consecutive records, a wavefront on its own ones.
     static constexpr int A_IO = T_LOG - R_LOG < 6 ? T_LOG - R_LOG : 6;
 
-    // layout reached after stages (q_start .. 0) starting from layout a;
-    // stage 0 in layout 1 runs across lane pairs and keeps the layout
+    // Layout for stage q: as many of the stages below it as the registers hold,
+    // but none below the last one wanted.
+    static constexpr int layout_for(int q, int qlo)
+    {
+        const int a = q - R_LOG + 1 > qlo ? q - R_LOG + 1 : qlo;
+        return a < T_LOG - R_LOG ? a : T_LOG - R_LOG;
+    }
+    // Stages on bits below layouts 1 and 2 run between lanes (LANES) and keep
+    // the layout.
+    static constexpr bool lane_stage(int q, int a) { return LANES && a <= 2 && q < a; }
+
+    // layout reached after stages (q_start .. qlo) starting from layout a
     static constexpr int end_layout(int q, int a, int qlo = 0)
     {
         while (q >= qlo) {
-            if (LANE0 && q == 0 && a == 1) break;
-            if (!(a <= q && q < a + R_LOG)) a = q - R_LOG + 1 > 0 ? q - R_LOG + 1 : 0;
+            if (lane_stage(q, a)) break;
+            if (!(a <= q && q < a + R_LOG)) a = layout_for(q, qlo);
             q = (a > qlo ? a : qlo) - 1;
         }
         return a;
     }
 
-    // Stage 0 of level P in layout 1: record index bit 0 is thread index
-    // bit 0, so the pair of register m is register m of lanes (2t, 2t+1).
-    // Issue-bound, so it is kept to six VALU instructions a record: the borrow
-    // chain of lt_mask96 reads the partner's words through a DPP quad
-    // permutation (lanes 1 0 3 2), and the words move by DPP moves under the
-    // execution mask of the swapping pairs.  (Written with selects it compiled
-    // to 64-bit compares per record and took 10 us of a 2^23-record pass, as
-    // long as the other twelve stages and the three relayouts together.)
+    // Stage Q (0 or 1) of level P in layouts 1 and 2: record index bit Q is
+    // thread index bit Q, so the pair of register m is register m of two lanes
+    // of a quad.  Issue-bound, so it is kept to six VALU instructions a record:
+    // the borrow chain of lt_mask96 reads the partner's words through a DPP quad
+    // permutation, and the words move by DPP moves under the execution mask of
+    // the swapping pairs.  (Written with selects it compiled to 64-bit compares
+    // per record and took 10 us of a 2^23-record pass, as long as the other
+    // twelve stages and the three relayouts together.)
     // Built for the 12-byte record, the only one whose layouts need it.
-    static constexpr bool LANE0 = R::TIE && R::KW == 1 && sizeof(P) == 4;
+    static constexpr bool LANES = R::TIE && R::KW == 1 && sizeof(P) == 4;
 
     // Exchanges the records of the lane pairs that are out of order: ascending
-    // pairs where the odd lane's record is the smaller one, descending pairs
+    // pairs where the upper lane's record is the smaller one, descending pairs
     // (both lanes set in descm) where it is not (equal records are identical).
+    template <int Q>
     static __device__ __forceinline__ void lane_cmpx(R &r, uint64_t descm)
     {
         uint32_t w0 = (uint32_t)r.p, w1 = (uint32_t)r.k[0], w2 = (uint32_t)(r.k[0] >> 32), t;
         uint64_t sw, ex;
-        // s_nop: a DPP read needs two wait states after a VALU write of the register
-        asm("s_nop 1\n\t"
-            "v_sub_co_u32_dpp %3, vcc, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_subb_co_u32_dpp %3, vcc, %1, %1, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_subb_co_u32_dpp %3, vcc, %2, %2, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "s_and_b64 %4, vcc, %6\n\t" // partner < own, even lanes
-            "s_lshl_b64 vcc, %4, 1\n\t"
-            "s_or_b64 %4, %4, vcc\n\t" // both lanes of the pair
-            "s_xor_b64 %4, %4, %7\n\t"
-            "s_and_saveexec_b64 %5, %4\n\t"
-            "v_mov_b32_dpp %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_mov_b32_dpp %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "v_mov_b32_dpp %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-            "s_mov_b64 exec, %5"
-            : "+v"(w0), "+v"(w1), "+v"(w2), "=&v"(t), "=&s"(sw), "=&s"(ex)
-            : "s"(0x5555555555555555ull), "s"(descm)
-            : "vcc", "scc");
+        // s_nop: a DPP read needs two wait states after a VALU write of the
+        // register; %6 holds the lower lane of every pair
+#define VO_LANE_CMPX(PERM, SHIFT, LOWER)                                                                               \
+    asm("s_nop 1\n\t"                                                                                                  \
+        "v_sub_co_u32_dpp %3, vcc, %0, %0 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                            \
+        "v_subb_co_u32_dpp %3, vcc, %1, %1, vcc quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                      \
+        "v_subb_co_u32_dpp %3, vcc, %2, %2, vcc quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                      \
+        "s_and_b64 %4, vcc, %6\n\t"                                                                                    \
+        "s_lshl_b64 vcc, %4, " SHIFT "\n\t"                                                                            \
+        "s_or_b64 %4, %4, vcc\n\t"                                                                                     \
+        "s_xor_b64 %4, %4, %7\n\t"                                                                                     \
+        "s_and_saveexec_b64 %5, %4\n\t"                                                                                \
+        "v_mov_b32_dpp %0, %0 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                        \
+        "v_mov_b32_dpp %1, %1 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                        \
+        "v_mov_b32_dpp %2, %2 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                                        \
+        "s_mov_b64 exec, %5"                                                                                           \
+        : "+v"(w0), "+v"(w1), "+v"(w2), "=&v"(t), "=&s"(sw), "=&s"(ex)                                                 \
+        : "s"(LOWER), "s"(descm)                                                                                       \
+        : "vcc", "scc")
+        if constexpr (Q == 0)
+            VO_LANE_CMPX("[1,0,3,2]", "1", 0x5555555555555555ull);
+        else
+            VO_LANE_CMPX("[2,3,0,1]", "2", 0x3333333333333333ull);
+#undef VO_LANE_CMPX
         r.p = (P)w0;
         r.k[0] = (uint64_t)w1 | ((uint64_t)w2 << 32);
     }
 
-    template <int P>
-    static __device__ __forceinline__ void lane_stage0(R (&r)[RR], uint32_t tau, bool asc_hi, int p_top)
+    template <int P, int A, int Q>
+    static __device__ __forceinline__ void lane_stages(R (&r)[RR], uint32_t tau, bool asc_hi, int p_top)
     {
-        const uint32_t base = lay_base<R_LOG>(tau, 1);
+        const uint32_t base = lay_base<R_LOG>(tau, A);
 #pragma unroll
         for (int m = 0; m < RR; ++m) {
             bool asc;
             if constexpr (P < 0) {
                 asc = asc_hi;
             } else {
-                const uint32_t l = base | ((uint32_t)m << 1);
+                const uint32_t l = base | ((uint32_t)m << A);
                 asc = (P >= p_top) | (P >= T_LOG ? asc_hi : (((l >> P) & 1u) == 0));
             }
-            lane_cmpx(r[m], __builtin_amdgcn_ballot_w64(!asc));
+            lane_cmpx<Q>(r[m], __builtin_amdgcn_ballot_w64(!asc));
         }
+        if constexpr (Q > 0) lane_stages<P, A, Q - 1>(r, tau, asc_hi, p_top);
     }
 
-    // LDS bytes of one block: a single column buffer (the widest column)
-    // that every column passes through in turn.  Keeping it to 8 B per slot
-    // lets two 2^13-record tiles share a CU's 160 KB.
-    static constexpr size_t lds_bytes() { return (size_t)TPAD * sizeof(uint64_t); }
+    // LDS of one block: a single buffer that every column passes through in
+    // turn.  On 2^14-record tiles the 12-byte records pass in 32-bit words: half
+    // the buffer, and 64 VGPRs instead of 72-75, so two 1024-thread blocks share
+    // a CU.  On 2^13-record tiles the same gives four blocks a CU instead of two
+    // and is faster at 2^23 records (748 -> 699 us) but slower below (one tile a
+    // CU at 2^20: 176 -> 184 us, barriers) and above (39.5 -> 40.6 ms at 2^28).
+    // Other records keep 8-byte columns (halves cost them registers and moves:
+    // two key words 108 -> 133 VGPRs).
+    static constexpr bool NARROW = R::TIE && R::KW == 1 && sizeof(P) == 4 && T_LOG >= 14;
+    static constexpr size_t lds_bytes() { return (size_t)TPAD * (NARROW ? 4 : 8); }
 
     template <int A, typename C>
     static __device__ __forceinline__ void put_col(const C (&v)[RR], C *buf, uint32_t tau, uint64_t &h, uint32_t &n)
@@ -544,7 +569,7 @@ struct TileCT {
 
     // Before a column enters the buffer: every wave is done with what it read
     // there.  Between relayouts inside the wavefronts each wave only uses its
-    // own part, [lpos(first record), ...) of 8 bytes a record.
+    // own part, of one column slot a record.
     template <int A_OLD, int A_NEW>
     static __device__ __forceinline__ void relayout(R (&r)[RR], TileBuf &lds, uint32_t tau, uint64_t &h, uint32_t &n)
     {
@@ -554,31 +579,77 @@ struct TileCT {
                 __syncthreads();
             else
                 wave_fence();
-#pragma unroll
-            for (int w = 0; w < R::KW; ++w) {
-                uint64_t v[RR];
-#pragma unroll
-                for (int m = 0; m < RR; ++m) v[m] = r[m].k[w];
-                move_col<A_OLD, A_NEW>(v, reinterpret_cast<uint64_t *>(lds.p), tau, h, n);
-                if constexpr (IN)
-                    wave_fence();
-                else
-                    __syncthreads();
-#pragma unroll
-                for (int m = 0; m < RR; ++m) r[m].k[w] = v[m];
-            }
-            P v[RR];
-#pragma unroll
-            for (int m = 0; m < RR; ++m) v[m] = r[m].p;
-            P *buf = reinterpret_cast<P *>(lds.p);
-            // a narrower column starts where the wavefront's 8-byte part does
-            if constexpr (IN && sizeof(P) < 8)
-                buf += lpos(__builtin_amdgcn_readfirstlane(tau >> 6) << (6 + R_LOG)) * (8 / sizeof(P) - 1);
-            move_col<A_OLD, A_NEW>(v, buf, tau, h, n);
-#pragma unroll
-            for (int m = 0; m < RR; ++m) r[m].p = v[m];
+            if constexpr (NARROW)
+                move_words<A_OLD, A_NEW>(r, lds, tau, h, n);
+            else
+                move_cols<A_OLD, A_NEW>(r, lds, tau, h, n);
             lds.shared = !IN;
         }
+    }
+
+    // between two columns of one relayout
+    template <bool IN>
+    static __device__ __forceinline__ void next_col()
+    {
+        if constexpr (IN)
+            wave_fence();
+        else
+            __syncthreads();
+    }
+
+    template <int A_OLD, int A_NEW>
+    static __device__ __forceinline__ void move_words(R (&r)[RR], TileBuf &lds, uint32_t tau, uint64_t &h, uint32_t &n)
+    {
+        constexpr bool IN = in_wave(A_OLD, A_NEW);
+        constexpr int WORDS = 2 + (int)sizeof(P) / 4;
+        uint32_t *buf = reinterpret_cast<uint32_t *>(lds.p);
+#pragma unroll
+        for (int w = 0; w < WORDS; ++w) {
+            uint32_t v[RR];
+#pragma unroll
+            for (int m = 0; m < RR; ++m) {
+                const uint64_t x = w < 2 ? r[m].k[0] : (uint64_t)r[m].p;
+                v[m] = (w & 1) ? (uint32_t)(x >> 32) : (uint32_t)x;
+            }
+            move_col<A_OLD, A_NEW>(v, buf, tau, h, n);
+            if (w + 1 < WORDS) next_col<IN>();
+#pragma unroll
+            for (int m = 0; m < RR; ++m) {
+                const uint64_t x = w < 2 ? r[m].k[0] : (uint64_t)r[m].p;
+                const uint64_t y = (w & 1) ? (x & 0xFFFFFFFFull) | ((uint64_t)v[m] << 32)
+                                           : (x & ~0xFFFFFFFFull) | v[m];
+                if (w < 2)
+                    r[m].k[0] = y;
+                else
+                    r[m].p = (P)y;
+            }
+        }
+    }
+
+    template <int A_OLD, int A_NEW>
+    static __device__ __forceinline__ void move_cols(R (&r)[RR], TileBuf &lds, uint32_t tau, uint64_t &h, uint32_t &n)
+    {
+        constexpr bool IN = in_wave(A_OLD, A_NEW);
+#pragma unroll
+        for (int w = 0; w < R::KW; ++w) {
+            uint64_t v[RR];
+#pragma unroll
+            for (int m = 0; m < RR; ++m) v[m] = r[m].k[w];
+            move_col<A_OLD, A_NEW>(v, reinterpret_cast<uint64_t *>(lds.p), tau, h, n);
+            next_col<IN>();
+#pragma unroll
+            for (int m = 0; m < RR; ++m) r[m].k[w] = v[m];
+        }
+        P v[RR];
+#pragma unroll
+        for (int m = 0; m < RR; ++m) v[m] = r[m].p;
+        P *buf = reinterpret_cast<P *>(lds.p);
+        // a narrower column starts where the wavefront's 8-byte part does
+        if constexpr (IN && sizeof(P) < 8)
+            buf += lpos(__builtin_amdgcn_readfirstlane(tau >> 6) << (6 + R_LOG)) * (8 / sizeof(P) - 1);
+        move_col<A_OLD, A_NEW>(v, buf, tau, h, n);
+#pragma unroll
+        for (int m = 0; m < RR; ++m) r[m].p = v[m];
     }
 
     // Stages q = QHI .. QLO of level P (P >= 0 compile-time; P < 0 means a
@@ -610,11 +681,11 @@ struct TileCT {
     static __device__ __forceinline__ void level(R (&r)[RR], TileBuf &lds, uint32_t tau, bool asc_hi, int p_top,
                                                  uint64_t &h, uint32_t &n)
     {
-        if constexpr (LANE0 && Q == 0 && A == 1 && QLO == 0) {
-            lane_stage0<P>(r, tau, asc_hi, p_top);
+        if constexpr (Q >= QLO && lane_stage(Q, A)) {
+            lane_stages<P, A, Q>(r, tau, asc_hi, p_top);
         } else if constexpr (Q >= QLO) {
             constexpr bool covered = (A <= Q && Q < A + R_LOG);
-            constexpr int AN = covered ? A : (Q - R_LOG + 1 > 0 ? Q - R_LOG + 1 : 0);
+            constexpr int AN = covered ? A : layout_for(Q, QLO);
             constexpr int LO = AN > QLO ? AN : QLO;
             relayout<A, AN>(r, lds, tau, h, n);
             stages<P, AN, Q, LO>(r, tau, asc_hi, p_top);

@@ -259,7 +259,7 @@ __device__ __forceinline__ void body_merge(Bufs<R> b, IMap map, int p, int p_top
 }
 
 template <class R, int T_LOG, int R_LOG, int BLOCK, bool TRACE, int CP = 0, bool XC = true>
-__global__ __launch_bounds__(BLOCK) void k_sort_merge(Bufs<R> b, IMap map, int p, int p_top, TraceSlot *slot)
+__global__ __launch_bounds__(BLOCK, BLOCK >= 1024 ? 8 : 1) void k_sort_merge(Bufs<R> b, IMap map, int p, int p_top, TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
     body_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP>(b, map, p, p_top, slot, lds, xcd_block<XC>());
@@ -379,7 +379,7 @@ __device__ __forceinline__ void body_strided(Bufs<R> b, IMap map, int p, int q_l
 }
 
 template <class R, int T_LOG, int R_LOG, int BLOCK, int S, bool TRACE, int CP = 0, bool XC = true>
-__global__ __launch_bounds__(BLOCK) void k_sort_hybrid(Bufs<R> b, IMap map, int p, int q_lo, int p_top,
+__global__ __launch_bounds__(BLOCK, BLOCK >= 1024 ? 8 : 1) void k_sort_hybrid(Bufs<R> b, IMap map, int p, int q_lo, int p_top,
                                                        TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(BLOCK) void k_sort_hybrid(Bufs<R> b, IMap map, int 
 }
 
 template <class R, int T_LOG, int R_LOG, int BLOCK, int S, bool TRACE, int CP = 0, bool XC = true>
-__global__ __launch_bounds__(BLOCK) void k_sort_wrap(Bufs<R> b, IMap map, int p, int q_lo, int p_top, TraceSlot *slot)
+__global__ __launch_bounds__(BLOCK, BLOCK >= 1024 ? 8 : 1) void k_sort_wrap(Bufs<R> b, IMap map, int p, int q_lo, int p_top, TraceSlot *slot)
 {
     extern __shared__ __align__(16) char lds[];
     body_strided<R, T_LOG, R_LOG, BLOCK, T_LOG - S, true, TRACE, CP>(b, map, p, q_lo, p_top, slot, lds,
@@ -450,8 +450,11 @@ using dev::IMap;
 constexpr uint64_t kMaxSortRows = 1ull << 29;
 
 struct Pass {
-    int kind; // 0 tiny, 1 local, 2 global, 3 merge, 4 hybrid, 5 wrap
+    // 0 tiny, 1 local, 2 global, and on tiles of the local pass's size 3 merge,
+    // 4 hybrid; on tiles of 2^w records 5 wrap, 6 merge, 7 hybrid
+    int kind;
     int p, q_lo, s;
+    int w = 0;
 };
 
 // Pass schedule for n_log = log2(n_pad) with tiles of 2^t_log and at most
@@ -509,10 +512,11 @@ inline std::vector<Pass> plan_passes(int n_log, int t_log, int s_max, int r_log,
 // next (wrap).  Found by dynamic programming from the end over (level p, next
 // stage q); the costs are one pass's time at 2^28 records relative to a copy of
 // the array (below the MALL the order is the same).  A level-by-level schedule
-// needs ceil((p - t_log) / h_max) + 1 passes for level p; this one comes close
-// to (p - 5) / h_max on average: 31 passes instead of 38 at 2^28 on 2^13-record
-// tiles, 18 instead of 23 at 2^23.
-inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int s_max, int r_log, int h_max)
+// needs ceil((p - t_log) / h_max) + 1 passes for level p; this one, on tiles of
+// 2^w_log records above the local pass's 2^t_log, comes close to (p - 5) /
+// (w_log - 5) on average: at 2^28 31 passes instead of 38 on 2^13-record tiles
+// and 28 on 2^14-record ones.
+inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int w_log, int s_max, int r_log)
 {
     std::vector<Pass> v;
     if (n_log <= t_log) return plan_passes(n_log, t_log, s_max, r_log);
@@ -538,13 +542,13 @@ inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int s_max, int r_log
             };
             for (int s = 1; s <= s_max && q - s + 1 >= 8; ++s)
                 consider(s <= 3 ? 1.f : 1.08f, {2, p, q - s + 1, s}, p, q - s);
-            for (int s = 4; s <= h_max; ++s)
-                if (q - s + 1 >= t_log - s) consider(s <= 7 ? 1.1f : 1.14f, {4, p, q - s + 1, s}, p, q - s);
-            if (q < t_log) consider(1.12f, {3, p, 0, 0}, p, -1);
+            for (int s = 4; s <= w_log - 5; ++s) // runs of 2^(w_log - s) records, at least 32
+                if (q - s + 1 >= w_log - s) consider(s <= w_log - 6 ? 1.1f : 1.14f, {7, p, q - s + 1, s, w_log}, p, q - s);
+            if (q < w_log) consider(1.12f, {6, p, 0, 0, w_log}, p, -1);
             // stages q .. 0 and the next level's first s (a run of 32 records
             // may repeat a stage above q, which changes nothing)
-            const int c = std::max(5, q + 1), s = t_log - c;
-            if (s >= 1 && p < n_log) consider(c <= 5 ? 1.17f : 1.13f, {5, p + 1, p + 1 - s, s}, p + 1, p - s);
+            const int c = std::max(5, q + 1), s = w_log - c;
+            if (s >= 1 && p < n_log) consider(c <= 5 ? 1.17f : 1.13f, {5, p + 1, p + 1 - s, s, w_log}, p + 1, p - s);
         }
     for (int p = t_log + 1, q = t_log; p <= n_log;) {
         const Best &b = best[p][q];
@@ -563,11 +567,12 @@ inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int s_max, int r_log
 // WRAP = false builds the level-by-level schedule alone, BATCH = true the
 // passes over many small instances whose arrays together exceed the MALL.
 template <class R, int T_LOG, int R_LOG, int BLOCK, int S_MAX, int H_MAX = 0, int S_LARGE = S_MAX, int LARGE_LOG = 64,
-          int HW_MAX = 0, bool WRAP = true, bool BATCH = false>
+          int HW_MAX = 0, int W_LOG = T_LOG, bool WRAP = true, bool BATCH = false>
 struct SortImpl {
     static_assert(T_LOG >= 8, "global passes need q_lo >= 8 (256-thread blocks)");
     static_assert(H_MAX == 0 || (T_LOG - H_MAX >= 5 && BLOCK << R_LOG == 1 << T_LOG), "hybrid tile shape");
     static_assert(S_LARGE >= 1 && S_LARGE <= S_MAX, "register cap for large sorts");
+    static_assert(W_LOG >= T_LOG && W_LOG - R_LOG <= 10, "wide tiles");
 
     static int smax(vo_ctx *ctx, int n_log)
     {
@@ -579,20 +584,28 @@ struct SortImpl {
     // The default tuning runs the wrapped schedule; a tuning word that picks
     // pass widths or block shapes, and recorded programs (whose bodies they
     // are), run level by level.
-    static std::vector<Pass> plan(vo_ctx *ctx, int n_log)
+    // Wide tiles take one more stage bit per pass (28 passes instead of 31 for
+    // 2^28 12-byte records, 32 instead of 37 for 16-byte ones) with twice the
+    // threads behind each barrier.  They are used from 512 tiles, two a CU:
+    // 12-byte records at 2^22 (256 tiles) 366 -> 420 us, 2^23 748 -> 728, 2^24
+    // 1553 -> 1507, 2^26 8.39 -> 7.89 ms, 2^28 39.5 -> 37.1; 16-byte ones at 2^22
+    // 549 -> 546 us, 2^24 2.40 -> 2.30 ms, 2^26 12.9 -> 12.0; two key words at
+    // 2^22 758 -> 749 us, 2^24 3.90 -> 3.59 ms, 2^26 18.1 -> 16.0.
+    static std::vector<Pass> plan(vo_ctx *ctx, int n_log, uint64_t n_virtual)
     {
         const SortTuning &t = ctx->tuning, d;
         const bool wrapped = WRAP && !ctx->rec && t.max_fused_stages == d.max_fused_stages &&
                              t.max_hybrid_stages == d.max_hybrid_stages && !t.pipe_merge && !t.wide_block &&
                              !t.flip_hybrid_block;
         if (!wrapped) return plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx));
-        static const std::vector<std::vector<Pass>> plans = [] {
+        static const auto make = [](int w) {
             std::vector<std::vector<Pass>> v;
             for (int l = 0; (1ull << l) <= kMaxSortRows; ++l)
-                v.push_back(plan_wrapped(l, T_LOG, l >= LARGE_LOG ? S_LARGE : S_MAX, R_LOG, H_MAX));
+                v.push_back(plan_wrapped(l, T_LOG, w, l >= LARGE_LOG ? S_LARGE : S_MAX, R_LOG));
             return v;
-        }();
-        return plans[n_log];
+        };
+        static const std::vector<std::vector<Pass>> plans = make(T_LOG), wide = make(W_LOG);
+        return (n_log >= W_LOG && (n_virtual >> W_LOG) >= 512 ? wide : plans)[n_log];
     }
 
     template <bool TRACE, int S, int RL, int BL, int CP, bool XC>
@@ -653,22 +666,47 @@ struct SortImpl {
         return false;
     }
 
-    // Wrap passes of S = 1 .. T_LOG - 5 stages of the upper level.
-    template <bool TRACE, int CP, bool XC, int S = 1>
-    static void launch_wrap(vo_ctx *ctx, Bufs<R> b, IMap map, int p, int q_lo, int s, int p_top, uint64_t n_virtual)
+    // A kernel over tiles of 2^WL records.
+    template <bool TRACE, int WL, class K, class... A>
+    static void launch_tiles(vo_ctx *ctx, const char *family, uint64_t n_virtual, uint64_t hash, K k, A... args)
     {
-        if constexpr (WRAP && S <= T_LOG - 5) {
-            if (s != S) return launch_wrap<TRACE, CP, XC, S + 1>(ctx, b, map, p, q_lo, s, p_top, n_virtual);
-            static const char *const names[] = {"sort_wrap_s1", "sort_wrap_s2", "sort_wrap_s3", "sort_wrap_s4",
-                                                "sort_wrap_s5", "sort_wrap_s6", "sort_wrap_s7", "sort_wrap_s8"};
-            const size_t lds = dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes();
-            LaunchInfo li{names[S - 1], dim3((uint32_t)(n_virtual >> T_LOG)), dim3(BLOCK), (uint32_t)lds,
-                          hash_mix(hash_mix(p, q_lo), hash_mix(S + 200, p_top))};
-            auto k = dev::k_sort_wrap<R, T_LOG, R_LOG, BLOCK, S, TRACE, CP, XC>;
-            VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            launch(ctx, li, k, b, map, p, q_lo, p_top, trace_slot(ctx));
+        const size_t lds = dev::TileCT<R, WL, R_LOG, TRACE>::lds_bytes();
+        LaunchInfo li{family, dim3((uint32_t)(n_virtual >> WL)), dim3(1u << (WL - R_LOG)), (uint32_t)lds, hash};
+        VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        launch(ctx, li, k, args..., trace_slot(ctx));
+    }
+
+    // Wrap passes of S = 1 .. WL - 5 stages of the upper level, hybrid passes of
+    // S = 4 .. WL - 5 stages, and the merge, on tiles of 2^WL records.
+    template <bool TRACE, int CP, bool XC, int WL, int S = 1>
+    static void tile_pass(vo_ctx *ctx, Bufs<R> b, IMap map, const Pass &ps, int p_top, uint64_t n_virtual, bool txc)
+    {
+        constexpr int BW = 1 << (WL - R_LOG);
+        if constexpr (!WRAP || S > WL - 5) {
+            throw Error{VO_ERR_INVALID, "tile pass not built"};
         } else {
-            throw Error{VO_ERR_INVALID, "bad wrap stage count"};
+            static const char *const wraps[] = {"sort_wrap_s1", "sort_wrap_s2", "sort_wrap_s3",
+                                                "sort_wrap_s4", "sort_wrap_s5", "sort_wrap_s6",
+                                                "sort_wrap_s7", "sort_wrap_s8", "sort_wrap_s9"};
+            static const char *const hybrids[] = {"sort_hybrid_s4", "sort_hybrid_s5", "sort_hybrid_s6",
+                                                  "sort_hybrid_s7", "sort_hybrid_s8", "sort_hybrid_s9"};
+            if (ps.kind == 6) {
+                auto k = dev::k_sort_merge<R, WL, R_LOG, BW, TRACE, CP, XC>;
+                if (!XC && txc) k = dev::k_sort_merge<R, WL, R_LOG, BW, TRACE, CP, true>;
+                launch_tiles<TRACE, WL>(ctx, "sort_merge", n_virtual, hash_mix(ps.p, p_top), k, b, map, ps.p, p_top);
+                return;
+            }
+            if (ps.s != S) return tile_pass<TRACE, CP, XC, WL, S + 1>(ctx, b, map, ps, p_top, n_virtual, txc);
+            const uint64_t h = hash_mix(ps.p, ps.q_lo);
+            if (ps.kind == 5)
+                launch_tiles<TRACE, WL>(ctx, wraps[S - 1], n_virtual, hash_mix(h, hash_mix(S + 200, p_top)),
+                                        dev::k_sort_wrap<R, WL, R_LOG, BW, S, TRACE, CP, XC>, b, map, ps.p, ps.q_lo,
+                                        p_top);
+            if constexpr (S >= 4)
+                if (ps.kind == 7)
+                    launch_tiles<TRACE, WL>(ctx, hybrids[S - 4], n_virtual, hash_mix(h, hash_mix(S + 100, p_top)),
+                                            dev::k_sort_hybrid<R, WL, R_LOG, BW, S, TRACE, CP, XC>, b, map, ps.p,
+                                            ps.q_lo, p_top);
         }
     }
 
@@ -703,7 +741,7 @@ struct SortImpl {
     static void run_t(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill, IMap map, int p_top,
                       uint64_t n_virtual)
     {
-        for (const Pass &ps : plan(ctx, n_log)) {
+        for (const Pass &ps : plan(ctx, n_log, n_virtual)) {
             switch (ps.kind) {
             case 0: {
                 LaunchInfo li{"sort_tiny", dim3(1), dim3(64), 0, hash_mix(n_log, fill)};
@@ -740,7 +778,14 @@ struct SortImpl {
                 default: throw Error{VO_ERR_INVALID, "bad hybrid stage count"};
                 }
                 break;
-            case 5: launch_wrap<TRACE, CP, XC>(ctx, b, map, ps.p, ps.q_lo, ps.s, p_top, n_virtual); break;
+            case 5:
+            case 6:
+            case 7:
+                if (ps.w == T_LOG)
+                    tile_pass<TRACE, CP, XC, T_LOG>(ctx, b, map, ps, p_top, n_virtual, tiles_xc(n_log));
+                else
+                    tile_pass<TRACE, CP, XC, W_LOG>(ctx, b, map, ps, p_top, n_virtual, tiles_xc(n_log));
+                break;
             case 3: {
                 const size_t lds = dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes();
                 const uint32_t n_tiles = (uint32_t)(n_virtual >> T_LOG);
@@ -811,7 +856,7 @@ struct SortImpl {
         dispatch(ctx, b, c, 0, 1, IMap{offsets, c, ns}, c, count << c);
     }
 
-    static int passes(vo_ctx *ctx, int n_log) { return (int)plan(ctx, n_log).size(); }
+    static int passes(vo_ctx *ctx, int n_log) { return (int)plan(ctx, n_log, 1ull << n_log).size(); }
 };
 
 // Record kinds and their tile shapes (LDS = 2^T_LOG * 17/16 * record bytes).

@@ -18,13 +18,13 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // passes win (2^25: 5.06 vs 5.13 ms per sort, 2^23: 1.107 vs 1.128 ms).
 // Hybrid passes of 4-6 stages with 1024-thread blocks: at 2^28, 5494 -> 5611,
 // 5147 -> 5216 and 5319 -> 5483 GB/s (7 and 8 stages are faster at 512).
-using SortKP = SortImpl<RecKP, 13, 4, 512, 5, 8, 3, 27, 6, true, true>;
+using SortKP = SortImpl<RecKP, 13, 4, 512, 5, 8, 3, 27, 6, 14, true, true>;
 // The resident queue kernel runs 256-thread blocks: the 12-byte sort runs
 // there on 2^12-record tiles (the same network, so the same output).
-using SortKP_R = SortImpl<RecKP, 12, 4, 256, 5, 7, 3, 27, 0, false>;
+using SortKP_R = SortImpl<RecKP, 12, 4, 256, 5, 7, 3, 27, 0, 12, false>;
 // The same tiles with 1024-thread blocks of 8 records per thread (tuning
 // bit 0x200): the same passes at up to twice the waves per SIMD.
-using SortKP_W = SortImpl<RecKP, 13, 3, 1024, 5, 8, 3, 27, 0, false>;
+using SortKP_W = SortImpl<RecKP, 13, 3, 1024, 5, 8, 3, 27, 0, 13, false>;
 
 void run_kp(vo_ctx *ctx, Bufs<RecKP> b, int n_log, uint64_t n_valid, int fill)
 {

@@ -16,7 +16,7 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // 4.80-4.99 TB/s against 5.11-5.36 for its LDS-staged passes
 // (512-thread hybrid passes measured no faster for it: 78.04-78.05 vs 78.06-78.14 ms per
 // 2^28-row shuffle with permutation output)
-using SortKV = SortImpl<RecKV, 12, 4, 256, 5, 7, 3, 27>;
+using SortKV = SortImpl<RecKV, 12, 4, 256, 5, 7, 3, 27, 0, 13>;
 
 } // namespace
 

@@ -14,13 +14,12 @@ namespace {
 
 using namespace smulti_k;
 
-const std::pair<const void *, BodyInfo> kBodies[] = {VO_SORT_M12_BODIES(VO_BODY_ENTRY) VO_SORT_PACK_BODIES(VO_BODY_ENTRY)};
+const std::pair<const void *, BodyInfo> kBodies[] = {VO_SORT_M1_BODIES(VO_BODY_ENTRY) VO_SORT_PACK_BODIES(VO_BODY_ENTRY)};
 const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodies[0]), true);
 
 // 1- and 2-word keys: register passes of at most 3 stages, wider groups as
 // LDS-staged hybrid passes (ORDER BY of two keys at 2^24: 5.66 -> 5.39 ms)
-using SortM1 = SortImpl<RecM1, 12, 4, 256, 3, 7>;
-using SortM2 = SortImpl<RecM2, 12, 4, 256, 3, 7>;
+using SortM1 = SortImpl<RecM1, 12, 4, 256, 3, 7, 3, 64, 0, 13>;
 
 // ------------------------------------------------- multi-column (OP_SORT)
 
@@ -126,13 +125,7 @@ void op_sort_multi(vo_ctx *ctx, const vo_sort_args &a)
         SortM1::run(ctx, b, n_log, n_pad, 0);
         break;
     }
-    case 2: {
-        Bufs<RecM2> b;
-        for (int w = 0; w < 2; ++w) b.k[w] = wp[w];
-        b.p = idx;
-        SortM2::run(ctx, b, n_log, n_pad, 0);
-        break;
-    }
+    case 2: sort_words2(ctx, wp, idx, n_log); break;
     case 4: sort_words4(ctx, wp, idx, n_log); break;
     default: sort_words8(ctx, wp, idx, n_log); break;
     }

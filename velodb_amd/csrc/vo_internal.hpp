@@ -256,8 +256,9 @@ void queue_wait_seq_locked(vo_ctx *ctx, uint64_t seq); // caller holds ctx->mu
 // ---- shared device helpers (sort.hip) used by other ops
 // Sort (u64 key, u64 value) records by (key, value) ascending, n_pad = 2^k.
 void sort_kv(vo_ctx *ctx, uint64_t *keys, uint64_t *vals, uint64_t n_pad);
-// Sort rows of four or eight key words and a u32 payload by the words (ties not
-// broken), 2^n_log rows, all live (sort_multi48.hip).
+// Sort rows of two, four or eight key words and a u32 payload by the words (ties
+// not broken), 2^n_log rows, all live (sort_multi2.hip, sort_multi48.hip).
+void sort_words2(vo_ctx *ctx, uint64_t *const *words, uint32_t *payload, int n_log);
 void sort_words4(vo_ctx *ctx, uint64_t *const *words, uint32_t *payload, int n_log);
 void sort_words8(vo_ctx *ctx, uint64_t *const *words, uint32_t *payload, int n_log);
 // Sort (u64 key, u32 payload) without padding (all n_pad rows are live).
