@@ -584,6 +584,13 @@ struct SortImpl {
     // The default tuning runs the wrapped schedule; a tuning word that picks
     // pass widths or block shapes, and recorded programs (whose bodies they
     // are), run level by level.
+    static bool wrapped(vo_ctx *ctx)
+    {
+        const SortTuning &t = ctx->tuning, d;
+        return WRAP && !ctx->rec && t.max_fused_stages == d.max_fused_stages &&
+               t.max_hybrid_stages == d.max_hybrid_stages && !t.pipe_merge && !t.wide_block && !t.flip_hybrid_block;
+    }
+
     // Wide tiles take one more stage bit per pass (28 passes instead of 31 for
     // 2^28 12-byte records, 32 instead of 37 for 16-byte ones) with twice the
     // threads behind each barrier.  They are used from 512 tiles, two a CU:
@@ -593,11 +600,7 @@ struct SortImpl {
     // 2^22 758 -> 749 us, 2^24 3.90 -> 3.59 ms, 2^26 18.1 -> 16.0.
     static std::vector<Pass> plan(vo_ctx *ctx, int n_log, uint64_t n_virtual)
     {
-        const SortTuning &t = ctx->tuning, d;
-        const bool wrapped = WRAP && !ctx->rec && t.max_fused_stages == d.max_fused_stages &&
-                             t.max_hybrid_stages == d.max_hybrid_stages && !t.pipe_merge && !t.wide_block &&
-                             !t.flip_hybrid_block;
-        if (!wrapped) return plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx));
+        if (!wrapped(ctx)) return plan_passes(n_log, T_LOG, smax(ctx, n_log), R_LOG, hmax(ctx));
         static const auto make = [](int w) {
             std::vector<std::vector<Pass>> v;
             for (int l = 0; (1ull << l) <= kMaxSortRows; ++l)
@@ -644,18 +647,20 @@ struct SortImpl {
     }
 
     // Arrays of one tile smaller than 2^T_LOG (t = 8 .. T_LOG - 1), of at most
-    // two key words: the
-    // compile-time tile sort at their own size, on at most 16 records a thread
-    // and at least one whole wavefront.  (The run-time form below kept its LDS
-    // addresses in registers and a barrier around every relayout: one array of
-    // 4096 12-byte records, call and wait included: 61 -> 40 us.)
+    // two key words: the compile-time tile sort at their own size, on at least
+    // one whole wavefront.  (The run-time form below keeps its LDS addresses in
+    // registers and a barrier around every relayout: one array of 4096 12-byte
+    // records, call and wait included, 61 -> 40 us.)
     template <bool TRACE, int T = 8>
     static bool launch_small(vo_ctx *ctx, Bufs<R> b, IMap map, int t, int p_top, uint64_t n_valid, int fill,
                              uint64_t n_virtual)
     {
         if constexpr (WRAP && T < T_LOG && R::KW <= 2) {
             if (t != T) return launch_small<TRACE, T + 1>(ctx, b, map, t, p_top, n_valid, fill, n_virtual);
-            constexpr int RL = T - 6 < R_LOG ? T - 6 : R_LOG;
+            // few records a thread: a lone tile's time is its waves' latency
+            // (2^12 records on 256, 512 and 1024 threads: 29.0, 23.4, 28.3 us;
+            // 2^10 on 64, 128 and 256: 18.3, 11.4, 9.6)
+            constexpr int RL = std::min(R_LOG, T >= 12 ? 3 : 2);
             const size_t lds = dev::TileCT<R, T, RL, TRACE>::lds_bytes();
             LaunchInfo li{"sort_local", dim3((uint32_t)(n_virtual >> T)), dim3(1u << (T - RL)), (uint32_t)lds,
                           hash_mix(hash_mix(T, p_top), fill)};

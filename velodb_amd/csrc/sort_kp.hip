@@ -19,6 +19,13 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // Hybrid passes of 4-6 stages with 1024-thread blocks: at 2^28, 5494 -> 5611,
 // 5147 -> 5216 and 5319 -> 5483 GB/s (7 and 8 stages are faster at 512).
 using SortKP = SortImpl<RecKP, 13, 4, 512, 5, 8, 3, 27, 6, 14, true, true>;
+// Up to 2^20 records a sort has at most 128 tiles of 2^13 and its passes are one
+// tile's latency on half of the CUs.  Tiles of 2^12 on 512 threads, 8 records
+// each, give every CU one: local pass at 2^20 48 -> 26 us, merge and wrap passes
+// 11 -> 7.5 us for 15 passes instead of 12.  Whole sorts: 2^13 47 -> 34 us, 2^16
+// 86 -> 59, 2^18 116 -> 83, 2^20 177 -> 146; at 2^21 both take 214.
+using SortKP_S = SortImpl<RecKP, 12, 3, 512, 5, 7, 3, 27, 0, 12>;
+constexpr int kSmallLog = 20;
 // The resident queue kernel runs 256-thread blocks: the 12-byte sort runs
 // there on 2^12-record tiles (the same network, so the same output).
 using SortKP_R = SortImpl<RecKP, 12, 4, 256, 5, 7, 3, 27, 0, 12, false>;
@@ -26,12 +33,19 @@ using SortKP_R = SortImpl<RecKP, 12, 4, 256, 5, 7, 3, 27, 0, 12, false>;
 // bit 0x200): the same passes at up to twice the waves per SIMD.
 using SortKP_W = SortImpl<RecKP, 13, 3, 1024, 5, 8, 3, 27, 0, 13, false>;
 
+bool small_sort(vo_ctx *ctx, int n_log)
+{
+    return n_log <= kSmallLog && !ctx->rec && !ctx->tuning.wide_block && SortKP_S::wrapped(ctx);
+}
+
 void run_kp(vo_ctx *ctx, Bufs<RecKP> b, int n_log, uint64_t n_valid, int fill)
 {
     if (ctx->rec)
         SortKP_R::run(ctx, b, n_log, n_valid, fill);
     else if (ctx->tuning.wide_block)
         SortKP_W::run(ctx, b, n_log, n_valid, fill);
+    else if (small_sort(ctx, n_log))
+        SortKP_S::run(ctx, b, n_log, n_valid, fill);
     else
         SortKP::run(ctx, b, n_log, n_valid, fill);
 }
@@ -56,7 +70,11 @@ void sort_kp_full(vo_ctx *ctx, uint64_t *keys, uint32_t *payload, uint64_t n_pad
     run_kp(ctx, b, ilog2(n_pad), n_pad, 0);
 }
 
-int sort_plan_passes(vo_ctx *ctx, uint64_t n_pad) { return SortKP::passes(ctx, ilog2(n_pad)); }
+int sort_plan_passes(vo_ctx *ctx, uint64_t n_pad)
+{
+    const int n_log = ilog2(n_pad);
+    return small_sort(ctx, n_log) ? SortKP_S::passes(ctx, n_log) : SortKP::passes(ctx, n_log);
+}
 
 // ------------------------------------------------------------ batched sorts
 

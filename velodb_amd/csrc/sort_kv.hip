@@ -17,6 +17,9 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // (512-thread hybrid passes measured no faster for it: 78.04-78.05 vs 78.06-78.14 ms per
 // 2^28-row shuffle with permutation output)
 using SortKV = SortImpl<RecKV, 12, 4, 256, 5, 7, 3, 27, 0, 13>;
+// Up to 2^20 records, one tile or fewer a CU: 512 threads of 8 records each (as
+// in sort_kp.hip); a shuffle of 2^20 rows with its permutation 222 -> 203 us.
+using SortKV_S = SortImpl<RecKV, 12, 3, 512, 5, 7, 3, 27, 0, 12>;
 
 } // namespace
 
@@ -25,7 +28,11 @@ void sort_kv(vo_ctx *ctx, uint64_t *keys, uint64_t *vals, uint64_t n_pad)
     Bufs<RecKV> b;
     b.k[0] = keys;
     b.p = vals;
-    SortKV::run(ctx, b, ilog2(n_pad), n_pad, 0);
+    const int n_log = ilog2(n_pad);
+    if (n_log <= 20 && SortKV_S::wrapped(ctx))
+        SortKV_S::run(ctx, b, n_log, n_pad, 0);
+    else
+        SortKV::run(ctx, b, n_log, n_pad, 0);
 }
 
 } // namespace vo

@@ -20,6 +20,9 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // 1- and 2-word keys: register passes of at most 3 stages, wider groups as
 // LDS-staged hybrid passes (ORDER BY of two keys at 2^24: 5.66 -> 5.39 ms)
 using SortM1 = SortImpl<RecM1, 12, 4, 256, 3, 7, 3, 64, 0, 13>;
+// up to 2^20 rows, one tile or fewer a CU: 512 threads of 8 rows (sort_kp.hip);
+// OP_SORT of 2^20 rows 194 -> 173 us
+using SortM1_S = SortImpl<RecM1, 12, 3, 512, 3, 7, 3, 64, 0, 12>;
 
 // ------------------------------------------------- multi-column (OP_SORT)
 
@@ -122,7 +125,10 @@ void op_sort_multi(vo_ctx *ctx, const vo_sort_args &a)
         Bufs<RecM1> b;
         b.k[0] = wp[0];
         b.p = idx;
-        SortM1::run(ctx, b, n_log, n_pad, 0);
+        if (n_log <= 20 && SortM1_S::wrapped(ctx))
+            SortM1_S::run(ctx, b, n_log, n_pad, 0);
+        else
+            SortM1::run(ctx, b, n_log, n_pad, 0);
         break;
     }
     case 2: sort_words2(ctx, wp, idx, n_log); break;
