@@ -24,7 +24,7 @@ HBM_PEAK_GBS = 8000.0
 # launch families of the sort passes: local, merge, register passes of 1-5
 # stages, LDS-staged passes of 4-8 stages
 SORT_FAMS = (["sort_local", "sort_merge"] + [f"sort_global_s{s}" for s in range(1, 6)] +
-             [f"sort_hybrid_s{s}" for s in range(4, 9)] + [f"sort_wrap_s{s}" for s in range(1, 9)])
+             [f"sort_hybrid_s{s}" for s in range(4, 10)] + [f"sort_wrap_s{s}" for s in range(1, 10)])
 METRIC = "oblivious sort Mrec/s at 2^28 (%HBM peak); served QPS + p50/p99 vs plain"
 REC_BYTES = 12  # u64 key + u32 payload, structure of arrays
 

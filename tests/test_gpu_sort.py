@@ -415,3 +415,32 @@ def test_sort_wide_tiles(vctx, log2n, short):
     o = o[torch.sort(first[:n][o], descending=True, stable=True).indices]
     assert torch.equal(c[:n], first[:n][o]) and torch.equal(k[:n], k0[:n][o])
     assert torch.equal(torch.sort(idx[:n]).values, torch.arange(n, device="cuda:0"))
+
+
+@pytest.mark.parametrize("log2n,short", [(13, 0), (13, 4095), (20, 0), (20, 3)])
+def test_sort_one_tile_per_cu(vctx, log2n, short):
+    """The smallest and largest sizes of more than one tile that take the tiles
+    of eight records a thread: the 12-byte and 16-byte records, and OP_SORT's
+    ties of one and two key words against the oracle."""
+    npad, n = 1 << log2n, (1 << log2n) - short
+    print(f"one tile per CU n={n} npad={npad}", flush=True)
+    rng = np.random.default_rng(log2n + short)
+    k = rng.integers(0, 1 << 62, n).astype(np.uint64) >> np.uint64(50)
+    p = rng.integers(0, 3, n).astype(np.uint32)
+    gk, gp = _run_sort(vctx, k, p, n, npad)
+    order = np.lexsort((p, k))
+    assert np.array_equal(gk[:n], k[order]) and np.array_equal(gp[:n], p[order])
+    assert np.array_equal(gk[n:], np.full(npad - n, M64)) and np.array_equal(gp[n:], np.arange(n, npad, dtype=np.uint32))
+    a, b, perm = (to_dev(np.arange(npad, dtype=np.uint32)) for _ in range(3))
+    vctx.shuffle(a, npad, 7, perm_out=perm, n=n)
+    vctx.shuffle(b, npad, 7, n=n)
+    assert np.array_equal(from_dev(a, np.uint32), from_dev(perm, np.uint32))
+    assert np.array_equal(from_dev(a, np.uint32), from_dev(b, np.uint32))
+    for types, asc in (([5], [False]), ([4, 5], [True, False])):
+        cols = [_rand_col(rng, t, npad, 3) for t in types]
+        ecols, eidx = oracle.bitonic_sort_multi(cols, types, asc, n, npad)
+        dcols, didx = [to_dev(c) for c in cols], empty_dev(npad, np.int64)
+        vctx.sort(dcols, types, asc, didx, n, npad)
+        assert np.array_equal(from_dev(didx, np.int64), eidx)
+        for dc, ec, t in zip(dcols, ecols, types):
+            assert np.array_equal(from_dev(dc, TYPES[t]).view(np.uint8), ec.view(np.uint8))
