@@ -80,7 +80,7 @@ void op_gather_oblivious(vo_ctx *ctx, const vo_gather_oblivious_args &a)
            (const uint64_t *)keys, (const void *)vals, tiles, trace_slot(ctx));
     launch(ctx, LaunchInfo{"gather_obl_carry", dim3(1), dim3(kScanThreads), 0, nt},
            tr ? k_og_carry<true> : k_og_carry<false>, (const Last *)tiles, nt, carry, trace_slot(ctx));
-    launch(ctx, LaunchInfo{"gather_obl_rows", dim3(nt), dim3(GB), 0, n_pad},
+    launch(ctx, LaunchInfo{"gather_obl_rows", dim3(nt), dim3(GB), dev::kRowsLds, n_pad},
            pick(k_og_rows<false, false>, k_og_rows<true, false>, k_og_rows<false, true>, k_og_rows<true, true>),
            (const uint64_t *)keys, (const void *)vals, (const Last *)carry, c0, c1, mask, trace_slot(ctx));
     compact_rows2(ctx, c0, c1, mask, n_pad, cnt);

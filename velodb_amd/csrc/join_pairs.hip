@@ -384,7 +384,7 @@ uint64_t op_join_pairs_count(vo_ctx *ctx, const vo_join_pairs_args &a)
            (const uint64_t *)keys, (const void *)vals, n_pad, (const Min2 *)bc, aux, ft, trace_slot(ctx));
     launch(ctx, LaunchInfo{"join_pairs_fwd_carry", dim3(1), dim3(kScanThreads), 0, nt},
            tr ? k_jp_fwd_carry<true> : k_jp_fwd_carry<false>, (const Fwd *)ft, nt, fc, trace_slot(ctx));
-    launch(ctx, LaunchInfo{"join_pairs_fwd_rows", dim3(nt), dim3(PB), 0, n_pad},
+    launch(ctx, LaunchInfo{"join_pairs_fwd_rows", dim3(nt), dim3(PB), dev::kRowsLds, n_pad},
            pick(k_jp_fwd_rows<false, false>, k_jp_fwd_rows<true, false>, k_jp_fwd_rows<false, true>,
                 k_jp_fwd_rows<true, true>),
            (const uint64_t *)keys, (const void *)vals, (const uint32_t *)aux, n_pad, (const Fwd *)fc, sp.cl, ml,

@@ -180,7 +180,7 @@
     X(kB_jp_bwd_tiles_##TAG, (jp_k::k_jp_bwd_tiles<false, KP>), (jp_k::b_jp_bwd_tiles<false, KP>(a..., vb, nvb)),  \
       0)                                                                                                           \
     X(kB_jp_bwd_rows_##TAG, (jp_k::k_jp_bwd_rows<false, KP>), (jp_k::b_jp_bwd_rows<false, KP>(a..., vb, nvb)), 0)  \
-    X(kB_jp_fwd_rows_##TAG, (jp_k::k_jp_fwd_rows<false, KP>), (jp_k::b_jp_fwd_rows<false, KP>(a..., vb, nvb)), 0)
+    X(kB_jp_fwd_rows_##TAG, (jp_k::k_jp_fwd_rows<false, KP>), (jp_k::b_jp_fwd_rows<false, KP>(a..., lds, vb, nvb)), 0)
 
 #define VO_JP_BODIES(X)                                                                                            \
     X(kB_jp_build, (jp_k::k_jp_build<false>), (jp_k::b_jp_build<false>(a..., vb, nvb)), 0)                         \
@@ -201,7 +201,7 @@
 #define VO_OG_KP(X, KP, TAG)                                                                                       \
     X(kB_og_build_##TAG, (og_k::k_og_build<false, KP>), (og_k::b_og_build<false, KP>(a..., vb, nvb)), 0)           \
     X(kB_og_tiles_##TAG, (og_k::k_og_tiles<false, KP>), (og_k::b_og_tiles<false, KP>(a..., vb, nvb)), 0)           \
-    X(kB_og_rows_##TAG, (og_k::k_og_rows<false, KP>), (og_k::b_og_rows<false, KP>(a..., vb, nvb)), 0)
+    X(kB_og_rows_##TAG, (og_k::k_og_rows<false, KP>), (og_k::b_og_rows<false, KP>(a..., lds, vb, nvb)), 0)
 
 #define VO_OG_BODIES(X)                                                                                            \
     VO_OG_KP(X, true, kp) VO_OG_KP(X, false, kv)                                                                   \

@@ -712,5 +712,23 @@ struct TileCT {
     }
 };
 
+// A column of a 2^12-row tile on 256 threads between layout 6 (64 lanes on
+// consecutive rows: what memory likes) and layout 0 (16 consecutive rows a
+// thread: what a scan over rows likes), inside the wavefronts.  lds:
+// kRowsLds bytes; a barrier stands between its last use by other waves and the
+// first call.
+using Rows12 = TileCT<Rec<1, uint64_t, true>, 12, 4, false>;
+constexpr uint32_t kRowsLds = Rows12::TPAD * 8;
+
+template <int A_FROM, int A_TO>
+__device__ __forceinline__ void wave_rows(uint64_t (&v)[16], char *lds, uint32_t tau)
+{
+    static_assert(Rows12::in_wave(A_FROM, A_TO), "layouts inside the wavefront");
+    uint64_t h = 0;
+    uint32_t n = 0;
+    Rows12::wave_fence();
+    Rows12::move_col<A_FROM, A_TO>(v, reinterpret_cast<uint64_t *>(lds), tau, h, n);
+}
+
 } // namespace dev
 } // namespace vo
