@@ -388,8 +388,7 @@ def bench_join_pairs(args):
     fams = ["join_pairs_build"] + SORT_FAMS + ["join_pairs_bwd_tiles",
             "join_pairs_bwd_carry", "join_pairs_bwd_rows", "join_pairs_fwd_carry", "join_pairs_fwd_rows",
             "compact_count", "compact_scan", "compact_local", "compact_hybrid", "compact_global",
-            "join_pairs_dist_init_w1", "join_pairs_dist_init_w2", "join_pairs_dist_level_w1",
-            "join_pairs_dist_level_w2", "join_pairs_dist_tile_w1", "join_pairs_dist_tile_w2",
+            "join_pairs_dist_level_w1", "join_pairs_dist_level_w2", "join_pairs_dist_tile_w1", "join_pairs_dist_tile_w2",
             "join_pairs_fill_carry", "join_pairs_fill_left", "join_pairs_fill_right", "join_pairs_out"]
     stats = _family_stats(ctx, fams)
     # algorithmic bytes per padded row and launch: a distribution pass (three

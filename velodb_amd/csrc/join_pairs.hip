@@ -167,41 +167,31 @@ void distribute(vo_ctx *ctx, const uint64_t *s0, const uint64_t *s1, uint64_t sr
                 Elem<NW> *tc, uint64_t **res0, uint64_t **res1)
 {
     const bool tr = ctx->tracing;
-    launch(ctx, LaunchInfo{NW == 1 ? "join_pairs_dist_init_w1" : "join_pairs_dist_init_w2", grid_for(m_pad), dim3(256),
-                           0, hash_mix(NW, m_pad)},
-           tr ? k_jp_dist_init<NW, true> : k_jp_dist_init<NW, false>, s0, s1, src_rows, kdev, m_pad, a0, a1,
-           trace_slot(ctx));
-    uint64_t *c0 = a0, *c1 = a1, *n0 = b0, *n1 = b1;
-    // levels m_pad/2 .. 256, up to kDistFuse per pass, as even as possible
+    // levels m_pad/2 .. 256 (at least one: m_pad >= TS), up to kDistFuse per
+    // pass, as even as possible; the first pass reads the compacted rows
+    const uint64_t *c0 = s0, *c1 = s1;
+    uint64_t *n0 = a0, *n1 = a1, *x0 = b0, *x1 = b1;
     const int count = ilog2(m_pad / 2) - ilog2(DH) + 1;
     const int groups = (count + kDistFuse - 1) / kDistFuse;
     uint64_t j = m_pad / 2;
     for (int gi = 0; gi < groups; ++gi) {
         const int sl = count / groups + (gi < count % groups ? 1 : 0);
-        LaunchInfo li{NW == 1 ? "join_pairs_dist_level_w1" : "join_pairs_dist_level_w2", grid_for(m_pad), dim3(256), 0,
-                      hash_mix(hash_mix(NW, m_pad), hash_mix(j, sl))};
-        auto go = [&](auto k) {
-            launch(ctx, li, k, (const uint64_t *)c0, (const uint64_t *)c1, m_pad, j, n0, n1, trace_slot(ctx));
-        };
-        if (sl <= 3) {
-            // lattice form: u = smallest stride of the group (>= DH = 256),
-            // rows = m_pad / u >= 2^sl, K = min(kLatticeRows, rows)
-            const uint64_t u = j >> (sl - 1);
-            const uint64_t rows = m_pad / u;
-            const int K = (int)std::min<uint64_t>(kLatticeRows<NW>, rows);
-            LaunchInfo ll = li;
-            ll.grid = dim3((uint32_t)(m_pad / (256ull * (uint64_t)K)));
-            ll.block = dim3(256);
-            auto lat = [&](auto k) {
-                launch(ctx, ll, k, (const uint64_t *)c0, (const uint64_t *)c1, u, n0, n1, trace_slot(ctx));
-            };
-            dist_lattice_launch<NW>(sl, K, tr, lat);
-        } else {
-            go(tr ? k_jp_dist_levels<NW, 4, true> : k_jp_dist_levels<NW, 4, false>);
-        }
+        // lattice form: u = smallest stride of the group (>= DH = 256),
+        // rows = m_pad / u >= 2^sl, K = min(kLatticeRows, rows)
+        const uint64_t u = j >> (sl - 1);
+        const int K = (int)std::min<uint64_t>(kLatticeRows<NW>, m_pad / u);
+        const LaunchInfo li{NW == 1 ? "join_pairs_dist_level_w1" : "join_pairs_dist_level_w2",
+                            dim3((uint32_t)(m_pad / (256ull * (uint64_t)K))), dim3(256), 0,
+                            hash_mix(hash_mix(NW, m_pad), hash_mix(j, sl))};
+        dist_lattice_launch<NW>(sl, K, tr, [&](auto k) {
+            launch(ctx, li, k, c0, c1, gi ? m_pad : src_rows, gi ? (const uint64_t *)nullptr : kdev, u, n0, n1,
+                   trace_slot(ctx));
+        });
         j >>= sl;
-        std::swap(c0, n0);
-        std::swap(c1, n1);
+        c0 = n0;
+        c1 = n1;
+        std::swap(n0, x0);
+        std::swap(n1, x1);
     }
     const uint32_t nt = (uint32_t)(m_pad / TS);
     const size_t lds = (size_t)2 * NW * (TS + DH) * 8;
@@ -209,8 +199,7 @@ void distribute(vo_ctx *ctx, const uint64_t *s0, const uint64_t *s1, uint64_t sr
     VO_HIP(hipFuncSetAttribute((const void *)kt, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     launch(ctx, LaunchInfo{NW == 1 ? "join_pairs_dist_tile_w1" : "join_pairs_dist_tile_w2", dim3(nt), dim3(PB),
                            (uint32_t)lds, hash_mix(NW, m_pad)},
-           kt,
-           (const uint64_t *)c0, (const uint64_t *)c1, n0, n1, tl, trace_slot(ctx));
+           kt, c0, c1, n0, n1, tl, trace_slot(ctx));
     launch(ctx, LaunchInfo{"join_pairs_fill_carry", dim3(1), dim3(kScanThreads), 0, hash_mix(NW, nt)},
            tr ? k_jp_fill_carry<NW, true> : k_jp_fill_carry<NW, false>, (const Elem<NW> *)tl, nt, tc,
            trace_slot(ctx));

@@ -595,46 +595,8 @@ __global__ __launch_bounds__(PB) void k_jp_fwd_rows(const uint64_t *__restrict__
 
 __device__ __forceinline__ uint32_t tgt(uint64_t w0) { return (uint32_t)(w0 >> 32); }
 
-// Copy of the compacted rows into the first slots; slots >= k are empty.
-template <int NW, bool TRACE>
-__device__ __forceinline__ void b_jp_dist_init(const uint64_t *__restrict__ s0, const uint64_t *__restrict__ s1, uint64_t src_rows,
-                               const uint64_t *__restrict__ kdev, uint64_t m_pad, uint64_t *__restrict__ d0,
-                               uint64_t *__restrict__ d1, TraceSlot *slot, uint32_t vb, uint32_t nvb)
-{
-    dev::AtrT<TRACE> tr(slot);
-    const uint64_t kk = kdev[0];
-    for (uint64_t i = (uint64_t)vb * 256 + threadIdx.x; i < m_pad; i += (uint64_t)nvb * 256) {
-        uint64_t a = EMPTY, b = EMPTY;
-        if (i < src_rows) { // public
-            a = s0[i];
-            if constexpr (NW == 2) b = s1[i];
-            tr.at(1, i);
-        }
-        const bool valid = i < kk;
-        d0[i] = valid ? a : EMPTY;
-        if constexpr (NW == 2) d1[i] = valid ? b : EMPTY;
-        tr.at(2, i);
-    }
-    tr.done(dev::gtid());
-}
-
-template <int NW, bool TRACE>
-__global__ void k_jp_dist_init(const uint64_t *__restrict__ s0, const uint64_t *__restrict__ s1, uint64_t src_rows,
-                               const uint64_t *__restrict__ kdev, uint64_t m_pad, uint64_t *__restrict__ d0,
-                               uint64_t *__restrict__ d1, TraceSlot *slot)
-{
-    b_jp_dist_init<NW, TRACE>(s0, s1, src_rows, kdev, m_pad, d0, d1, slot, blockIdx.x, gridDim.x);
-}
-
-// S levels j_top, j_top/2, .., j_top/2^(S-1) in one pass: the value of slot
-// p after them depends only on the 2^S slots p - m * (j_top >> (S-1)),
-// m < 2^S, so each output reads those (the neighbours' reads are the same
-// rows and come from the caches) and applies the levels in order.
-#ifndef VO_DIST_FUSE
-#define VO_DIST_FUSE 3
-#endif
-constexpr int kDistFuse = VO_DIST_FUSE;
-static_assert(kDistFuse >= 1 && kDistFuse <= 4, "1 to 4 distribution levels per pass");
+// At most three levels share a pass: two measured the same, four slower.
+constexpr int kDistFuse = 3;
 
 template <int NW>
 __device__ __forceinline__ Elem<NW> dist_step(const Elem<NW> &cur, const Elem<NW> &prv, int64_t p, uint64_t j)
@@ -647,64 +609,27 @@ __device__ __forceinline__ Elem<NW> dist_step(const Elem<NW> &cur, const Elem<NW
     return r;
 }
 
-template <int S, int NW, class Tr>
-__device__ __forceinline__ Elem<NW> dist_val(const uint64_t *__restrict__ i0, const uint64_t *__restrict__ i1,
-                                             int64_t p, uint64_t j_top, Tr &tr)
-{
-    if constexpr (S == 0) {
-        Elem<NW> e;
-        e.w[0] = EMPTY;
-        if constexpr (NW == 2) e.w[1] = EMPTY;
-        if (p >= 0) { // public: the position only
-            e.w[0] = i0[p];
-            if constexpr (NW == 2) e.w[1] = i1[p];
-            tr.at(1, (uint64_t)p);
-        }
-        return e;
-    } else {
-        const uint64_t j = j_top >> (S - 1);
-        const Elem<NW> a = dist_val<S - 1, NW>(i0, i1, p, j_top, tr);
-        const Elem<NW> b = dist_val<S - 1, NW>(i0, i1, p - (int64_t)j, j_top, tr);
-        return dist_step<NW>(a, b, p, j);
-    }
-}
-
-template <int NW, int S, bool TRACE>
-__device__ __forceinline__ void b_jp_dist_levels(const uint64_t *__restrict__ i0, const uint64_t *__restrict__ i1, uint64_t m_pad,
-                                 uint64_t j_top, uint64_t *__restrict__ o0, uint64_t *__restrict__ o1,
-                                 TraceSlot *slot, uint32_t vb, uint32_t nvb)
-{
-    dev::AtrT<TRACE> tr(slot);
-    for (uint64_t p = (uint64_t)vb * 256 + threadIdx.x; p < m_pad; p += (uint64_t)nvb * 256) {
-        const Elem<NW> e = dist_val<S, NW>(i0, i1, (int64_t)p, j_top, tr);
-        o0[p] = e.w[0];
-        if constexpr (NW == 2) o1[p] = e.w[1];
-        tr.at(2, p);
-    }
-    tr.done(dev::gtid());
-}
-
-template <int NW, int S, bool TRACE>
-__global__ void k_jp_dist_levels(const uint64_t *__restrict__ i0, const uint64_t *__restrict__ i1, uint64_t m_pad,
-                                 uint64_t j_top, uint64_t *__restrict__ o0, uint64_t *__restrict__ o1,
-                                 TraceSlot *slot)
-{
-    b_jp_dist_levels<NW, S, TRACE>(i0, i1, m_pad, j_top, o0, o1, slot, blockIdx.x, gridDim.x);
-}
-
-// The same levels on the lattice of the smallest stride u = j_top >> (S-1):
-// slot p = q + k u with residue q < u and row k.  Output row k reads rows
+// S levels j_top, j_top/2, .., j_top/2^(S-1) in one pass, on the lattice of the
+// smallest stride u = j_top >> (S-1): slot p = q + k u with residue q < u and row k.  Output row k reads rows
 // k, k-1, .., k-(2^S-1) of the same residue only, so a block takes 256
 // consecutive residues and K rows plus the 2^S - 1 rows before them into
 // registers and runs the S levels there, largest stride first (each slot
 // read (K + 2^S - 1) / K times instead of 2^S).  A level with lattice
 // stride s updates rows from the top down, so row r - s still holds the
 // previous level; rows below the running sum of strides hold partial values
-// that no output row reads.  Rows k < 0 (p < 0) are empty, as in dist_val.
+// that no output row reads.  Rows k < 0 (p < 0) are empty.
 // Needs u >= 256 and K <= m_pad / u.
+//
+// The first pass takes the compacted rows themselves: i0, i1 then hold src_rows
+// rows of which the first *kdev are elements, and every slot after those is
+// empty.  (A copy into the slots before it moved every slot once more: 46 us of
+// two-word and 24 us of one-word slots at 2^23; the join into pairs there
+// 2.55 -> 2.51 ms.)  The others read m_pad slots
+// and have no kdev.
 template <int NW, int S, int K, bool TRACE>
 __device__ __forceinline__ void b_jp_dist_lattice(const uint64_t *__restrict__ i0,
-                                                         const uint64_t *__restrict__ i1, uint64_t u,
+                                                         const uint64_t *__restrict__ i1, uint64_t src_rows,
+                                                         const uint64_t *__restrict__ kdev, uint64_t u,
                                                          uint64_t *__restrict__ o0, uint64_t *__restrict__ o1,
                                                          TraceSlot *slot, uint32_t vb, uint32_t nvb)
 {
@@ -714,17 +639,25 @@ __device__ __forceinline__ void b_jp_dist_lattice(const uint64_t *__restrict__ i
     const uint64_t res_blocks = u / 256;
     const uint64_t q = (vb % res_blocks) * 256 + threadIdx.x;
     const int64_t k0 = (int64_t)(vb / res_blocks) * K - H;
+    const uint64_t live = kdev ? kdev[0] : src_rows;
     Elem<NW> v[W];
 #pragma unroll
     for (int r = 0; r < W; ++r) {
         const int64_t k = k0 + r;
 #pragma unroll
         for (int w = 0; w < NW; ++w) v[r].w[w] = EMPTY;
-        if (k >= 0) { // public: the row only
-            const uint64_t pp = q + (uint64_t)k * u;
+        const uint64_t pp = q + (uint64_t)k * u;
+        if (k >= 0 && pp < src_rows) { // public: the row only
             v[r].w[0] = i0[pp];
             if constexpr (NW == 2) v[r].w[1] = i1[pp];
             tr.at(1, pp);
+        }
+    }
+    if (kdev) { // uniform
+#pragma unroll
+        for (int r = 0; r < W; ++r) {
+            const bool in = (int64_t)q + (k0 + r) * (int64_t)u < (int64_t)live;
+            v[r].w[0] = in ? v[r].w[0] : EMPTY;
         }
     }
 #pragma unroll
@@ -750,11 +683,12 @@ __device__ __forceinline__ void b_jp_dist_lattice(const uint64_t *__restrict__ i
 
 template <int NW, int S, int K, bool TRACE>
 __global__ __launch_bounds__(256) void k_jp_dist_lattice(const uint64_t *__restrict__ i0,
-                                                         const uint64_t *__restrict__ i1, uint64_t u,
+                                                         const uint64_t *__restrict__ i1, uint64_t src_rows,
+                                                         const uint64_t *__restrict__ kdev, uint64_t u,
                                                          uint64_t *__restrict__ o0, uint64_t *__restrict__ o1,
                                                          TraceSlot *slot)
 {
-    b_jp_dist_lattice<NW, S, K, TRACE>(i0, i1, u, o0, o1, slot, blockIdx.x, gridDim.x);
+    b_jp_dist_lattice<NW, S, K, TRACE>(i0, i1, src_rows, kdev, u, o0, o1, slot, blockIdx.x, gridDim.x);
 }
 
 // Levels 128 .. 1 of one TS-slot tile in LDS (window of the 256 slots

@@ -166,9 +166,6 @@
     X(kB_jp_lat##NW##_##S##_##K, (jp_k::k_jp_dist_lattice<NW, S, K, false>),                                       \
       (jp_k::b_jp_dist_lattice<NW, S, K, false>(a..., vb, nvb)), 0)
 #define VO_JP_NW(X, NW)                                                                                            \
-    X(kB_jp_dist_init##NW, (jp_k::k_jp_dist_init<NW, false>), (jp_k::b_jp_dist_init<NW, false>(a..., vb, nvb)), 0) \
-    X(kB_jp_dist_levels##NW, (jp_k::k_jp_dist_levels<NW, 4, false>),                                              \
-      (jp_k::b_jp_dist_levels<NW, 4, false>(a..., vb, nvb)), 0)                                                    \
     X(kB_jp_dist_tile##NW, (jp_k::k_jp_dist_tile<NW, 1024, false>),                                                \
       (jp_k::b_jp_dist_tile<NW, 1024, false>(a..., (uint64_t *)lds, vb)), 0)                                       \
     X(kB_jp_fill_carry##NW, (jp_k::k_jp_fill_carry<NW, false>),                                                    \
