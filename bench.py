@@ -690,18 +690,15 @@ def bench_batch(args):
     tp = run(per_instance, max(1, min(args.steps, 3)))
     same = bool(torch.equal(kb, keys) and torch.equal(pb, pay))
     # roofline over every sort pass of one batched call: each instance of
-    # padded size p moves 24 B x p per pass, and a class runs the pass plan of
-    # its size, so the call's algorithmic bytes are sum(24 p passes(p)).  The
+    # padded size p moves 24 B x p per pass, and its class runs as many passes
+    # as the class alone launches (counted below: a class's tiles follow its
+    # total rows, not the plan of one instance), so the call's algorithmic
+    # bytes are sum(24 p passes(p)).  The
     # size classes run on several streams forked from the context stream and
     # joined back into it, so the call is timed by HIP events on that stream
     # around the whole call; per-launch events (a second context) would add up
     # overlapping kernels.
     from velodb_amd import _abi
-    plan = {}
-    for _, _, p in items:
-        if p not in plan:
-            plan[p] = ctx.sort_plan(p)
-    alg = sum(2 * 12 * p * plan[p] for _, _, p in items)
     ctx.gen_sort_input(7, keys, pay, total)
     torch.cuda.synchronize()
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -719,13 +716,20 @@ def bench_batch(args):
     fams = ["sort_tiny"] + SORT_FAMS
     st = _family_stats(tctx, fams)
     k_ms = sum(v[1] for v in st.values())
+    plan = {}
+    for p in sorted({p for _, _, p in items}):
+        tctx.kernel_stats_reset()
+        tctx.sort_batch(keys, pay, [it for it in items if it[2] == p])
+        torch.cuda.synchronize()
+        plan[p] = sum(v[0] for v in _family_stats(tctx, fams).values())
     tctx.close()
+    alg = sum(2 * 12 * p * plan[p] for _, _, p in items)
     ach = alg / (call_ms * 1e-3) / 1e9
     roof = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": None,
             "kernel": "every sort pass of one batched call (local, merge, global, hybrid), timed as the whole call",
             "call_ms": round(call_ms, 3), "launch_ms_summed_over_streams": round(k_ms, 3),
-            "alg_bytes_per_call": alg, "passes_by_class": {str(p): plan[p] for p in sorted(plan)},
+            "alg_bytes_per_call": alg, "passes_by_class": {str(p): plan[p] for p in plan},
             "tuning": "default"}
     resident = _batch_resident(args, ctx, keys, pay, total, items, kb, pb, tp)
     compact = _compact_batch(args)
