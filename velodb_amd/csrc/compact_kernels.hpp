@@ -153,8 +153,18 @@ __device__ __forceinline__ uint64_t swap_lanes(uint32_t d, int q)
 template <int NW>
 __device__ __forceinline__ void swap_rows(uint64_t m, uint64_t (&x)[NW], uint64_t (&y)[NW])
 {
+    uint32_t a[2 * NW], b[2 * NW];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) dev::swap_m(m, x[w], y[w]);
+    for (int w = 0; w < 2 * NW; ++w) {
+        a[w] = (uint32_t)(x[w / 2] >> (32 * (w & 1)));
+        b[w] = (uint32_t)(y[w / 2] >> (32 * (w & 1)));
+    }
+    dev::swap_words<dev::Join::kCopy, 2 * NW>({m, 0}, a, b);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        x[w] = (uint64_t)a[2 * w] | ((uint64_t)a[2 * w + 1] << 32);
+        y[w] = (uint64_t)b[2 * w] | ((uint64_t)b[2 * w + 1] << 32);
+    }
 }
 
 // Instances of one size class 2^c of a batch: virtual row v of the class is

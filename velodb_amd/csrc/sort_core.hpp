@@ -56,110 +56,218 @@ __device__ __forceinline__ bool rec_gt(const R &a, const R &b)
 // Compare-exchange: afterwards a <= b when asc, a >= b otherwise.  Ties
 // (equal over every compared field) are left in place, as needSwap does
 // (sort.cuh:31-40).
-// The comparison runs on wavefront lane masks: each field costs one v_cmp
-// for > and one for <, the lexicographic combination and the direction are
-// scalar mask operations, and the swap is v_cndmask on the resulting mask
-// (2 per 32-bit word).  `ascm` holds the lanes whose pair sorts ascending.
-// Lanes where (a2:a1:a0) < (b2:b1:b0) as unsigned 96-bit numbers: the borrow
-// out of a subtract-with-borrow chain (three VALU ops, no scalar logic).
-__device__ __forceinline__ uint64_t lt_mask96(uint32_t a0, uint32_t b0, uint32_t a1, uint32_t b1, uint32_t a2,
-                                              uint32_t b2)
+// The comparison runs on wavefront lane masks and the swap is v_cndmask on the
+// resulting mask (2 per 32-bit word).  `ascm` holds the lanes whose pair sorts
+// ascending.
+//
+// Wait states.  On gfx950 a VALU instruction that reads a mask or a carry (an
+// SGPR pair or vcc) stands at least two wait states behind the VALU instruction
+// that wrote it: hipcc puts s_nop 1 between v_sub_co and v_subb_co, and fills
+// the distance from a v_cmp to its v_cndmask.  It does not look into asm blocks,
+// so they keep the distance themselves: borrow chains run interleaved (or on
+// s_nop), and a block of selects makes its mask with a scalar instruction of its
+// own, whose operands and result the hardware waits for (outside the block a
+// mask may come from a v_cmp, or from the v_readlane of a spilled register).
+
+// lt[i] = lanes where pair i has a < b as one unsigned integer of WORDS 32-bit
+// words: the borrow out of a subtract-with-borrow chain, a VALU instruction a
+// word and no scalar logic.  Four chains side by side keep the two wait states
+// for nothing; two need one s_nop 0 a word.
+#define VO_SUB(M, A, B) "v_sub_co_u32_e64 %[t], %[" M "], %[" A "], %[" B "]\n\t"
+#define VO_SUBB(M, A, B) "v_subb_co_u32_e64 %[t], %[" M "], %[" A "], %[" B "], %[" M "]\n\t"
+#define VO_WORD4(OP, W) OP("m0", "a0" W, "b0" W) OP("m1", "a1" W, "b1" W) OP("m2", "a2" W, "b2" W) OP("m3", "a3" W, "b3" W)
+#define VO_WORD2(OP, W) OP("m0", "a0" W, "b0" W) OP("m1", "a1" W, "b1" W)
+#define VO_WORD1(OP, W) OP("m0", "a0" W, "b0" W)
+#define VO_IN(I, W) [a##I##W] "v"(a[I][W]), [b##I##W] "v"(b[I][W])
+#define VO_IN3(I) VO_IN(I, 0), VO_IN(I, 1), VO_IN(I, 2)
+#define VO_IN4(I) VO_IN3(I), VO_IN(I, 3)
+#define VO_OUT(I) [m##I] "=&s"(lt[I])
+
+template <int N, int WORDS>
+__device__ __forceinline__ void lt_masks(uint64_t (&lt)[N], const uint32_t (&a)[N][WORDS],
+                                         const uint32_t (&b)[N][WORDS])
 {
-    uint64_t m;
-    uint32_t t0, t1, t2;
-    asm("v_sub_co_u32_e64 %0, %3, %4, %5\n\t"
-        "v_subb_co_u32_e64 %1, %3, %6, %7, %3\n\t"
-        "v_subb_co_u32_e64 %2, %3, %8, %9, %3"
-        : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&s"(m)
-        : "v"(a0), "v"(b0), "v"(a1), "v"(b1), "v"(a2), "v"(b2));
-    return m;
+    static_assert((N == 1 || N == 2 || N == 4) && (WORDS == 3 || WORDS == 4), "chains built");
+    uint32_t t;
+    if constexpr (N == 4 && WORDS == 3)
+        asm(VO_WORD4(VO_SUB, "0") VO_WORD4(VO_SUBB, "1") VO_WORD4(VO_SUBB, "2")
+            : [t] "=&v"(t), VO_OUT(0), VO_OUT(1), VO_OUT(2), VO_OUT(3)
+            : VO_IN3(0), VO_IN3(1), VO_IN3(2), VO_IN3(3));
+    else if constexpr (N == 4)
+        asm(VO_WORD4(VO_SUB, "0") VO_WORD4(VO_SUBB, "1") VO_WORD4(VO_SUBB, "2") VO_WORD4(VO_SUBB, "3")
+            : [t] "=&v"(t), VO_OUT(0), VO_OUT(1), VO_OUT(2), VO_OUT(3)
+            : VO_IN4(0), VO_IN4(1), VO_IN4(2), VO_IN4(3));
+    else if constexpr (N == 2 && WORDS == 3)
+        asm(VO_WORD2(VO_SUB, "0") "s_nop 0\n\t" VO_WORD2(VO_SUBB, "1") "s_nop 0\n\t" VO_WORD2(VO_SUBB, "2")
+            : [t] "=&v"(t), VO_OUT(0), VO_OUT(1)
+            : VO_IN3(0), VO_IN3(1));
+    else if constexpr (N == 2)
+        asm(VO_WORD2(VO_SUB, "0") "s_nop 0\n\t" VO_WORD2(VO_SUBB, "1") "s_nop 0\n\t" VO_WORD2(VO_SUBB, "2")
+            "s_nop 0\n\t" VO_WORD2(VO_SUBB, "3")
+            : [t] "=&v"(t), VO_OUT(0), VO_OUT(1)
+            : VO_IN4(0), VO_IN4(1));
+    else if constexpr (WORDS == 3)
+        asm(VO_WORD1(VO_SUB, "0") "s_nop 1\n\t" VO_WORD1(VO_SUBB, "1") "s_nop 1\n\t" VO_WORD1(VO_SUBB, "2")
+            : [t] "=&v"(t), VO_OUT(0)
+            : VO_IN3(0));
+    else
+        asm(VO_WORD1(VO_SUB, "0") "s_nop 1\n\t" VO_WORD1(VO_SUBB, "1") "s_nop 1\n\t" VO_WORD1(VO_SUBB, "2")
+            "s_nop 1\n\t" VO_WORD1(VO_SUBB, "3")
+            : [t] "=&v"(t), VO_OUT(0)
+            : VO_IN4(0));
 }
 
-__device__ __forceinline__ uint64_t lt_mask128(uint32_t a0, uint32_t b0, uint32_t a1, uint32_t b1, uint32_t a2,
-                                               uint32_t b2, uint32_t a3, uint32_t b3)
-{
-    uint64_t m;
-    uint32_t t0, t1, t2, t3;
-    asm("v_sub_co_u32_e64 %0, %4, %5, %6\n\t"
-        "v_subb_co_u32_e64 %1, %4, %7, %8, %4\n\t"
-        "v_subb_co_u32_e64 %2, %4, %9, %10, %4\n\t"
-        "v_subb_co_u32_e64 %3, %4, %11, %12, %4"
-        : "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3), "=&s"(m)
-        : "v"(a0), "v"(b0), "v"(a1), "v"(b1), "v"(a2), "v"(b2), "v"(a3), "v"(b3));
-    return m;
-}
+#undef VO_SUB
+#undef VO_SUBB
+#undef VO_WORD4
+#undef VO_WORD2
+#undef VO_WORD1
+#undef VO_IN
+#undef VO_IN3
+#undef VO_IN4
+#undef VO_OUT
 
-// Selects run as the VOP3 form of v_cndmask on a mask in scalar registers.  The
-// compiler shrinks a select whose mask it has put in vcc to the VOP2 form, and
-// that form issues in 23 cycles a wavefront on this chip where the VOP3 one
-// takes 4.5 (a compare and three selects: 14.1 against 4.2 cycles each).
-__device__ __forceinline__ uint32_t sel32(uint64_t m, uint32_t t, uint32_t f)
-{
-    uint32_t o;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(o) : "v"(f), "v"(t), "s"(m));
-    return o;
-}
+// The lanes that swap, as two masks and the scalar instruction that joins them.
+enum class Join { kXor, kOr, kCopy };
+struct SwapMask {
+    uint64_t a, b; // kCopy: a alone
+};
 
-// Exchanges x and y in the lanes of m.
-template <typename T>
-__device__ __forceinline__ void swap_m(uint64_t m, T &x, T &y)
+// Exchanges x[0 .. W-1] and y[0 .. W-1] in the lanes of m.  Selects run as the
+// VOP3 form of v_cndmask on a mask in scalar registers: the compiler shrinks a
+// select whose mask it has put in vcc to the VOP2 form, and that form issues in
+// 23 cycles a wavefront on this chip where the VOP3 one takes 4.5 (a compare,
+// its wait states and three selects: 14.2 against 4.2 cycles an instruction).
+#define VO_SEL(I)                                                                                                      \
+    "v_cndmask_b32_e64 %[o" I "], %[x" I "], %[y" I "], %[s]\n\t"                                                     \
+    "v_cndmask_b32_e64 %[y" I "], %[y" I "], %[x" I "], %[s]\n\t"
+#define VO_OUT(I) [o##I] "=&v"(o[I]), [y##I] "+v"(y[I])
+#define VO_SWAP(OP, ...)                                                                                               \
+    if constexpr (W == 2)                                                                                              \
+        asm(OP VO_SEL("0") VO_SEL("1")                                                                                 \
+            : [s] "=&s"(s), VO_OUT(0), VO_OUT(1)                                                                       \
+            : [x0] "v"(x[0]), [x1] "v"(x[1]), __VA_ARGS__                                                              \
+            : "scc");                                                                                                  \
+    else if constexpr (W == 3)                                                                                         \
+        asm(OP VO_SEL("0") VO_SEL("1") VO_SEL("2")                                                                     \
+            : [s] "=&s"(s), VO_OUT(0), VO_OUT(1), VO_OUT(2)                                                            \
+            : [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), __VA_ARGS__                                              \
+            : "scc");                                                                                                  \
+    else                                                                                                               \
+        asm(OP VO_SEL("0") VO_SEL("1") VO_SEL("2") VO_SEL("3")                                                         \
+            : [s] "=&s"(s), VO_OUT(0), VO_OUT(1), VO_OUT(2), VO_OUT(3)                                                 \
+            : [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), [x3] "v"(x[3]), __VA_ARGS__                              \
+            : "scc")
+
+template <Join J, int W>
+__device__ __forceinline__ void swap_block(SwapMask m, uint32_t *x, uint32_t *y)
 {
-    if constexpr (sizeof(T) == 8) {
-        const uint32_t xl = (uint32_t)x, xh = (uint32_t)((uint64_t)x >> 32);
-        const uint32_t yl = (uint32_t)y, yh = (uint32_t)((uint64_t)y >> 32);
-        x = (T)((uint64_t)sel32(m, yl, xl) | ((uint64_t)sel32(m, yh, xh) << 32));
-        y = (T)((uint64_t)sel32(m, xl, yl) | ((uint64_t)sel32(m, xh, yh) << 32));
+    static_assert(W >= 2 && W <= 4, "words of one block");
+    uint64_t s;
+    uint32_t o[W];
+    if constexpr (J == Join::kXor) {
+        VO_SWAP("s_xor_b64 %[s], %[a], %[b]\n\t", [a] "s"(m.a), [b] "s"(m.b));
+    } else if constexpr (J == Join::kOr) {
+        VO_SWAP("s_or_b64 %[s], %[a], %[b]\n\t", [a] "s"(m.a), [b] "s"(m.b));
     } else {
-        const uint32_t xv = (uint32_t)x, yv = (uint32_t)y;
-        x = (T)sel32(m, yv, xv);
-        y = (T)sel32(m, xv, yv);
+        VO_SWAP("s_mov_b64 %[s], %[a]\n\t", [a] "s"(m.a));
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w) x[w] = o[w];
+}
+
+#undef VO_OUT
+#undef VO_SEL
+#undef VO_SWAP
+
+template <Join J, int W>
+__device__ __forceinline__ void swap_words(SwapMask m, uint32_t *x, uint32_t *y)
+{
+    if constexpr (W > 4) {
+        swap_block<J, 3>(m, x, y);
+        swap_words<J, W - 3>(m, x + 3, y + 3);
+    } else {
+        swap_block<J, W>(m, x, y);
     }
 }
 
+// A record as 32-bit words, payload lowest.
 template <class R>
-__device__ __forceinline__ void cmpx_m(R &a, R &b, uint64_t ascm)
+constexpr int rec_words() { return 2 * R::KW + (int)sizeof(typename R::P) / 4; }
+
+template <class R>
+__device__ __forceinline__ void rec_to_words(uint32_t (&v)[rec_words<R>()], const R &r)
 {
-    uint64_t sw;
-    if constexpr (R::TIE && R::KW == 1) {
-        // (key, payload) records compare as one integer, key high.  Records
-        // equal in every field are identical, so exchanging them on a tie
-        // changes nothing and the swap is simply lt(a, b) xor ascending.
-        uint64_t lt;
-        if constexpr (sizeof(typename R::P) == 4)
-            lt = lt_mask96((uint32_t)a.p, (uint32_t)b.p, (uint32_t)a.k[0], (uint32_t)b.k[0],
-                           (uint32_t)(a.k[0] >> 32), (uint32_t)(b.k[0] >> 32));
-        else
-            lt = lt_mask128((uint32_t)a.p, (uint32_t)b.p, (uint32_t)((uint64_t)a.p >> 32),
-                            (uint32_t)((uint64_t)b.p >> 32), (uint32_t)a.k[0], (uint32_t)b.k[0],
-                            (uint32_t)(a.k[0] >> 32), (uint32_t)(b.k[0] >> 32));
-        sw = lt ^ ascm;
-    } else {
-        uint64_t gt = 0, lt = 0, eq = ~0ull;
+    constexpr int PW = (int)sizeof(typename R::P) / 4;
 #pragma unroll
-        for (int w = 0; w < R::KW; ++w) {
-            const uint64_t g = __builtin_amdgcn_ballot_w64(a.k[w] > b.k[w]);
-            const uint64_t l = __builtin_amdgcn_ballot_w64(a.k[w] < b.k[w]);
-            gt |= eq & g;
-            lt |= eq & l;
-            eq &= ~(g | l);
-        }
-        if constexpr (R::TIE) {
-            const uint64_t g = __builtin_amdgcn_ballot_w64(a.p > b.p);
-            const uint64_t l = __builtin_amdgcn_ballot_w64(a.p < b.p);
-            gt |= eq & g;
-            lt |= eq & l;
-        }
-        sw = (ascm & gt) | (~ascm & lt);
-    }
+    for (int w = 0; w < PW; ++w) v[w] = (uint32_t)((uint64_t)r.p >> (32 * w));
 #pragma unroll
-    for (int w = 0; w < R::KW; ++w) swap_m(sw, a.k[w], b.k[w]);
-    swap_m(sw, a.p, b.p);
+    for (int w = 0; w < 2 * R::KW; ++w) v[PW + w] = (uint32_t)(r.k[w / 2] >> (32 * (w & 1)));
 }
 
 template <class R>
-__device__ __forceinline__ void cmpx(R &a, R &b, bool asc)
+__device__ __forceinline__ void rec_from_words(R &r, const uint32_t (&v)[rec_words<R>()])
 {
-    cmpx_m(a, b, __builtin_amdgcn_ballot_w64(asc));
+    constexpr int PW = (int)sizeof(typename R::P) / 4;
+    if constexpr (PW == 2)
+        r.p = (typename R::P)((uint64_t)v[0] | ((uint64_t)v[1] << 32));
+    else
+        r.p = (typename R::P)v[0];
+#pragma unroll
+    for (int w = 0; w < R::KW; ++w) r.k[w] = (uint64_t)v[PW + 2 * w] | ((uint64_t)v[PW + 2 * w + 1] << 32);
+}
+
+// Compare-exchanges of one stage on a thread's registers: register m with
+// m | 1 << bit, ascending where asc(m).  Four pairs at a time, whose compares
+// are interleaved.
+template <class R, int RR, class D>
+__device__ __forceinline__ void cmpx_stage(R (&r)[RR], int bit, D asc)
+{
+    constexpr int N = RR / 2 < 4 ? RR / 2 : 4, W = rec_words<R>();
+#pragma unroll
+    for (int g = 0; g < RR / 2; g += N) {
+        auto lower = [&](int i) { return (((g + i) >> bit) << (bit + 1)) | ((g + i) & ((1 << bit) - 1)); };
+        uint32_t x[N][W], y[N][W];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            rec_to_words(x[i], r[lower(i)]);
+            rec_to_words(y[i], r[lower(i) | (1 << bit)]);
+        }
+        if constexpr (R::TIE && R::KW == 1) {
+            // (key, payload) records compare as one integer, key high.  Records
+            // equal in every field are identical, so exchanging them on a tie
+            // changes nothing and the swap is simply lt(x, y) xor ascending.
+            uint64_t lt[N];
+            lt_masks<N, W>(lt, x, y);
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                swap_words<Join::kXor, W>({lt[i], __builtin_amdgcn_ballot_w64(asc(lower(i)))}, x[i], y[i]);
+        } else {
+            static_assert(!R::TIE, "other records leave ties in place");
+            // each key word costs one v_cmp for > and one for <; the lexicographic
+            // combination and the direction are scalar mask operations
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const R &a = r[lower(i)], &b = r[lower(i) | (1 << bit)];
+                const uint64_t ascm = __builtin_amdgcn_ballot_w64(asc(lower(i)));
+                uint64_t gt = 0, lt = 0, eq = ~0ull;
+#pragma unroll
+                for (int w = 0; w < R::KW; ++w) {
+                    const uint64_t g = __builtin_amdgcn_ballot_w64(a.k[w] > b.k[w]);
+                    const uint64_t l = __builtin_amdgcn_ballot_w64(a.k[w] < b.k[w]);
+                    gt |= eq & g;
+                    lt |= eq & l;
+                    eq &= ~(g | l);
+                }
+                swap_words<Join::kOr, W>({ascm & gt, ~ascm & lt}, x[i], y[i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            rec_from_words(r[lower(i)], x[i]);
+            rec_from_words(r[lower(i) | (1 << bit)], y[i]);
+        }
+    }
 }
 
 // Scalar reference form of the same exchange (used by the one-thread kernel,
@@ -349,12 +457,7 @@ __device__ __forceinline__ void reg_stages(R (&r)[1 << R_LOG], uint32_t tau, int
     for (int qq = R_LOG - 1; qq >= 0; --qq) {
         const int q = a + qq;
         if (q > q_hi || q < q_lo) continue;
-#pragma unroll
-        for (int m = 0; m < (1 << R_LOG); ++m) {
-            if (m & (1 << qq)) continue;
-            const uint64_t g = vbase + (base | ((uint32_t)m << a));
-            cmpx(r[m], r[m | (1 << qq)], dir_asc(g, p, p_top));
-        }
+        cmpx_stage(r, qq, [&](int m) { return dir_asc(vbase + (base | ((uint32_t)m << a)), p, p_top); });
     }
 }
 
@@ -435,7 +538,7 @@ struct TileCT {
     // Stage Q (0 or 1) of level P in layouts 1 and 2: record index bit Q is
     // thread index bit Q, so the pair of register m is register m of two lanes
     // of a quad.  Issue-bound, so it is kept to six VALU instructions a record:
-    // the borrow chain of lt_mask96 reads the partner's words through a DPP quad
+    // the borrow chain of lt_masks reads the partner's words through a DPP quad
     // permutation, and the words move by DPP moves under the execution mask of
     // the swapping pairs.  (Written with selects it compiled to 64-bit compares
     // per record and took 10 us of a 2^23-record pass, as long as the other
@@ -451,12 +554,15 @@ struct TileCT {
     {
         uint32_t w0 = (uint32_t)r.p, w1 = (uint32_t)r.k[0], w2 = (uint32_t)(r.k[0] >> 32), t;
         uint64_t sw, ex;
-        // s_nop: a DPP read needs two wait states after a VALU write of the
-        // register; %6 holds the lower lane of every pair
+        // s_nop: two wait states before a DPP read of a register that a VALU
+        // instruction wrote, and before each read of the borrow (see
+        // lt_masks); %6 holds the lower lane of every pair
 #define VO_LANE_CMPX(PERM, SHIFT, LOWER)                                                                               \
     asm("s_nop 1\n\t"                                                                                                  \
         "v_sub_co_u32_dpp %3, vcc, %0, %0 quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                            \
+        "s_nop 1\n\t"                                                                                                 \
         "v_subb_co_u32_dpp %3, vcc, %1, %1, vcc quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                      \
+        "s_nop 1\n\t"                                                                                                 \
         "v_subb_co_u32_dpp %3, vcc, %2, %2, vcc quad_perm:" PERM " row_mask:0xf bank_mask:0xf\n\t"                      \
         "s_and_b64 %4, vcc, %6\n\t"                                                                                    \
         "s_lshl_b64 vcc, %4, " SHIFT "\n\t"                                                                            \
@@ -660,19 +766,14 @@ struct TileCT {
         const uint32_t base = lay_base<R_LOG>(tau, A);
 #pragma unroll
         for (int q = QHI; q >= QLO; --q) {
-            const int qq = q - A;
-#pragma unroll
-            for (int m = 0; m < RR; ++m) {
-                if (m & (1 << qq)) continue;
-                bool asc;
+            cmpx_stage(r, q - A, [&](int m) -> bool {
                 if constexpr (P < 0) {
-                    asc = asc_hi;
+                    return asc_hi;
                 } else {
                     const uint32_t l = base | ((uint32_t)m << A);
-                    asc = (P >= p_top) | (P >= T_LOG ? asc_hi : (((l >> P) & 1u) == 0));
+                    return (P >= p_top) | (P >= T_LOG ? asc_hi : (((l >> P) & 1u) == 0));
                 }
-                cmpx(r[m], r[m | (1 << qq)], asc);
-            }
+            });
         }
     }
 

@@ -417,13 +417,7 @@ __device__ __forceinline__ void body_global(Bufs<R> b, IMap map, int p, int q_lo
     for (int m = 0; m < (1 << S); ++m) gload_t<R, TRACE, CP>(r[m], b, pbase, (uint32_t)m << q_lo, tid, h, nops);
     const bool asc = dir_asc(ubase, p, p_top);
 #pragma unroll
-    for (int qq = S - 1; qq >= 0; --qq) {
-#pragma unroll
-        for (int m = 0; m < (1 << S); ++m) {
-            if (m & (1 << qq)) continue;
-            cmpx(r[m], r[m | (1 << qq)], asc);
-        }
-    }
+    for (int qq = S - 1; qq >= 0; --qq) cmpx_stage(r, qq, [&](int) { return asc; });
 #pragma unroll
     for (int m = 0; m < (1 << S); ++m) gstore_t<R, TRACE, CP>(r[m], b, pbase, (uint32_t)m << q_lo, tid, h, nops);
     if constexpr (TRACE) tcommit(slot, g0 + tid, h, nops);
