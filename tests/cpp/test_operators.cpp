@@ -8,10 +8,14 @@
 // every case is also checked against a host stable sort of the same rows.
 #include "velodb_amd/operators.hpp"
 
+#include <dlfcn.h>
+
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <functional>
+#include <new>
 #include <numeric>
 #include <random>
 #include <set>
@@ -49,6 +53,23 @@ static int g_fail = 0;
             ++g_fail;                                                                                                  \
         }                                                                                                              \
     } while (0)
+
+// Host allocations made by the library itself while g_count_allocs is set (the
+// library's operator new resolves to the program's).
+static bool g_count_allocs = false;
+static size_t g_lib_allocs = 0;
+
+__attribute__((noinline)) void *operator new(std::size_t n)
+{
+    Dl_info at;
+    if (g_count_allocs && dladdr(__builtin_return_address(0), &at) && at.dli_fname &&
+        std::strstr(at.dli_fname, "libvelodb_amd"))
+        ++g_lib_allocs;
+    if (void *p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+__attribute__((noinline)) void operator delete(void *p) noexcept { std::free(p); }
+__attribute__((noinline)) void operator delete(void *p, std::size_t) noexcept { std::free(p); }
 
 // employees (test_order_by.cpp:35-42)
 static const std::vector<int32_t> kId = {3, 1, 5, 2, 4, 6, 7, 8};
@@ -1081,6 +1102,49 @@ static void test_task_manager_queue(ExecutionContext &)
 // --persistent: the shared TaskManager runs every operator's commands in the
 // resident queue kernel (TaskManager::start with persistent = true), as a
 // reference caller with a persistent TaskManager would.
+// vo_compact_noalloc allocates nothing, on the host either, and compacts every
+// column in order of its rows (launch mode: a resident queue would be parked first).
+static void test_compact_noalloc_allocates_nothing(TaskManager &tm)
+{
+    constexpr uint64_t N = 4096;
+    const uint32_t widths[VO_MAX_SORT_COLUMNS] = {8, 4, 1, 2, 8, 1, 4, 2};
+    char *dev = nullptr;
+    CHECK(hipMalloc((void **)&dev, N * 8 * (VO_MAX_SORT_COLUMNS + 1)) == hipSuccess);
+    std::vector<uint8_t> mask(N);
+    std::vector<uint64_t> want;
+    for (uint64_t i = 0; i < N; ++i) {
+        mask[i] = i % 3 == 1;
+        if (mask[i]) want.push_back(i);
+    }
+    vo_compact_args a{};
+    a.mask = (const uint8_t *)dev;
+    a.n = a.n_pad = N;
+    a.n_cols = VO_MAX_SORT_COLUMNS;
+    CHECK(hipMemcpy(dev, mask.data(), N, hipMemcpyHostToDevice) == hipSuccess);
+    for (uint32_t c = 0; c < a.n_cols; ++c) {
+        std::vector<char> host(N * 8);
+        for (uint64_t i = 0; i < N; ++i) std::memcpy(&host[i * widths[c]], &i, widths[c]);
+        a.cols[c] = dev + N * 8 * (c + 1);
+        a.col_bytes[c] = widths[c];
+        CHECK(hipMemcpy(a.cols[c], host.data(), N * widths[c], hipMemcpyHostToDevice) == hipSuccess);
+    }
+    g_lib_allocs = 0;
+    g_count_allocs = true;
+    const int st = vo_compact_noalloc(tm.native(), &a);
+    g_count_allocs = false;
+    CHECK(st == VO_OK);
+    CHECK(vo_sync(tm.native()) == VO_OK);
+    CHECK(g_lib_allocs == 0);
+    for (uint32_t c = 0; c < a.n_cols; ++c) {
+        std::vector<char> host(want.size() * widths[c]);
+        CHECK(hipMemcpy(host.data(), a.cols[c], host.size(), hipMemcpyDeviceToHost) == hipSuccess);
+        bool same = true;
+        for (size_t k = 0; k < want.size(); ++k) same &= !std::memcmp(&host[k * widths[c]], &want[k], widths[c]);
+        CHECK(same);
+    }
+    CHECK(hipFree(dev) == hipSuccess);
+}
+
 int main(int argc, char **argv)
 {
     const bool persistent = argc > 1 && std::string(argv[1]) == "--persistent";
@@ -1112,6 +1176,10 @@ int main(int argc, char **argv)
         {"errors_are_results", [&] { test_errors_are_results(ctx); }},
         {"task_manager_queue", [&] { test_task_manager_queue(ctx); }},
         {"plan_nodes", [&] { test_plan_nodes(ctx); }},
+        {"compact_noalloc_allocates_nothing",
+         [&] {
+             if (!persistent) test_compact_noalloc_allocates_nothing(tm);
+         }},
         {"multi_batch_sort", [&] { test_multi_batch_sort(ctx); }},
         {"multi_batch_filter", [&] { test_multi_batch_filter(ctx); }},
         {"multi_batch_sort_merge_join", [&] { test_multi_batch_sort_merge_join(ctx); }},

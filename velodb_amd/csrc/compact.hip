@@ -237,37 +237,40 @@ Word word8(void *p) { return Word{{p}, {8}}; }
 // the mask only, so how columns share words changes no output.  (8-, 4- and
 // 1-byte columns of 10M rows / 2^24: one run of two words instead of one of two
 // and one of one, WHERE and compaction together 616 -> 432 us.)
-std::vector<Word> pack_words(void *const *cols, const uint32_t *bytes, uint32_t n)
+// A fixed array: vo_compact_noalloc allocates nothing, on the host either.
+struct Words {
+    Word v[VO_MAX_SORT_COLUMNS];
+    uint32_t n = 0;
+};
+
+Words pack_words(void *const *cols, const uint32_t *bytes, uint32_t n)
 {
-    std::vector<Word> v;
-    std::vector<uint32_t> used;
+    Words ws{};
+    uint32_t used[VO_MAX_SORT_COLUMNS] = {};
     for (uint32_t width : {8u, 4u, 2u, 1u})
         for (uint32_t c = 0; c < n; ++c) {
             if (bytes[c] != width) continue;
-            size_t i = 0;
-            while (i < v.size() && (used[i] + width > 8 || v[i].w[kParts - 1] != 0)) ++i;
-            if (i == v.size()) {
-                v.push_back(Word{});
-                used.push_back(0);
-            }
+            uint32_t i = 0;
+            while (i < ws.n && (used[i] + width > 8 || ws.v[i].w[kParts - 1] != 0)) ++i;
+            ws.n = std::max(ws.n, i + 1);
             int k = 0;
-            while (v[i].w[k] != 0) ++k;
-            v[i].p[k] = cols[c];
-            v[i].w[k] = width;
+            while (ws.v[i].w[k] != 0) ++k;
+            ws.v[i].p[k] = cols[c];
+            ws.v[i].w[k] = width;
             used[i] += width;
         }
-    return v;
+    return ws;
 }
 
 // One run of the network per two words.
 template <class F>
-void run_words(const std::vector<Word> &v, F &&run)
+void run_words(const Words &ws, F &&run)
 {
-    for (size_t i = 0; i < v.size(); i += 2) {
-        if (i + 1 < v.size())
-            run(Cols<2>{{v[i], v[i + 1]}});
+    for (uint32_t i = 0; i < ws.n; i += 2) {
+        if (i + 1 < ws.n)
+            run(Cols<2>{{ws.v[i], ws.v[i + 1]}});
         else
-            run(Cols<1>{{v[i]}});
+            run(Cols<1>{{ws.v[i]}});
     }
 }
 
@@ -399,7 +402,7 @@ void op_compact_batch(vo_ctx *ctx, const vo_compact_batch_args &a)
     char *base = (char *)scratch(ctx, bytes);
     uint64_t *dtab = (uint64_t *)base;
     upload_async(ctx, dtab, host.data(), host.size() * 8);
-    const std::vector<Word> words = pack_words(a.cols, a.col_bytes, a.n_cols);
+    const Words words = pack_words(a.cols, a.col_bytes, a.n_cols);
     run_tracks(ctx, classes.size(), [&](size_t t) {
         const int c = classes[t];
         const uint64_t k = off[c].size();
