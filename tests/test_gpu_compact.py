@@ -256,3 +256,25 @@ def test_compact_pass_shapes(log2n, widths, tuning):
     assert int(cnt.item()) == int((sel != 0).sum())
     want = oracle.compact(_rows(cols), (sel != 0).astype(np.uint8))
     assert np.array_equal(_rows([from_dev(d, c.dtype) for d, c in zip(dc, cols)]), want)
+
+
+@pytest.mark.parametrize("widths,same", [([8, 4, 8, 8], (2, 3)), ([8, 8, 4], (0, 1)), ([8, 4, 1, 1], (2, 3)),
+                                         ([8, 1, 8, 2, 2], (3, 4))])
+def test_compact_column_named_twice(vctx, widths, same):
+    """A column that stands twice in the list is compacted once, wherever
+    packing puts its two entries."""
+    import torch
+    n = 1 << 13
+    print(f"column named twice widths={widths} same={same}", flush=True)
+    rng = np.random.default_rng(len(widths))
+    mask = (rng.random(n) < 0.4).astype(np.uint8)
+    cols = [rng.integers(0, 1 << (8 * w - 1), n).astype({1: np.uint8, 2: np.uint16, 4: np.uint32, 8: np.uint64}[w])
+            for w in widths]
+    cols[same[1]] = cols[same[0]]
+    dc = [to_dev(c) for c in cols]
+    dc[same[1]] = dc[same[0]]
+    cnt = torch.zeros(1, dtype=torch.int64, device="cuda:0")
+    vctx.compact(to_dev(mask), dc, widths, n, n, out_count=cnt)
+    assert int(cnt.item()) == int(mask.sum())
+    got = _rows([from_dev(d, c.dtype) for d, c in zip(dc, cols)])
+    assert np.array_equal(got, oracle.compact(_rows(cols), mask))

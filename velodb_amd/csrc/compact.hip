@@ -250,6 +250,9 @@ Words pack_words(void *const *cols, const uint32_t *bytes, uint32_t n)
     for (uint32_t width : {8u, 4u, 2u, 1u})
         for (uint32_t c = 0; c < n; ++c) {
             if (bytes[c] != width) continue;
+            bool again = false; // named before: in place, it is compacted once
+            for (uint32_t d = 0; d < c; ++d) again |= cols[d] == cols[c] && bytes[d] == width;
+            if (again) continue;
             uint32_t i = 0;
             while (i < ws.n && (used[i] + width > 8 || ws.v[i].w[kParts - 1] != 0)) ++i;
             ws.n = std::max(ws.n, i + 1);
