@@ -278,3 +278,22 @@ def test_compact_column_named_twice(vctx, widths, same):
     assert int(cnt.item()) == int(mask.sum())
     got = _rows([from_dev(d, c.dtype) for d, c in zip(dc, cols)])
     assert np.array_equal(got, oracle.compact(_rows(cols), mask))
+
+
+@pytest.mark.parametrize("widths,at", [([4, 2, 2, 2, 1, 1, 1, 1], 6), ([1, 8, 8], 0), ([8, 8, 1, 2], 2), ([1], 0)])
+def test_compact_mask_among_the_columns(vctx, widths, at):
+    """The mask may stand among the columns: it is compacted with them, after
+    every other column has been routed by it."""
+    import torch
+    n = 1 << 13
+    print(f"mask among the columns widths={widths} at={at}", flush=True)
+    rng = np.random.default_rng(at)
+    mask = (rng.random(n) < 0.4).astype(np.uint8)
+    cols = [rng.integers(0, 1 << (8 * w - 1), n).astype({1: np.uint8, 2: np.uint16, 4: np.uint32, 8: np.uint64}[w])
+            for w in widths]
+    cols[at] = mask
+    dc = [to_dev(c) for c in cols]
+    cnt = torch.zeros(1, dtype=torch.int64, device="cuda:0")
+    vctx.compact(dc[at], dc, widths, n, n, out_count=cnt)
+    assert int(cnt.item()) == int(mask.sum())
+    assert np.array_equal(_rows([from_dev(d, c.dtype) for d, c in zip(dc, cols)]), oracle.compact(_rows(cols), mask))

@@ -243,25 +243,36 @@ struct Words {
     uint32_t n = 0;
 };
 
-Words pack_words(void *const *cols, const uint32_t *bytes, uint32_t n)
+Words pack_words(const uint8_t *mask, void *const *cols, const uint32_t *bytes, uint32_t n)
 {
     Words ws{};
     uint32_t used[VO_MAX_SORT_COLUMNS] = {};
+    auto place = [&](uint32_t c) {
+        uint32_t i = 0;
+        while (i < ws.n && (used[i] + bytes[c] > 8 || ws.v[i].w[kParts - 1] != 0)) ++i;
+        ws.n = std::max(ws.n, i + 1);
+        int k = 0;
+        while (ws.v[i].w[k] != 0) ++k;
+        ws.v[i].p[k] = cols[c];
+        ws.v[i].w[k] = bytes[c];
+        used[i] += bytes[c];
+    };
+    auto is_mask = [&](uint32_t c) { return cols[c] == mask && bytes[c] == 1; };
+    uint32_t own = n;
     for (uint32_t width : {8u, 4u, 2u, 1u})
         for (uint32_t c = 0; c < n; ++c) {
             if (bytes[c] != width) continue;
             bool again = false; // named before: in place, it is compacted once
             for (uint32_t d = 0; d < c; ++d) again |= cols[d] == cols[c] && bytes[d] == width;
             if (again) continue;
-            uint32_t i = 0;
-            while (i < ws.n && (used[i] + width > 8 || ws.v[i].w[kParts - 1] != 0)) ++i;
-            ws.n = std::max(ws.n, i + 1);
-            int k = 0;
-            while (ws.v[i].w[k] != 0) ++k;
-            ws.v[i].p[k] = cols[c];
-            ws.v[i].w[k] = width;
-            used[i] += width;
+            if (is_mask(c))
+                own = c;
+            else
+                place(c);
         }
+    // the mask itself goes with the last run, when it has routed the others
+    // (every word but the last has no room for a byte)
+    if (own < n) place(own);
     return ws;
 }
 
@@ -337,7 +348,7 @@ void compact_with(vo_ctx *ctx, const vo_compact_args &a, const Workspace &ws)
         VO_CHECK(a.cols[c] && (w == 1 || w == 2 || w == 4 || w == 8), VO_ERR_INVALID, "bad column");
     }
     count_and_scan(ctx, a.mask, a.n, a.n_pad, ws, a.out_count);
-    run_words(pack_words(a.cols, a.col_bytes, a.n_cols), [&](auto cs) {
+    run_words(pack_words(a.mask, a.cols, a.col_bytes, a.n_cols), [&](auto cs) {
         run_network(ctx, cs, cs, a.mask, a.n, a.n_pad, ws.tile_pre);
     });
 }
@@ -405,7 +416,7 @@ void op_compact_batch(vo_ctx *ctx, const vo_compact_batch_args &a)
     char *base = (char *)scratch(ctx, bytes);
     uint64_t *dtab = (uint64_t *)base;
     upload_async(ctx, dtab, host.data(), host.size() * 8);
-    const Words words = pack_words(a.cols, a.col_bytes, a.n_cols);
+    const Words words = pack_words(a.mask, a.cols, a.col_bytes, a.n_cols);
     run_tracks(ctx, classes.size(), [&](size_t t) {
         const int c = classes[t];
         const uint64_t k = off[c].size();
