@@ -297,3 +297,39 @@ def test_compact_mask_among_the_columns(vctx, widths, at):
     vctx.compact(dc[at], dc, widths, n, n, out_count=cnt)
     assert int(cnt.item()) == int(mask.sum())
     assert np.array_equal(_rows([from_dev(d, c.dtype) for d, c in zip(dc, cols)]), oracle.compact(_rows(cols), mask))
+
+
+@pytest.mark.parametrize("log2n", [12, 13, 14, 20, 21, 22])
+@pytest.mark.parametrize("short", [0, 4099])
+@pytest.mark.parametrize("tuning", [0, 0x800])
+def test_filter_sum_tile_sizes(log2n, short, tuning):
+    """One partial sum per tile of 2^12 or 2^13 rows, on both sides of every
+    change of the tile and with rows missing from the last ones: products of
+    both signs below 2^104, so that the sum carries between the halves of the
+    int128 and stays below 2^126 over 2^22 rows; count and sum against Python integers, whole columns (given or in
+    place) against the oracle's network."""
+    import torch
+    import velodb_amd
+    n_pad = 1 << log2n
+    n = max(1, n_pad - short)
+    print(f"filter tiles 2^{log2n} n={n} tuning={tuning:#x}", flush=True)
+    rng = np.random.default_rng(log2n + short)
+    day = rng.integers(8600, 9300, n_pad).astype(np.int32)
+    qty = rng.integers(1, 51, n_pad)
+    price, disc = (rng.integers(-(1 << 52), 1 << 52, n_pad) for _ in range(2))
+    sel = (day >= 8766) & (day < 9131) & (qty < 24) & (np.arange(n_pad) < n)
+    dd = [to_dev(a) for a in (day, qty, price, disc)]
+    out, op, od = empty_dev(4, np.uint64), empty_dev(n_pad, np.int64), empty_dev(n_pad, np.int64)
+    with velodb_amd.Context(stream=torch.cuda.current_stream().cuda_stream, tuning=tuning) as ctx:
+        wide = dict(disc_lo=-(1 << 63), disc_hi=(1 << 63) - 1)
+        if log2n % 2:
+            ctx.filter_sum(*dd, n, n_pad, out, out_price=op, out_disc=od, **wide)
+        else:
+            ctx.filter_sum(*dd, n, n_pad, out, **wide)
+            op, od = dd[2], dd[3]
+    o = [int(x) for x in from_dev(out, np.uint64)]
+    total = o[2] | (o[3] << 64)
+    assert o[0] == int(sel.sum())
+    assert total - (1 << 128 if total >> 127 else 0) == sum(int(a) * int(b) for a, b in zip(price[sel], disc[sel]))
+    want = oracle.compact(_rows([price, disc]), sel.astype(np.uint8))
+    assert np.array_equal(_rows([from_dev(op, np.int64), from_dev(od, np.int64)]), want)
