@@ -138,33 +138,50 @@ struct SwapMask {
 // select whose mask it has put in vcc to the VOP2 form, and that form issues in
 // 23 cycles a wavefront on this chip where the VOP3 one takes 4.5 (a compare,
 // its wait states and three selects: 14.2 against 4.2 cycles an instruction).
-#define VO_SEL(I)                                                                                                      \
+// OWN: the new y stays in y's registers.  It saves W registers, which the
+// 12-byte sort's 64-VGPR passes need (nine-stage pass: no spill instead of 7
+// VGPRs), but costs moves where 8-byte columns must stand in register pairs
+// (two key words, local pass: 10477 VALU instructions instead of 9035).
+#define VO_SEL(I, D)                                                                                                   \
     "v_cndmask_b32_e64 %[o" I "], %[x" I "], %[y" I "], %[s]\n\t"                                                     \
-    "v_cndmask_b32_e64 %[y" I "], %[y" I "], %[x" I "], %[s]\n\t"
-#define VO_OUT(I) [o##I] "=&v"(o[I]), [y##I] "+v"(y[I])
+    "v_cndmask_b32_e64 %[" D I "], %[y" I "], %[x" I "], %[s]\n\t"
+#define VO_NEW(I) [o##I] "=&v"(o[I]), [n##I] "=&v"(n[I])
+#define VO_OWN(I) [o##I] "=&v"(o[I]), [y##I] "+v"(y[I])
+#define VO_IN(I) [x##I] "v"(x[I]), [y##I] "v"(y[I])
 #define VO_SWAP(OP, ...)                                                                                               \
-    if constexpr (W == 2)                                                                                              \
-        asm(OP VO_SEL("0") VO_SEL("1")                                                                                 \
-            : [s] "=&s"(s), VO_OUT(0), VO_OUT(1)                                                                       \
-            : [x0] "v"(x[0]), [x1] "v"(x[1]), __VA_ARGS__                                                              \
-            : "scc");                                                                                                  \
-    else if constexpr (W == 3)                                                                                         \
-        asm(OP VO_SEL("0") VO_SEL("1") VO_SEL("2")                                                                     \
-            : [s] "=&s"(s), VO_OUT(0), VO_OUT(1), VO_OUT(2)                                                            \
+    if constexpr (OWN)                                                                                                 \
+        asm(OP VO_SEL("0", "y") VO_SEL("1", "y") VO_SEL("2", "y")                                                      \
+            : [s] "=&s"(s), VO_OWN(0), VO_OWN(1), VO_OWN(2)                                                            \
             : [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), __VA_ARGS__                                              \
             : "scc");                                                                                                  \
+    else if constexpr (W == 2)                                                                                         \
+        asm(OP VO_SEL("0", "n") VO_SEL("1", "n")                                                                       \
+            : [s] "=&s"(s), VO_NEW(0), VO_NEW(1)                                                                       \
+            : VO_IN(0), VO_IN(1), __VA_ARGS__                                                                          \
+            : "scc");                                                                                                  \
+    else if constexpr (W == 3)                                                                                         \
+        asm(OP VO_SEL("0", "n") VO_SEL("1", "n") VO_SEL("2", "n")                                                      \
+            : [s] "=&s"(s), VO_NEW(0), VO_NEW(1), VO_NEW(2)                                                            \
+            : VO_IN(0), VO_IN(1), VO_IN(2), __VA_ARGS__                                                                \
+            : "scc");                                                                                                  \
+    else if constexpr (W == 4)                                                                                         \
+        asm(OP VO_SEL("0", "n") VO_SEL("1", "n") VO_SEL("2", "n") VO_SEL("3", "n")                                     \
+            : [s] "=&s"(s), VO_NEW(0), VO_NEW(1), VO_NEW(2), VO_NEW(3)                                                 \
+            : VO_IN(0), VO_IN(1), VO_IN(2), VO_IN(3), __VA_ARGS__                                                      \
+            : "scc");                                                                                                  \
     else                                                                                                               \
-        asm(OP VO_SEL("0") VO_SEL("1") VO_SEL("2") VO_SEL("3")                                                         \
-            : [s] "=&s"(s), VO_OUT(0), VO_OUT(1), VO_OUT(2), VO_OUT(3)                                                 \
-            : [x0] "v"(x[0]), [x1] "v"(x[1]), [x2] "v"(x[2]), [x3] "v"(x[3]), __VA_ARGS__                              \
+        asm(OP VO_SEL("0", "n") VO_SEL("1", "n") VO_SEL("2", "n") VO_SEL("3", "n") VO_SEL("4", "n")                    \
+            : [s] "=&s"(s), VO_NEW(0), VO_NEW(1), VO_NEW(2), VO_NEW(3), VO_NEW(4)                                      \
+            : VO_IN(0), VO_IN(1), VO_IN(2), VO_IN(3), VO_IN(4), __VA_ARGS__                                            \
             : "scc")
 
 template <Join J, int W>
 __device__ __forceinline__ void swap_block(SwapMask m, uint32_t *x, uint32_t *y)
 {
-    static_assert(W >= 2 && W <= 4, "words of one block");
+    static_assert(W >= 2 && W <= 5, "words of one block");
+    constexpr bool OWN = J == Join::kXor && W == 3;
     uint64_t s;
-    uint32_t o[W];
+    uint32_t o[W], n[W];
     if constexpr (J == Join::kXor) {
         VO_SWAP("s_xor_b64 %[s], %[a], %[b]\n\t", [a] "s"(m.a), [b] "s"(m.b));
     } else if constexpr (J == Join::kOr) {
@@ -173,19 +190,25 @@ __device__ __forceinline__ void swap_block(SwapMask m, uint32_t *x, uint32_t *y)
         VO_SWAP("s_mov_b64 %[s], %[a]\n\t", [a] "s"(m.a));
     }
 #pragma unroll
-    for (int w = 0; w < W; ++w) x[w] = o[w];
+    for (int w = 0; w < W; ++w) {
+        x[w] = o[w];
+        if constexpr (!OWN) y[w] = n[w];
+    }
 }
 
-#undef VO_OUT
 #undef VO_SEL
+#undef VO_NEW
+#undef VO_OWN
+#undef VO_IN
 #undef VO_SWAP
 
 template <Join J, int W>
 __device__ __forceinline__ void swap_words(SwapMask m, uint32_t *x, uint32_t *y)
 {
-    if constexpr (W > 4) {
-        swap_block<J, 3>(m, x, y);
-        swap_words<J, W - 3>(m, x + 3, y + 3);
+    if constexpr (W > 5) {
+        constexpr int F = W == 6 ? 4 : 5; // at least two words stay
+        swap_block<J, F>(m, x, y);
+        swap_words<J, W - F>(m, x + F, y + F);
     } else {
         swap_block<J, W>(m, x, y);
     }
