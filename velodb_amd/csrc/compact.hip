@@ -177,12 +177,7 @@ void run_network_t(vo_ctx *ctx, Cols<NW> src, Cols<NW> cols, const uint8_t *mask
         case 2: launch(ctx, li, k_compact_global<NW, 2, TR, NT>, cols, tile_pre, q, in, trace_slot(ctx)); break;
         case 3: launch(ctx, li, k_compact_global<NW, 3, TR, NT>, cols, tile_pre, q, in, trace_slot(ctx)); break;
         case 4: launch(ctx, li, k_compact_global<NW, 4, TR, NT>, cols, tile_pre, q, in, trace_slot(ctx)); break;
-        default:
-            if constexpr (NW == 1) {
-                launch(ctx, li, k_compact_global<NW, 5, TR, NT>, cols, tile_pre, q, in, trace_slot(ctx));
-                break;
-            }
-            throw Error{VO_ERR_INVALID, "compaction pass width"};
+        default: throw Error{VO_ERR_INVALID, "compaction pass width"};
         }
         q += s;
     }
@@ -411,7 +406,7 @@ void op_compact_batch(vo_ctx *ctx, const vo_compact_batch_args &a)
         cnt_at[c] = bytes;
         bytes += al(tiles * 4);
         pre_at[c] = bytes;
-        bytes += al((tiles + 1) * 8); // the hybrid pass reads one prefix past its group
+        bytes += al(tiles * 8);
     }
     char *base = (char *)scratch(ctx, bytes);
     uint64_t *dtab = (uint64_t *)base;

@@ -609,7 +609,6 @@ __device__ __forceinline__ void b_compact_local(Cols<NW> src, Cols<NW> dst, cons
                                                 __int128 *__restrict__ partial, TraceSlot *slot, char *lds_raw,
                                                 uint32_t vb)
 {
-    using TL = CTileOf<T>;
     constexpr int NTHR = 1 << (T - 4), AS = T - 4;
     dev::TileBuf buf{lds_raw};
     uint32_t *c16 = reinterpret_cast<uint32_t *>(lds_raw + cbuf_bytes<T>());
@@ -798,7 +797,6 @@ template <int NW, int S, bool W8, bool TRACE, bool NT = false, int T = CT_LOG>
 __device__ __forceinline__ void b_compact_hybrid(Cols<NW> cols, const uint64_t *__restrict__ tile_pre, int q_lo,
                                                  Inst in, TraceSlot *slot, char *lds_raw, uint32_t vb)
 {
-    using TL = CTileOf<T>;
     dev::AtrT<TRACE> tr(slot);
     constexpr int C = T - S, NTHR = 1 << (T - 4), AS = T - 4;
     static_assert(S >= 5 && C >= 4, "hybrid widths 5..T-4");

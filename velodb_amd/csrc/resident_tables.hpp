@@ -112,7 +112,7 @@
 // the 1024-thread tile scan runs as a 256-thread body on the resident grid;
 // LDS_EXTRA: the scan's 256 words, the int128 reductions' 256 values
 #define VO_COMPACT_BODIES(X)                                                                                       \
-    VO_COMPACT_NW(X, 1) VO_COMPACT_NW(X, 2) VO_COMPACT_G(X, 1, 5)                                                  \
+    VO_COMPACT_NW(X, 1) VO_COMPACT_NW(X, 2)                                                  \
     X(kB_count_mask, (compact_k::k_count_mask), (compact_k::b_count_mask(a..., vb)), 0)                           \
     X(kB_filter_count, (compact_k::k_filter_count<false>), (compact_k::b_filter_count<false>(a..., vb)), 0)       \
     X(kB_scan_tiles, (compact_k::k_scan_tiles), (compact_k::b_scan_tiles<256>(a..., (uint64_t *)lds)), 2048)      \
