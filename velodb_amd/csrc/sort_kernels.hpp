@@ -5,16 +5,25 @@
 // same compare-exchange network is grouped into far fewer HBM passes:
 //   pass 0       k_sort_local_ct : every tile of 2^T_LOG records fully
 //                                  sorted (levels p <= T_LOG), registers+LDS;
-//   per level p > T_LOG:
-//                k_sort_global   : stages q >= T_LOG, up to S_MAX per pass;
-//                k_sort_merge    : stages q < T_LOG in one tile pass.
-// The schedule is a function of n_pad only.
+// then either the wrapped schedule (the default, plan_wrapped), on tiles of
+// 2^T_LOG or 2^W_LOG records:
+//                k_sort_global   : up to S_MAX strided stages in registers;
+//                k_sort_hybrid   : 4 and more strided stages through LDS;
+//                k_sort_merge    : a level's stages inside contiguous tiles;
+//                k_sort_wrap     : a level's last stages and the next one's
+//                                  first ones in one pass;
+// or level by level (plan_passes; tuning words and recorded programs): for
+// each p > T_LOG the stages q >= T_LOG by global and hybrid passes, then a
+// merge.  Either is a function of the sizes, the record kind and the tuning.
 //
-// Addressing: every block's records sit at one uniform (scalar) base plus a
-// per-thread offset below 2^13, so loads and stores use the scalar-base +
-// 32-bit vector-offset form and the address costs one VGPR.  Batched sorts
-// map a block's uniform virtual base through a per-instance offset table
-// (instances are never smaller than a tile on these kernels).
+// Addressing: a block's records sit at one uniform (scalar) base; every column
+// has a buffer resource there, the register's element offset goes to the
+// scalar offset field and the thread's to the vector offset.  In strided tiles
+// and global passes both reach across the array: below 2^29 elements
+// (kMaxSortRows) and of disjoint bits, so that their sum is below 2^32 bytes
+// for 8-byte columns too.  Batched sorts map a block's uniform virtual base
+// through a per-instance offset table (instances are never smaller than a tile
+// on these kernels).
 #pragma once
 
 #include "sort_core.hpp"
@@ -56,8 +65,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *ubase)
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // Tile form: one buffer resource per column for the tile's uniform base u,
-// the per-register offset so (elements, uniform, < 2^16) in the scalar
-// offset field and the per-thread offset vi in the vector offset.
+// the per-register offset so (elements, uniform) in the scalar offset field and
+// the per-thread offset vi in the vector offset; so + vi < 2^29 (see the top).
 template <typename T, int CP = 0>
 __device__ __forceinline__ T ld_t(__amdgpu_buffer_rsrc_t r, uint32_t vi, uint32_t so)
 {
@@ -505,11 +514,13 @@ inline std::vector<Pass> plan_passes(int n_log, int t_log, int s_max, int r_log,
 // the tile, in network order, where a pass may also end one level and start the
 // next (wrap).  Found by dynamic programming from the end over (level p, next
 // stage q); the costs are one pass's time at 2^28 records relative to a copy of
-// the array (below the MALL the order is the same).  A level-by-level schedule
-// needs ceil((p - t_log) / h_max) + 1 passes for level p; this one, on tiles of
-// 2^w_log records above the local pass's 2^t_log, comes close to (p - 5) /
-// (w_log - 5) on average: at 2^28 31 passes instead of 38 on 2^13-record tiles
-// and 28 on 2^14-record ones.
+// the array.  (Inside the MALL they differ: at 2^23 records the nine-stage hybrid,
+// here the dearest one, is the cheapest pass, 32 us against 36 for the merge and
+// 38-43 for wraps; the plan found with those times is the same 16 passes.)  A
+// level-by-level schedule needs ceil((p - t_log) / h_max) + 1 passes for level
+// p; this one, on tiles of 2^w_log records above the local pass's 2^t_log, comes
+// close to (p - 5) / (w_log - 5) on average: at 2^28 31 passes instead of 38 on
+// 2^13-record tiles and 28 on 2^14-record ones.
 inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int w_log, int s_max, int r_log)
 {
     std::vector<Pass> v;
@@ -558,10 +569,11 @@ inline std::vector<Pass> plan_wrapped(int n_log, int t_log, int w_log, int s_max
 // Hybrid passes of at most HW_MAX stages run with twice the threads per block
 // and half the records per thread (the same tiles, so the same records per
 // block): more waves per SIMD where that pass is faster.
-// WRAP = false builds the level-by-level schedule alone, BATCH = true the
+// WRAP = false builds the level-by-level schedule alone, LEVELS = false the
+// wrapped one alone (its callers ask wrapped() first), BATCH = true the
 // passes over many small instances whose arrays together exceed the MALL.
 template <class R, int T_LOG, int R_LOG, int BLOCK, int S_MAX, int H_MAX = 0, int S_LARGE = S_MAX, int LARGE_LOG = 64,
-          int HW_MAX = 0, int W_LOG = T_LOG, bool WRAP = true, bool BATCH = false>
+          int HW_MAX = 0, int W_LOG = T_LOG, bool WRAP = true, bool BATCH = false, bool LEVELS = true>
 struct SortImpl {
     static_assert(T_LOG >= 8, "global passes need q_lo >= 8 (256-thread blocks)");
     static_assert(H_MAX == 0 || (T_LOG - H_MAX >= 5 && BLOCK << R_LOG == 1 << T_LOG), "hybrid tile shape");
@@ -644,7 +656,9 @@ struct SortImpl {
     // two key words: the compile-time tile sort at their own size, on at least
     // one whole wavefront.  (The run-time form below keeps its LDS addresses in
     // registers and a barrier around every relayout: one array of 4096 12-byte
-    // records, call and wait included, 61 -> 40 us.)
+    // records, call and wait included, 61 -> 40 us.)  Batch classes of these
+    // sizes run the same form, however many their instances (64 of 2^10 records
+    // 81 -> 51 us, 1024 of 2^12 423 -> 354, call and item table included).
     template <bool TRACE, int T = 8>
     static bool launch_small(vo_ctx *ctx, Bufs<R> b, IMap map, int t, int p_top, uint64_t n_valid, int fill,
                              uint64_t n_virtual)
@@ -736,6 +750,41 @@ struct SortImpl {
         }
     }
 
+    // The level-by-level schedule's passes above the local one: merge (kind 3)
+    // and hybrid (kind 4) on tiles of the local pass's size.
+    template <bool TRACE, int CP, bool XC>
+    static void level_pass(vo_ctx *ctx, Bufs<R> b, IMap map, const Pass &ps, int n_log, int p_top, uint64_t n_virtual)
+    {
+        if (ps.kind == 4) {
+            switch (ps.s) {
+            case 4: launch_hybrid<TRACE, 4, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+            case 5: launch_hybrid<TRACE, 5, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+            case 6: launch_hybrid<TRACE, 6, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+            case 7: launch_hybrid<TRACE, 7, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+            case 8: launch_hybrid<TRACE, 8, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
+            default: throw Error{VO_ERR_INVALID, "bad hybrid stage count"};
+            }
+            return;
+        }
+        const size_t lds = dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes();
+        const uint32_t n_tiles = (uint32_t)(n_virtual >> T_LOG);
+        if (ctx->tuning.pipe_merge && !ctx->rec) { // resident: plain merge blocks
+            auto k = dev::k_sort_merge_pipe<R, T_LOG, R_LOG, BLOCK, TRACE>;
+            VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            int per_cu = 0;
+            VO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k, BLOCK, lds));
+            const uint32_t grid = std::min<uint32_t>(n_tiles, (uint32_t)std::max(1, per_cu) * ctx->num_cus);
+            LaunchInfo li{"sort_merge", dim3(grid), dim3(BLOCK), (uint32_t)lds, hash_mix(ps.p, p_top)};
+            launch(ctx, li, k, b, map, ps.p, p_top, n_tiles, trace_slot(ctx));
+        } else {
+            LaunchInfo li{"sort_merge", dim3(n_tiles), dim3(BLOCK), (uint32_t)lds, hash_mix(ps.p, p_top)};
+            auto k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP, XC>;
+            if (!XC && tiles_xc(n_log)) k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP, true>;
+            VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            launch(ctx, li, k, b, map, ps.p, p_top, trace_slot(ctx));
+        }
+    }
+
     template <bool TRACE, int CP, bool XC>
     static void run_t(vo_ctx *ctx, Bufs<R> b, int n_log, uint64_t n_valid, int fill, IMap map, int p_top,
                       uint64_t n_virtual)
@@ -767,16 +816,6 @@ struct SortImpl {
                 break;
             }
             case 2: global_pass<TRACE, CP, XC>(ctx, b, map, ps.p, ps.q_lo, ps.s, p_top, n_virtual); break;
-            case 4:
-                switch (ps.s) {
-                case 4: launch_hybrid<TRACE, 4, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 5: launch_hybrid<TRACE, 5, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 6: launch_hybrid<TRACE, 6, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 7: launch_hybrid<TRACE, 7, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                case 8: launch_hybrid<TRACE, 8, CP, XC>(ctx, b, map, ps.p, ps.q_lo, p_top, n_virtual); break;
-                default: throw Error{VO_ERR_INVALID, "bad hybrid stage count"};
-                }
-                break;
             case 5:
             case 6:
             case 7:
@@ -785,26 +824,13 @@ struct SortImpl {
                 else
                     tile_pass<TRACE, CP, XC, W_LOG>(ctx, b, map, ps, p_top, n_virtual, tiles_xc(n_log));
                 break;
-            case 3: {
-                const size_t lds = dev::TileCT<R, T_LOG, R_LOG, TRACE>::lds_bytes();
-                const uint32_t n_tiles = (uint32_t)(n_virtual >> T_LOG);
-                if (ctx->tuning.pipe_merge && !ctx->rec) { // resident: plain merge blocks
-                    auto k = dev::k_sort_merge_pipe<R, T_LOG, R_LOG, BLOCK, TRACE>;
-                    VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                    int per_cu = 0;
-                    VO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k, BLOCK, lds));
-                    const uint32_t grid = std::min<uint32_t>(n_tiles, (uint32_t)std::max(1, per_cu) * ctx->num_cus);
-                    LaunchInfo li{"sort_merge", dim3(grid), dim3(BLOCK), (uint32_t)lds, hash_mix(ps.p, p_top)};
-                    launch(ctx, li, k, b, map, ps.p, p_top, n_tiles, trace_slot(ctx));
-                } else {
-                    LaunchInfo li{"sort_merge", dim3(n_tiles), dim3(BLOCK), (uint32_t)lds, hash_mix(ps.p, p_top)};
-                    auto k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP, XC>;
-                    if (!XC && tiles_xc(n_log)) k = dev::k_sort_merge<R, T_LOG, R_LOG, BLOCK, TRACE, CP, true>;
-                    VO_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                    launch(ctx, li, k, b, map, ps.p, p_top, trace_slot(ctx));
-                }
+            case 3:
+            case 4:
+                if constexpr (LEVELS)
+                    level_pass<TRACE, CP, XC>(ctx, b, map, ps, n_log, p_top, n_virtual);
+                else
+                    throw Error{VO_ERR_INVALID, "level-by-level pass not built"};
                 break;
-            }
             }
         }
     }

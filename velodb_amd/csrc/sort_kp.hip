@@ -24,7 +24,7 @@ using SortKP = SortImpl<RecKP, 13, 4, 512, 5, 8, 3, 27, 6, 14, true, true>;
 // each, give every CU one: local pass at 2^20 48 -> 26 us, merge and wrap passes
 // 11 -> 7.5 us for 15 passes instead of 12.  Whole sorts: 2^13 47 -> 34 us, 2^16
 // 86 -> 59, 2^18 116 -> 83, 2^20 177 -> 146; at 2^21 both take 214.
-using SortKP_S = SortImpl<RecKP, 12, 3, 512, 5, 7, 3, 27, 0, 12>;
+using SortKP_S = SortImpl<RecKP, 12, 3, 512, 5, 0, 3, 27, 0, 12, true, false, false>;
 constexpr int kSmallLog = 20;
 // The resident queue kernel runs 256-thread blocks: the 12-byte sort runs
 // there on 2^12-record tiles (the same network, so the same output).

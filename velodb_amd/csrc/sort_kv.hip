@@ -19,7 +19,7 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 using SortKV = SortImpl<RecKV, 12, 4, 256, 5, 7, 3, 27, 0, 13>;
 // Up to 2^20 records, one tile or fewer a CU: 512 threads of 8 records each (as
 // in sort_kp.hip); a shuffle of 2^20 rows with its permutation 222 -> 203 us.
-using SortKV_S = SortImpl<RecKV, 12, 3, 512, 5, 7, 3, 27, 0, 12>;
+using SortKV_S = SortImpl<RecKV, 12, 3, 512, 5, 0, 3, 27, 0, 12, true, false, false>;
 
 } // namespace
 

@@ -22,7 +22,7 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 using SortM1 = SortImpl<RecM1, 12, 4, 256, 3, 7, 3, 64, 0, 13>;
 // up to 2^20 rows, one tile or fewer a CU: 512 threads of 8 rows (sort_kp.hip);
 // OP_SORT of 2^20 rows 194 -> 173 us
-using SortM1_S = SortImpl<RecM1, 12, 3, 512, 3, 7, 3, 64, 0, 12>;
+using SortM1_S = SortImpl<RecM1, 12, 3, 512, 3, 0, 3, 64, 0, 12, true, false, false>;
 
 // ------------------------------------------------- multi-column (OP_SORT)
 

@@ -15,7 +15,7 @@ const bool kRegistered = (register_bodies(kBodies, sizeof kBodies / sizeof kBodi
 // register passes and tiles as for one key word (sort_multi.hip)
 using SortM2 = SortImpl<RecM2, 12, 4, 256, 3, 7, 3, 64, 0, 13>;
 // (as there; two key words, 2^20 rows: 289 -> 247 us)
-using SortM2_S = SortImpl<RecM2, 12, 3, 512, 3, 7, 3, 64, 0, 12>;
+using SortM2_S = SortImpl<RecM2, 12, 3, 512, 3, 0, 3, 64, 0, 12, true, false, false>;
 
 } // namespace
 
