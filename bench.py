@@ -22,7 +22,8 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 # launch families of the sort passes: local, merge, register passes of 1-5
-# stages, LDS-staged passes of 4-8 stages
+# stages, LDS-staged passes of 4-9 stages, passes that end one level and start
+# the next with 1-9 stages of it
 SORT_FAMS = (["sort_local", "sort_merge"] + [f"sort_global_s{s}" for s in range(1, 6)] +
              [f"sort_hybrid_s{s}" for s in range(4, 10)] + [f"sort_wrap_s{s}" for s in range(1, 10)])
 METRIC = "oblivious sort Mrec/s at 2^28 (%HBM peak); served QPS + p50/p99 vs plain"

@@ -457,6 +457,9 @@ typedef struct vo_config {
                                 0x400 its LDS-staged passes with the other block shape, 0x800
                                 the other cache policy of the sort and compaction passes
                                 (streaming loads and stores are chosen above 256 MB of rows).
+                                A word that changes the stages per pass, or holds 0x100, 0x200
+                                or 0x400, sorts level by level instead of by the default
+                                schedule, whose passes also end one level and start the next.
                                 Every word applies the same network: the output does not
                                 change */
     uint32_t queue_idle_us;  /* the resident queue kernel leaves after this long without a

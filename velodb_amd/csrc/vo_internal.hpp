@@ -182,7 +182,8 @@ inline bool is_pow2(uint64_t v) { return v && !(v & (v - 1)); }
 // Tuning word (vo_config.tuning): bits 0-3 register-pass stages, bits 4-7
 // hybrid-pass stages + 1; bits 8-11 toggle the prefetching merge, the
 // 1024-thread 12-byte sort, its hybrid block shape and the sort passes'
-// cache policy.  0 keeps the defaults.
+// cache policy.  0 keeps the defaults.  Any word but 0x800 and the default
+// widths sorts level by level (SortImpl::wrapped).
 inline SortTuning apply_tuning_word(SortTuning t, uint32_t w)
 {
     if (w & 0xF) t.max_fused_stages = (int)(w & 0xF);
