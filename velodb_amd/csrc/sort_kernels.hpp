@@ -515,8 +515,8 @@ inline std::vector<Pass> plan_passes(int n_log, int t_log, int s_max, int r_log,
 // next (wrap).  Found by dynamic programming from the end over (level p, next
 // stage q); the costs are one pass's time at 2^28 records relative to a copy of
 // the array.  (Inside the MALL they differ: at 2^23 records the nine-stage hybrid,
-// here the dearest one, is the cheapest pass, 32 us against 36 for the merge and
-// 38-43 for wraps; the plan found with those times is the same 16 passes.)  A
+// here the dearest one, is the cheapest pass, 31 us against 37 for the merge and
+// 40-44 for wraps; the plan found with those times is the same 16 passes.)  A
 // level-by-level schedule needs ceil((p - t_log) / h_max) + 1 passes for level
 // p; this one, on tiles of 2^w_log records above the local pass's 2^t_log, comes
 // close to (p - 5) / (w_log - 5) on average: at 2^28 31 passes instead of 38 on
